@@ -419,6 +419,9 @@ struct WideRay {
     f3 o, d, binv, berr;
     float best_t;
     uint32_t best, oct, node, pmask, sp;
+    uint32_t perm;             // the node's slot order for the ray's octant (wide_node)
+    uint32_t k, kend, kfirst;  // the leaf being tested: next primitive, end, first
+    float t_leaf;              // best_t when the ray entered it
     TriHit hit;
 };
 
@@ -473,7 +476,7 @@ __device__ __forceinline__ bool leaf_box_hit(const WideTree &T, uint32_t first, 
 // reference). Rays without a direction, with NaNs or far outside any scene take the
 // reference's own test on the decoded planes (kRayGeneric, wide_box_generic). The
 // hits do not depend on any of this: a triangle hit counts only if its leaf's exact
-// box passes box_hit (wide_step).
+// box passes box_hit (wide_leaf).
 // The traversal is bound by instruction issue (VALU busy 62-76 %), and decoding each
 // plane to test it with box_hit's operations took about twice the instructions:
 // 1080p camera rays into 10M triangles 1995 -> 1780 us, their bounce 1490 -> 1327 us,
@@ -517,6 +520,7 @@ __device__ __forceinline__ bool wide_ray_start(WideRay &R, const float4 *__restr
     R.node = 0;
     R.pmask = 0xFFu;
     R.sp = 0;
+    R.k = R.kend = 0;
     return R.best_t > 0.f;
 }
 
@@ -551,22 +555,66 @@ __device__ __forceinline__ uint32_t wide_box_generic(const WNode *W, const WideR
     return hs;
 }
 
-// One node visit of one ray: tests the node's eight child boxes, then takes
-// the node's pending children in depth-first position order (leaves are
-// intersected on the spot, the first interior child is descended into, the
-// rest of the node is pushed), or pops the stack. Returns false once the ray
-// is finished. qi: the ray's queue slot, which owns the ray's spill area.
-template <bool COUNT, bool SHAPES>
-__device__ __forceinline__ bool wide_step(WideRay &R, const WideTree &T, const WideTrace &B, int any_hit,
-                                          uint32_t qi, uint32_t *__restrict__ err,
-                                          uint2 (*s_stack)[kWideBlock], uint32_t &visits, uint32_t &boxes,
-                                          uint32_t &tests) {
-    if (R.node >= T.num_nodes) {  // only a corrupt layout gets here
+// Takes the ray on to its next piece of work: the node's pending positions in
+// depth-first order (a leaf: its range in R.k .. R.kend; an interior child: the rest
+// of the node is pushed and the child is R.node), else the popped stack. Returns
+// false once the ray is finished. qi: the ray's queue slot, which owns the ray's
+// spill area.
+__device__ __forceinline__ bool wide_advance(WideRay &R, const WideTree &T, const WideTrace &B, uint32_t qi,
+                                             uint32_t *__restrict__ err, uint2 (*s_stack)[kWideBlock]) {
+    if (R.pmask == 0) {
+        if (R.sp == 0) return false;
+        const uint32_t sp = --R.sp;
+        const uint2 e = sp < kLdsStack ? s_stack[sp][threadIdx.x]
+                                       : B.spill[uint64_t(qi) * B.spill_per_ray + (sp - kLdsStack)];
+        R.node = e.x;
+        R.pmask = e.y;
+        return true;
+    }
+    const uint32_t p = __builtin_ctz(R.pmask);
+    const uint32_t rest = R.pmask & (R.pmask - 1);
+    const uint2 ref = *reinterpret_cast<const uint2 *>((T.nodes + R.node)->ref[(R.perm >> (4 * p)) & 7u]);
+    if (ref.x & kWideLeaf) {
+        const uint32_t first = ref.x & ~kWideLeaf;
+        if (uint64_t(first) + ref.y > T.tree->num_prims) {
+            atomicOr(err, uint32_t(kErrStack));
+            return false;
+        }
+        R.pmask = rest;
+        R.k = R.kfirst = first;
+        R.kend = first + ref.y;
+        R.t_leaf = R.best_t;
+        return true;
+    }
+    if (rest) {  // the rest of this node waits
+        const uint32_t sp = R.sp;
+        if (sp < kLdsStack) {
+            s_stack[sp][threadIdx.x] = make_uint2(R.node, rest);
+        } else if (sp - kLdsStack < B.spill_per_ray) {
+            B.spill[uint64_t(qi) * B.spill_per_ray + (sp - kLdsStack)] = make_uint2(R.node, rest);
+        } else {
+            atomicOr(err, uint32_t(kErrStack));
+            return false;
+        }
+        R.sp = sp + 1;
+    }
+    R.node = ref.x;
+    R.pmask = 0xFFu;
+    return true;
+}
+
+// One node visit of one ray: tests the node's eight child boxes; R.pmask becomes the
+// pending positions whose box passes, in depth-first order. Returns false for a node
+// outside the tree (only a corrupt layout gets there).
+template <bool COUNT>
+__device__ __forceinline__ bool wide_node(WideRay &R, const WideTree &T, uint32_t *__restrict__ err, uint32_t &visits,
+                                          uint32_t &boxes) {
+    if (R.node >= T.num_nodes) {
         atomicOr(err, uint32_t(kErrStack));
         return false;
     }
     const WNode *W = T.nodes + R.node;
-    const uint32_t perm = T.order[R.node * 8 + (R.oct & 7u)];
+    const uint32_t perm = R.perm = T.order[R.node * 8 + (R.oct & 7u)];
     if (COUNT) { ++visits; boxes += kWide; }
     // all eight child boxes (4 x 16-byte loads: origin, exponents, 48 plane
     // bytes), hit mask in slot order
@@ -626,84 +674,44 @@ __device__ __forceinline__ bool wide_step(WideRay &R, const WideTree &T, const W
     const uint32_t sel1 = (phi & 0xFu) | ((phi & 0xF0u) << 4) | ((phi & 0xF00u) << 8) | ((phi & 0xF000u) << 12);
     const uint32_t g0 = __builtin_amdgcn_perm(d1, d0, sel0), g1 = __builtin_amdgcn_perm(d1, d0, sel1);
     const uint32_t hm = (((g0 * 0x01020408u) >> 24) & 0xFu) | ((((g1 * 0x01020408u) >> 24) & 0xFu) << 4);
-    uint32_t pmask = R.pmask & hm;
-    const float t_at_visit = R.best_t;
-    while (pmask) {
-        const uint32_t p = __builtin_ctz(pmask);
-        pmask &= pmask - 1;
-        const uint32_t s = (perm >> (4 * p)) & 0xFu;
-        if (R.best_t != t_at_visit) {  // a leaf of this node shortened the ray: re-test at pop time
-            if (COUNT) ++boxes;
-            if ((R.oct & kRayGeneric) && !((wide_box_generic(W, R) >> s) & 1u)) continue;
-            float tn = 0.0f;
-#pragma unroll
-            for (int a = 0; a < 3; ++a)
-                tn = fmaxf(tn, fmaf(float(W->q[a + 3 * ((R.oct >> a) & 1u)][s]), ax[a].a, ax[a].bn));
-            if (!(tn <= R.best_t)) continue;
-        }
-        const uint32_t ref0 = W->ref[s][0];
-        if (ref0 & kWideLeaf) {
-            const uint32_t first = ref0 & ~kWideLeaf, cnt = W->ref[s][1];
-            if (uint64_t(first) + cnt > T.tree->num_prims) {
-                atomicOr(err, uint32_t(kErrStack));
-                return false;
-            }
-            const float t_leaf = R.best_t;
-            for (uint32_t k = first; k < first + cnt; ++k) {
-                const float4 *t4 = reinterpret_cast<const float4 *>(T.tree->tri_leaf) + 3ull * k;
-                const float4 q0 = t4[0], q1 = t4[1], q2 = t4[2];
-                if (COUNT) ++tests;
-                TriHit h;
-                bool hit, robust = false;
-                if (SHAPES && __float_as_uint(q2.y) != 0u) {
-                    pt::QHit qh;
-                    hit = pt::shape_hit(T.tree->shapes, __float_as_uint(q2.y) - 1u, R.o, R.d, R.best_t, &qh);
-                    h = TriHit{qh.p.x, qh.p.y, qh.p.z, qh.t};
-                } else {
-                    hit = tri_hit(R.o, R.d, R.best_t, f3{q0.x, q0.y, q0.z}, f3{q0.w, q1.x, q1.y},
-                                  f3{q1.z, q1.w, q2.x}, &h, &robust);
-                }
-                if (hit) {
-                    // The first hit in this leaf: would the binary traversal have entered
-                    // the leaf? Its exact box (the union of its primitives' boxes) against
-                    // the t at entry; the quantized slot box only contains it. A robust
-                    // triangle hit (tri_hit: clear of the edges and of t_max by its error
-                    // bounds, where t_max is the t at entry) passes every box holding the
-                    // triangle; only the others (ties on box faces, edge and grazing hits,
-                    // analytic shapes) assemble the leaf's box from its primitives.
-                    if (R.best_t == t_leaf && !robust && !leaf_box_hit(T, first, cnt, R, t_leaf)) break;
-                    R.best = T.tree->prim_order[k];
-                    R.hit = h;
-                    R.best_t = h.t;
-                    if (!(h.t == h.t)) R.oct |= kRayGeneric;  // NaN: no box passes the reference's test any more
-                    if (any_hit) return false;
-                }
-            }
-            continue;
-        }
-        if (pmask) {  // the rest of this node waits
-            const uint32_t sp = R.sp;
-            if (sp < kLdsStack) {
-                s_stack[sp][threadIdx.x] = make_uint2(R.node, pmask);
-            } else if (sp - kLdsStack < B.spill_per_ray) {
-                B.spill[uint64_t(qi) * B.spill_per_ray + (sp - kLdsStack)] = make_uint2(R.node, pmask);
-            } else {
-                atomicOr(err, uint32_t(kErrStack));
-                return false;
-            }
-            R.sp = sp + 1;
-        }
-        R.node = ref0;
-        R.pmask = 0xFFu;
+    R.pmask &= hm;
+    return true;
+}
+
+// One triangle (or analytic primitive) of the ray's current leaf, R.k. Returns false
+// when the ray is finished (an any-hit ray that hit).
+template <bool COUNT, bool SHAPES>
+__device__ __forceinline__ bool wide_leaf(WideRay &R, const WideTree &T, int any_hit, uint32_t &tests) {
+    const uint32_t k = R.k++;
+    const float4 *t4 = reinterpret_cast<const float4 *>(T.tree->tri_leaf) + 3ull * k;
+    const float4 q0 = t4[0], q1 = t4[1], q2 = t4[2];
+    if (COUNT) ++tests;
+    TriHit h;
+    bool hit, robust = false;
+    if (SHAPES && __float_as_uint(q2.y) != 0u) {
+        pt::QHit qh;
+        hit = pt::shape_hit(T.tree->shapes, __float_as_uint(q2.y) - 1u, R.o, R.d, R.best_t, &qh);
+        h = TriHit{qh.p.x, qh.p.y, qh.p.z, qh.t};
+    } else {
+        hit = tri_hit(R.o, R.d, R.best_t, f3{q0.x, q0.y, q0.z}, f3{q0.w, q1.x, q1.y}, f3{q1.z, q1.w, q2.x}, &h,
+                      &robust);
+    }
+    if (!hit) return true;
+    // The first hit in this leaf: would the binary traversal have entered the leaf?
+    // Its exact box (the union of its primitives' boxes) against the t at entry; the
+    // quantized slot box only contains it. A robust triangle hit (tri_hit: clear of
+    // the edges and of t_max by its error bounds, where t_max is the t at entry)
+    // passes every box holding the triangle; only the others (ties on box faces, edge
+    // and grazing hits, analytic shapes) assemble the leaf's box from its primitives.
+    if (R.best_t == R.t_leaf && !robust && !leaf_box_hit(T, R.kfirst, R.kend - R.kfirst, R, R.t_leaf)) {
+        R.k = R.kend;
         return true;
     }
-    if (R.sp == 0) return false;
-    const uint32_t sp = --R.sp;
-    const uint2 e = sp < kLdsStack ? s_stack[sp][threadIdx.x]
-                                   : B.spill[uint64_t(qi) * B.spill_per_ray + (sp - kLdsStack)];
-    R.node = e.x;
-    R.pmask = e.y;
-    return true;
+    R.best = T.tree->prim_order[k];
+    R.hit = h;
+    R.best_t = h.t;
+    if (!(h.t == h.t)) R.oct |= kRayGeneric;  // NaN: no box passes the reference's test any more
+    return !any_hit;
 }
 
 template <bool COUNT>
@@ -723,11 +731,21 @@ __device__ __forceinline__ void add_counts(unsigned long long *counts, uint32_t 
 // lane, G = waves in the grid) and a lane whose ray has finished takes the wave's
 // next slot as soon as kRefill lanes are idle, so that the waves keep most lanes
 // busy instead of waiting for their slowest ray. Each ray is traced on its own
-// (wide_ray_start, wide_step until it reports the ray finished, wide_ray_finish),
+// (wide_ray_start, then wide_node, wide_leaf and wide_advance until one reports the
+// ray finished, wide_ray_finish),
 // so which lane or wave takes it changes nothing. MULTI: every ray selects its own
 // tree, jw[ray_job[i >> job_shift]] (jobs of a batched render); the spill area
 // stays the launch's.
 constexpr uint32_t kRefill = 8;
+// A wave steps either its lanes that wait at a node or those that wait at a leaf's
+// primitive, never both paths for a few lanes each: the leaves go when they are at
+// least a quarter of the others. Waiting longer fills the leaf steps but idles more
+// lanes (and delays a wave's last rays): 1/4 against 1/6, 1/8, 1/12 or a fixed count
+// of 8 lanes was fastest or within 1 % on camera, bounce and shadow queues and path
+// tracing. Against testing every leaf where a lane met it: 1080p camera rays into 10M
+// triangles 1780 -> 1246 us, shadow rays into 1M 909 -> 701 us, 999 rays 209 -> 178 us
+// (and 96 -> 75 VGPRs, 6 waves per SIMD).
+constexpr uint32_t kLeafShare = 4;
 
 template <bool COUNT, bool MULTI, bool SHAPES>
 __device__ __forceinline__ void trace_wide_persistent_body(const WideTrace &B, const float4 *__restrict__ rays,
@@ -770,8 +788,19 @@ __device__ __forceinline__ void trace_wide_persistent_body(const WideTrace &B, c
             continue;
         }
         if (idle == ~0ull) break;  // nothing in flight and nothing left
-        if (live) {
-            live = wide_step<COUNT, SHAPES>(R, T, B, any_hit, qi, err, s_stack, visits, boxes, tests);
+        const bool in_leaf = live && R.k < R.kend;
+        const uint64_t leaves = __ballot(in_leaf);
+        if (uint32_t(__popcll(leaves)) * kLeafShare >= uint32_t(__popcll(~(leaves | idle)))) {
+            if (in_leaf) {
+                live = wide_leaf<COUNT, SHAPES>(R, T, any_hit, tests);
+                // a leaf that shortened the ray: the node's other boxes are tested again
+                if (live && R.k == R.kend && (R.pmask == 0 || R.best_t == R.t_leaf))
+                    live = wide_advance(R, T, B, qi, err, s_stack);
+                if (!live) wide_ray_finish(R, i, prim_out, t_out, bary_out);
+            }
+        } else if (live && !in_leaf) {
+            live = wide_node<COUNT>(R, T, err, visits, boxes);
+            if (live) live = wide_advance(R, T, B, qi, err, s_stack);
             if (!live) wide_ray_finish(R, i, prim_out, t_out, bary_out);
         }
     }
