@@ -41,8 +41,9 @@ constexpr uint32_t kIdle = 0xFFFFFFFFu;
 
 // counters[] layout (u32 words); 8..15 hold u64 accumulators of a batched render.
 // A slot holds a live path exactly when its ray is active, so the closest-hit
-// compaction's count (kCntQueue) is the round's live-path count.
-constexpr int kCntNextId = 0, kCntQueue = 2, kCntSQueue = 3, kCntRound = 5, kCntDone = 6, kCntAccRays = 8;
+// compaction's count (kCntQueue) is the round's live-path count. kCntQueue and
+// kCntSQueue are two words each (the traversal's queue_len), cleared together.
+constexpr int kCntNextId = 0, kCntQueue = 2, kCntSQueue = 4, kCntRound = 6, kCntDone = 7, kCntAccRays = 8;
 
 struct State {
     uint32_t *path_id, *flags, *dim;
@@ -949,8 +950,7 @@ __global__ __launch_bounds__(kBlock) void reduce_shards_kernel(float *d, uint32_
 // Start and end of a batched round (kernels, so that a captured graph holds no memset).
 __global__ void round_begin_kernel(uint32_t *counters) {
     if (threadIdx.x == 0) {
-        counters[kCntQueue] = 0;
-        counters[kCntSQueue] = 0;
+        for (int k = kCntQueue; k < kCntSQueue + 2; ++k) counters[k] = 0;
     }
 }
 // A round that traced no ray had no live path: the render is over and the round
@@ -1393,7 +1393,7 @@ hipError_t render(const SceneDev &S, const WideTrace &W0, uint32_t spp, uint32_t
         hipError_t e;
         hipEvent_t *E = ev + 3 + 5 * (round & 1);
         P.round = round;
-        PT_CK(hipMemsetAsync(st.counters + kCntQueue, 0, 8, stream));
+        PT_CK(hipMemsetAsync(st.counters + kCntQueue, 0, 16, stream));
         PT_CK(hipEventRecord(E[0], stream));
         const bool tuning = round >= kTuneFirst && round < kTuneFirst + 4;
         const bool sort_c = tuning ? ((round - kTuneFirst) % 2 == 0) : tune.sort_closest;

@@ -59,8 +59,9 @@ struct WideTrace {
 };
 
 // counts (device, nullable): adds [wide nodes visited, child box tests, triangle tests].
-// queue (device, n entries) and queue_len (device, zeroed by the caller) hold the
-// compacted active rays.
+// queue (device, n entries) and queue_len (device, two words, both zeroed by the
+// caller) hold the compacted active rays: queue_len[0] their number, queue_len[1]
+// the traversal's counter of runs handed out.
 hipError_t trace_wide(const WideTrace &B, const float *rays, uint32_t n, int any_hit, uint32_t *prim_out,
                       float *t_out, float *bary_out, uint32_t *err, unsigned long long *counts, uint32_t *queue,
                       uint32_t *queue_len, hipStream_t stream);
@@ -74,8 +75,8 @@ hipError_t trace_wide_multi(const WideTrace &B, const WideTrace *jobs, const uin
 
 // Orders the active rays of [n] by (direction octant, Morton code of the origin
 // on a 64^3 grid over the tree's box; 20-bit keys, two radix passes) into *queue
-// (a pointer into the scratch, n words) and counts them into *queue_len (zeroed
-// by the caller); inactive rays report a miss. trace_wide_queued then traces that
+// (a pointer into the scratch, n words) and counts them into *queue_len (two
+// words, zeroed by the caller, as above); inactive rays report a miss. trace_wide_queued then traces that
 // queue.
 struct RaySortScratch {
     DevBuf keys[2], vals[2], hist;
@@ -91,11 +92,11 @@ hipError_t reserve_ray_sort(RaySortScratch &s, uint32_t n);
 hipError_t trace_wide_multi_queued(const WideTrace &B, const WideTrace *jobs, const uint32_t *ray_job,
                                    uint32_t job_shift, const float *rays, uint32_t n, int any_hit, uint32_t *prim_out,
                                    float *t_out, float *bary_out, uint32_t *err, const uint32_t *queue,
-                                   const uint32_t *queue_len, hipStream_t stream);
+                                   uint32_t *queue_len, hipStream_t stream);
 // counts (device, nullable): adds [nodes visited, child box tests, primitive tests].
 hipError_t trace_wide_queued(const WideTrace &B, const float *rays, uint32_t n, int any_hit, uint32_t *prim_out,
                              float *t_out, float *bary_out, uint32_t *err, const uint32_t *queue,
-                             const uint32_t *queue_len, hipStream_t stream, unsigned long long *counts = nullptr);
+                             uint32_t *queue_len, hipStream_t stream, unsigned long long *counts = nullptr);
 
 constexpr uint32_t kLdsStack = 12;
 
