@@ -414,9 +414,14 @@ __global__ __launch_bounds__(kCompactBlock) void compact_rays_kernel(const float
 }
 
 // Traversal state of one ray. binv / berr: the box tests' reciprocal direction
-// (clamped, finite) and per-axis constant error term (wide_ray_start).
+// (clamped, finite) and per-axis constant error term (wide_ray_start). Instead of the
+// direction it holds the triangle test's shear; ray_dir fetches the direction again
+// where an unusual case needs it.
 struct WideRay {
-    f3 o, d, binv, berr;
+    f3 o, binv, berr;
+    RayShear sh;
+    const float4 *rays;  // the queue's rays (wave-uniform), and this ray's index
+    uint32_t id;
     float best_t;
     uint32_t best, oct, node, pmask, sp;
     uint32_t perm;             // the node's slot order for the ray's octant (wide_node)
@@ -442,6 +447,11 @@ __device__ __forceinline__ WideTree tree_of(const WideTrace *B) {
 // The exact box of the binary leaf at positions [first, first + cnt) (the union of
 // its primitives' boxes: the leaf-ordered vertices, or an analytic primitive's
 // box stored as the corners lo, hi, lo) against the ray with t_max (bounds3.h:146-195).
+__device__ __forceinline__ f3 ray_dir(const WideRay &R) {
+    const float4 r1 = R.rays[2 * size_t(R.id) + 1];
+    return {r1.x, r1.y, r1.z};
+}
+
 __device__ __forceinline__ bool leaf_box_hit(const WideTree &T, uint32_t first, uint32_t cnt,
                                                         const WideRay &R, float t_max) {
     Box b = box_empty();
@@ -452,7 +462,7 @@ __device__ __forceinline__ bool leaf_box_hit(const WideTree &T, uint32_t first, 
     }
     const float lo[3] = {b.lo.x, b.lo.y, b.lo.z}, hi[3] = {b.hi.x, b.hi.y, b.hi.z};
     const int neg[3] = {int(R.oct & 1u), int((R.oct >> 1) & 1u), int((R.oct >> 2) & 1u)};
-    const f3 inv = {1.0f / R.d.x, 1.0f / R.d.y, 1.0f / R.d.z};
+    const f3 d = ray_dir(R), inv = {1.0f / d.x, 1.0f / d.y, 1.0f / d.z};
     return box_hit(lo, hi, R.o, inv, neg, t_max);
 }
 
@@ -503,19 +513,21 @@ __device__ __forceinline__ float box_err_const(float o, float inv, float binv, f
 
 // Loads ray i; true when it has an interval to trace (t_max > 0).
 __device__ __forceinline__ bool wide_ray_start(WideRay &R, const float4 *__restrict__ rays, uint32_t i) {
-    const float4 r0 = rays[2 * i], r1 = rays[2 * i + 1];
+    const float4 r0 = rays[2 * size_t(i)], r1 = rays[2 * size_t(i) + 1];
     R.o = {r0.x, r0.y, r0.z};
-    R.d = {r1.x, r1.y, r1.z};
+    const f3 d = {r1.x, r1.y, r1.z};
+    R.id = i;
+    R.sh = ray_shear(d);
     R.best_t = r0.w;
     R.best = kNoHit;
     R.hit = TriHit{0.f, 0.f, 0.f, 0.f};
-    const f3 inv = {1.0f / R.d.x, 1.0f / R.d.y, 1.0f / R.d.z};
+    const f3 inv = {1.0f / d.x, 1.0f / d.y, 1.0f / d.z};
     R.oct = uint32_t(inv.x < 0.f) | (uint32_t(inv.y < 0.f) << 1) | (uint32_t(inv.z < 0.f) << 2);
     const float least = fminf(fminf(fabsf(inv.x), fabsf(inv.y)), fabsf(inv.z));
     R.binv = {box_clamp_inv(inv.x, least), box_clamp_inv(inv.y, least), box_clamp_inv(inv.z, least)};
     R.berr = {box_err_const(R.o.x, inv.x, R.binv.x, least), box_err_const(R.o.y, inv.y, R.binv.y, least),
               box_err_const(R.o.z, inv.z, R.binv.z, least)};
-    const float span = fabsf(R.o.x) + fabsf(R.o.y) + fabsf(R.o.z) + fabsf(R.d.x) + fabsf(R.d.y) + fabsf(R.d.z);
+    const float span = fabsf(R.o.x) + fabsf(R.o.y) + fabsf(R.o.z) + fabsf(d.x) + fabsf(d.y) + fabsf(d.z);
     if (!(least <= 0x1p20f && span <= 0x1p60f)) R.oct |= kRayGeneric;
     R.node = 0;
     R.pmask = 0xFFu;
@@ -524,8 +536,9 @@ __device__ __forceinline__ bool wide_ray_start(WideRay &R, const float4 *__restr
     return R.best_t > 0.f;
 }
 
-__device__ __forceinline__ void wide_ray_finish(const WideRay &R, uint32_t i, uint32_t *__restrict__ prim_out,
+__device__ __forceinline__ void wide_ray_finish(const WideRay &R, uint32_t *__restrict__ prim_out,
                                                 float *__restrict__ t_out, float *__restrict__ bary_out) {
+    const uint32_t i = R.id;
     prim_out[i] = R.best;
     if (t_out) t_out[i] = R.best == kNoHit ? 0.f : R.hit.t;
     if (bary_out) {
@@ -539,7 +552,7 @@ __device__ __forceinline__ void wide_ray_finish(const WideRay &R, uint32_t i, ui
 // planes through the reference's slab test.
 __device__ __forceinline__ uint32_t wide_box_generic(const WNode *W, const WideRay &R) {
     const int neg[3] = {int(R.oct & 1u), int((R.oct >> 1) & 1u), int((R.oct >> 2) & 1u)};
-    const f3 inv = {1.0f / R.d.x, 1.0f / R.d.y, 1.0f / R.d.z};
+    const f3 d = ray_dir(R), inv = {1.0f / d.x, 1.0f / d.y, 1.0f / d.z};
     uint32_t hs = 0;
 #pragma unroll 1
     for (int s = 0; s < kWide; ++s) {
@@ -690,10 +703,10 @@ __device__ __forceinline__ bool wide_leaf(WideRay &R, const WideTree &T, int any
     bool hit, robust = false;
     if (SHAPES && __float_as_uint(q2.y) != 0u) {
         pt::QHit qh;
-        hit = pt::shape_hit(T.tree->shapes, __float_as_uint(q2.y) - 1u, R.o, R.d, R.best_t, &qh);
+        hit = pt::shape_hit(T.tree->shapes, __float_as_uint(q2.y) - 1u, R.o, ray_dir(R), R.best_t, &qh);
         h = TriHit{qh.p.x, qh.p.y, qh.p.z, qh.t};
     } else {
-        hit = tri_hit(R.o, R.d, R.best_t, f3{q0.x, q0.y, q0.z}, f3{q0.w, q1.x, q1.y}, f3{q1.z, q1.w, q2.x}, &h,
+        hit = tri_hit(R.o, R.sh, R.best_t, f3{q0.x, q0.y, q0.z}, f3{q0.w, q1.x, q1.y}, f3{q1.z, q1.w, q2.x}, &h,
                       &robust);
     }
     if (!hit) return true;
@@ -770,7 +783,8 @@ __device__ __forceinline__ void trace_wide_persistent_body(const WideTrace &B, c
     uint32_t visits = 0, boxes = 0, tests = 0;
     WideRay R;
     bool live = false;
-    uint32_t qi = 0, i = 0;
+    uint32_t qi = 0;
+    R.rays = rays;
     // wave-uniform: the slots of the current row not handed out yet, [next, next + left),
     // and the rows dealt to this wave, the current one included
     uint32_t next = __builtin_amdgcn_readfirstlane(blockIdx.x * kWideBlock + (threadIdx.x & ~uint32_t(kWave - 1)));
@@ -786,10 +800,10 @@ __device__ __forceinline__ void trace_wide_persistent_body(const WideTrace &B, c
                 const uint32_t pos = uint32_t(__popcll(idle & lanemask_lt()));
                 if (pos < left) {
                     qi = next + pos;
-                    i = queue[qi];
+                    const uint32_t i = queue[qi];
                     if (MULTI) T = tree_of(jw + ray_job[i >> job_shift]);
                     live = wide_ray_start(R, rays, i);
-                    if (!live) wide_ray_finish(R, i, prim_out, t_out, bary_out);
+                    if (!live) wide_ray_finish(R, prim_out, t_out, bary_out);
                 }
             }
             const uint32_t taken = min(uint32_t(__popcll(idle)), left);
@@ -820,12 +834,12 @@ __device__ __forceinline__ void trace_wide_persistent_body(const WideTrace &B, c
                 // a leaf that shortened the ray: the node's other boxes are tested again
                 if (live && R.k == R.kend && (R.pmask == 0 || R.best_t == R.t_leaf))
                     live = wide_advance(R, T, B, qi, err, s_stack);
-                if (!live) wide_ray_finish(R, i, prim_out, t_out, bary_out);
+                if (!live) wide_ray_finish(R, prim_out, t_out, bary_out);
             }
         } else if (live && !in_leaf) {
             live = wide_node<COUNT>(R, T, err, visits, boxes);
             if (live) live = wide_advance(R, T, B, qi, err, s_stack);
-            if (!live) wide_ray_finish(R, i, prim_out, t_out, bary_out);
+            if (!live) wide_ray_finish(R, prim_out, t_out, bary_out);
         }
     }
     add_counts<COUNT>(counts, visits, boxes, tests);
