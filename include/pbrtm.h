@@ -284,8 +284,8 @@ int pbrtm_integrator_from_name(const char *name, uint32_t *flags_out);
 typedef struct pbrtm_render_stats {
     double ms_total, ms_trace, ms_shadow, ms_shade, ms_film;
     uint64_t rounds, rays, shadow_rays, paths;
-    uint32_t ray_order;  /* the ray-order autotuner's choice: bit 0 closest-hit rays sorted, bit 1 shadow rays */
-    uint32_t grid_quarters;  /* the occupancy autotuner's choice: traversal grid in quarters of the maximum */
+    uint32_t ray_order;  /* 0: rays are traced in queue order */
+    uint32_t grid_quarters;  /* 4: the traversal grid is every resident workgroup */
     /* with PBRTM_RENDER_COUNT: [wide nodes visited, child box tests, primitive tests]
        summed over the closest-hit and the shadow traversals (else zero) */
     uint64_t closest_counts[3], shadow_counts[3];
@@ -358,7 +358,7 @@ typedef struct pbrtm_job {
 
 typedef struct pbrtm_batch_params {
     uint32_t pool_size;           /* slots shared by the batch; 0 = 2^24 (capped at the batch's path count) */
-    uint32_t rounds_per_launch;   /* rounds per graph launch between done checks; 0 = 8 */
+    uint32_t rounds_per_launch;   /* rounds per graph launch between done checks (made even); 0 = 8 */
     uint32_t flags;               /* PBRTM_DEVICE_PTRS (films are device pointers), PBRTM_BATCH_NO_GRAPH */
     uint32_t solo_paths;          /* jobs with at least this many paths render alone, before the shared
                                      pool (they fill the GPU by themselves); 0 or 0xFFFFFFFF = never (the

@@ -267,9 +267,8 @@ void pbrtm_destroy(pbrtm_ctx *ctx) {
     auto &p = ctx->batch_pool;
     for (DevBuf *b : {&p.path_id, &p.flags, &p.rng, &p.dim, &p.lam, &p.lam_pdf, &p.L, &p.beta, &p.nee_L, &p.scal,
                       &p.prev, &p.rays, &p.prim, &p.thit, &p.bary, &p.srays, &p.sprim, &p.rec, &p.rec_round,
-                      &p.counters, &p.queue, &p.squeue, &p.spill, &p.job, &p.sround, &ctx->batch_jobs,
-                      &ctx->batch_films, &p.rsort.keys[0], &p.rsort.keys[1], &p.rsort.vals[0], &p.rsort.vals[1],
-                      &p.rsort.hist, &p.rsort.sort.status, &p.rsort.sort.offsets, &p.rsort.sort.counters})
+                      &p.counters, &p.queue, &p.squeue, &p.rayq, &p.spill, &p.job, &p.sround, &ctx->batch_jobs,
+                      &ctx->batch_films})
         b->release();
     for (auto &e : ctx->ev) hipEventDestroy(e);
     for (auto &e : ctx->aux_ev) hipEventDestroy(e);
@@ -749,9 +748,7 @@ void pbrtm_scene_free(pbrtm_scene *sc) {
     auto &p = sc->pool;
     for (pbrtm::DevBuf *b : {&p.path_id, &p.flags, &p.rng, &p.dim, &p.lam, &p.lam_pdf, &p.L, &p.beta, &p.nee_L,
                              &p.scal, &p.prev, &p.rays, &p.prim, &p.thit, &p.bary, &p.srays, &p.sprim, &p.rec,
-                             &p.rec_round, &p.counters, &p.queue, &p.squeue, &p.spill, &p.job, &p.sround,
-                             &p.rsort.keys[0], &p.rsort.keys[1], &p.rsort.vals[0], &p.rsort.vals[1], &p.rsort.hist,
-                             &p.rsort.sort.status, &p.rsort.sort.offsets, &p.rsort.sort.counters})
+                             &p.rec_round, &p.counters, &p.queue, &p.squeue, &p.rayq, &p.spill, &p.job, &p.sround})
         b->release();
     delete sc;
 }
@@ -869,10 +866,6 @@ WideTrace scene_trace(const pbrtm_scene *sc) {
     W.max_depth = bvh->wide.max_depth;
     W.shapes = sc->dev.shapes;
     W.spill_per_ray = W.max_depth > kLdsStack ? W.max_depth - kLdsStack + 1 : 0;
-    for (int a = 0; a < 3; ++a) {
-        W.lo[a] = bvh->bounds[a];
-        W.hi[a] = bvh->bounds[3 + a];
-    }
     return W;
 }
 
@@ -980,8 +973,8 @@ int pbrtm_render(pbrtm_ctx *ctx, pbrtm_scene *sc, const pbrtm_render_params *par
         stats->rays = rs.rays;
         stats->shadow_rays = rs.shadow_rays;
         stats->paths = rs.paths;
-        stats->ray_order = rs.sorted;
-        stats->grid_quarters = rs.grid_quarters;
+        stats->ray_order = 0;      // queue order
+        stats->grid_quarters = 4;  // all resident workgroups
         for (int k = 0; k < 3; ++k) {
             stats->closest_counts[k] = hcounts[k];
             stats->shadow_counts[k] = hcounts[3 + k];

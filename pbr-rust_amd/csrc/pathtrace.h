@@ -142,8 +142,7 @@ bool mat4_inverse_ref(const float in[16], float out[16]);
 
 struct PathPool {
     DevBuf path_id, flags, rng, dim, lam, lam_pdf, L, beta, nee_L, scal, prev, rays, prim, thit, bary, srays, sprim,
-        rec, rec_round, counters, queue, squeue, spill, job, sround;
-    RaySortScratch rsort;
+        rec, rec_round, counters, queue, squeue, rayq, spill, job, sround;
     uint32_t cap = 0;
     uint64_t rec_cap = 0;
 };
@@ -151,8 +150,6 @@ struct PathPool {
 struct RenderStats {
     double ms_total = 0, ms_trace = 0, ms_shadow = 0, ms_shade = 0, ms_film = 0;
     uint64_t rounds = 0, rays = 0, shadow_rays = 0, paths = 0;
-    uint32_t sorted = 0;  // the ray-order autotuner's choice: 1 closest-hit rays sorted, 2 shadow rays sorted
-    uint32_t grid_quarters = 4;  // the occupancy autotuner's choice: traversal grid in quarters of the maximum
 };
 
 // Renders the whole image; film_rgb (device, [h][w][3]) and film_aux (device,

@@ -24,29 +24,32 @@ namespace pt {
 namespace {
 
 constexpr uint32_t kBlock = 256;
-// Ray ordering autotuner: rounds kTuneFirst .. kTuneFirst + 3 alternate sorted
-// and unsorted queues (closest-hit and shadow rays separately); the cheaper
-// time per ray over each pair decides the rest of the render. The film does not
-// depend on the order.
-constexpr uint32_t kTuneFirst = 2;
-// Traversal occupancy autotuner: from round kOccFirst (after the ray order is
-// settled), six rounds give the persistent traversal grids 4, 3, 2, 4, 3, 2
-// quarters of the resident maximum; the least time per traced ray (closest-hit
-// and shadow together) over each pair decides the rest of the render.
-constexpr uint32_t kOccFirst = kTuneFirst + 5;
-constexpr uint32_t kOccQuarters[3] = {4, 3, 2};
 constexpr uint32_t kFlagSpecular = 1u << 16, kFlagAnyNonSpec = 1u << 17, kFlagNee = 1u << 18;
 constexpr uint32_t kDepthMask = 0xFFFFu;
 constexpr uint32_t kIdle = 0xFFFFFFFFu;
 
-// counters[] layout (u32 words); 8..15 hold u64 accumulators of a batched render.
-// A slot holds a live path exactly when its ray is active, so the closest-hit
-// compaction's count (kCntQueue) is the round's live-path count. kCntQueue and
-// kCntSQueue are two words each (the traversal's queue_len), cleared together.
-constexpr int kCntNextId = 0, kCntQueue = 2, kCntSQueue = 4, kCntRound = 6, kCntDone = 7, kCntAccRays = 8;
+// Queues of a round, double buffered by its parity: the live slots (every slot that
+// holds a path; the shading kernel runs over them), the closest-hit rays (by slot; for
+// the path integrators every live slot has one, so that queue is the live list itself)
+// and the shadow rays. The shading kernel of a round appends to the other parity's
+// queues, in runs per workgroup, so that nothing scans the pool for active rays and a
+// pool that drains, or never filled, costs what its live paths cost. (A compaction
+// kernel per ray class and round, and before it a radix sort of all slots, made up
+// 60 % of small renders and batches; ordering the rays by octant and cell saved 2-5 %
+// of the traversal and cost more than that.)
+// counters[] layout (u32 words): per parity a block of kCntBlock words, [kCntLive,
+// kCntShadow] the lengths of the live list and the shadow queue (one u64 for the
+// appends), [kCntRays] the closest-hit queue's where it is a queue of its own, and each
+// length's traversal counter kQueueHead words after it; kCntAccRays: u64 accumulators
+// of a batched render.
+constexpr int kCntNextId = 0, kCntRound = 1, kCntDone = 2, kCntAccRays = 4;
+constexpr int kCntBlock = 8, kCntLive = 0, kCntShadow = 1, kCntRays = 4;
+constexpr int kCntWords = 32;
+__host__ __device__ constexpr int cnt_block(uint32_t parity) { return kCntBlock * (1 + int(parity & 1u)); }
 
 struct State {
     uint32_t *path_id, *flags, *dim;
+    uint32_t *live[2], *rayq[2], *shadowq[2];  // by round parity; rayq: integrators with separate queues only
     uint64_t *rng;
     float4 *lam, *lam_pdf, *L, *beta, *nee_L, *scal, *prev;  // scal = (filter_w, pdf_bsdf, eta_scale, -)
     float4 *rays;                                             // [2 per slot]
@@ -426,36 +429,85 @@ __device__ __forceinline__ void start_path(const SceneDev &S, const State &st, u
     }
 }
 
-__device__ __forceinline__ void idle_slot(const State &st, uint32_t i) {
-    st.path_id[i] = kIdle;
-    st.rays[2 * size_t(i)] = make_float4(0.f, 0.f, 0.f, 0.f);
-}
-
 template <bool GRAD>
 __global__ __launch_bounds__(kBlock) void init_pool_kernel(SceneDev S, State st, Params P) {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= P.pool) return;
-    st.srays[4 * size_t(i)] = make_float4(0.f, 0.f, 0.f, 0.f);
-    st.srays[4 * size_t(i) + 2] = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (uint64_t(i) < P.total)
-        start_path<GRAD>(S, st, P.spd, i, i, i, P.gd.lfin, P.gd.pfin, P.gd.adj, P.gd.g, P.gd.ltot);
-    else idle_slot(st, i);
+    start_path<GRAD>(S, st, P.spd, i, i, i, P.gd.lfin, P.gd.pfin, P.gd.adj, P.gd.g, P.gd.ltot);
+    st.live[0][i] = i;
+    if (st.rayq[0]) st.rayq[0][i] = i;
 }
 
 __global__ __launch_bounds__(kBlock) void init_pool_multi_kernel(State st, Params P) {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= P.pool) return;
-    st.srays[4 * size_t(i)] = make_float4(0.f, 0.f, 0.f, 0.f);
-    st.srays[4 * size_t(i) + 2] = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (uint64_t(i) < P.total) {
-        const uint32_t j = find_job(P, i);
-        const JobDev &J = P.jobs[j];
-        start_path(J.S, st, J.spd, i, i - J.base, i);
-        st.job[i] = j;
-        st.sround[i] = 0;
-    } else {
-        idle_slot(st, i);
+    const uint32_t j = find_job(P, i);
+    const JobDev &J = P.jobs[j];
+    start_path(J.S, st, J.spd, i, i - J.base, i);
+    st.job[i] = j;
+    st.sround[i] = 0;
+    st.live[0][i] = i;
+}
+
+// The counters before round 0: `first` slots hold paths.
+__global__ void init_counters_kernel(uint32_t *counters, uint32_t first) {
+    const int k = threadIdx.x;
+    if (k >= kCntWords) return;
+    const int b = cnt_block(0);
+    counters[k] = (k == kCntNextId || k == b + kCntLive || k == b + kCntRays) ? first : 0u;
+}
+
+// What a slot does after a round of shading.
+constexpr uint32_t kOutLive = 1u, kOutRay = 2u, kOutShadow = 4u;
+
+// Appends the workgroup's slots to the queues of `parity`. Every thread of the workgroup
+// calls this. SEPARATE (the single-vertex integrators): the closest-hit queue is not the
+// live list, and a slot's shadow rays are one instead of two.
+template <bool SEPARATE>
+__device__ __forceinline__ void append_queues(const State &st, uint32_t parity, uint32_t i, uint32_t out) {
+    __shared__ uint32_t s_cnt[3][kBlock / kWave];
+    __shared__ uint32_t s_at[3];
+    const uint32_t wv = threadIdx.x / kWave;
+    const uint64_t live = __ballot((out & kOutLive) != 0u), shadow = __ballot((out & kOutShadow) != 0u);
+    const uint64_t ray = SEPARATE ? __ballot((out & kOutRay) != 0u) : 0ull;
+    if (lane_id() == 0) {
+        s_cnt[0][wv] = uint32_t(__popcll(live));
+        s_cnt[1][wv] = uint32_t(__popcll(shadow));
+        if (SEPARATE) s_cnt[2][wv] = uint32_t(__popcll(ray));
     }
+    __syncthreads();
+    constexpr uint32_t kPer = SEPARATE ? 1u : 2u;  // shadow rays per slot
+    if (threadIdx.x == 0) {
+        uint32_t *c = st.counters + cnt_block(parity);
+        uint32_t n[3] = {0u, 0u, 0u};
+        for (uint32_t k = 0; k < kBlock / kWave; ++k) {
+            n[0] += s_cnt[0][k];
+            n[1] += s_cnt[1][k];
+            if (SEPARATE) n[2] += s_cnt[2][k];
+        }
+        if (n[0]) {
+            const unsigned long long at = atomicAdd(reinterpret_cast<unsigned long long *>(c + kCntLive),
+                                                    (unsigned long long)(n[0]) | ((unsigned long long)(kPer * n[1]) << 32));
+            s_at[0] = uint32_t(at);
+            s_at[1] = uint32_t(at >> 32);
+        }
+        if (SEPARATE) s_at[2] = n[2] ? atomicAdd(c + kCntRays, n[2]) : 0u;
+    }
+    __syncthreads();
+    uint32_t before[3] = {0u, 0u, 0u};
+    for (uint32_t k = 0; k < wv; ++k) {
+        before[0] += s_cnt[0][k];
+        before[1] += s_cnt[1][k];
+        if (SEPARATE) before[2] += s_cnt[2][k];
+    }
+    const uint64_t lt = lanemask_lt();
+    if (out & kOutLive) st.live[parity & 1u][s_at[0] + before[0] + uint32_t(__popcll(live & lt))] = i;
+    if (out & kOutShadow) {
+        const uint32_t at = s_at[1] + kPer * (before[1] + uint32_t(__popcll(shadow & lt)));
+        if (SEPARATE) st.shadowq[parity & 1u][at] = 2u * i;
+        else *reinterpret_cast<uint2 *>(st.shadowq[parity & 1u] + at) = make_uint2(2u * i, 2u * i + 1u);
+    }
+    if (SEPARATE && (out & kOutRay)) st.rayq[parity & 1u][s_at[2] + before[2] + uint32_t(__popcll(ray & lt))] = i;
 }
 
 // One round for slot i: deferred NEE, control_logic, film record, new path,
@@ -476,7 +528,7 @@ __device__ __forceinline__ float dot4(const S4 &a, const S4 &b) {
 // run the megakernel integrators (base/megakernel_integrator.cu:82-147) on the
 // same pool, one round per path vertex.
 template <bool MULTI, bool GRAD, uint32_t MODE = kIntPath>
-__device__ __forceinline__ void shade_impl(const SceneDev &S, const State &st, const Params &P, uint32_t i,
+__device__ __forceinline__ uint32_t shade_impl(const SceneDev &S, const State &st, const Params &P, uint32_t i,
                                            uint32_t pid, uint32_t lid, uint32_t spd, uint32_t max_depth,
                                            uint32_t round, float4 *erec, float4 *grec) {
     const bool live = pid != kIdle;
@@ -486,7 +538,8 @@ __device__ __forceinline__ void shade_impl(const SceneDev &S, const State &st, c
     if (GRAD && live) gadj = f4s(P.gd.g[i]);
     // 1. the previous round's light sample, if both shadow rays missed
     if (live && (fl & kFlagNee)) {
-        if (st.sprim[2 * size_t(i)] == kNoHit && st.sprim[2 * size_t(i) + 1] == kNoHit) {
+        if (st.sprim[2 * size_t(i)] == kNoHit &&
+            (MODE == kIntAmbientOcclusion || st.sprim[2 * size_t(i) + 1] == kNoHit)) {
             L = s4add(L, f4s(st.nee_L[i]));
             if (GRAD) {
                 // C = beta f cos Le w(pmf p) / (pmf p) with w = g^2 / (g^2 + b^2), g = pmf p:
@@ -498,8 +551,10 @@ __device__ __forceinline__ void shade_impl(const SceneDev &S, const State &st, c
         }
         fl &= ~kFlagNee;
     }
-    const uint32_t prim = live ? st.prim[i] : kNoHit;
     const uint32_t depth = fl & kDepthMask;
+    // a single-vertex integrator's second visit has no ray: the path ends
+    const bool traced = live && (MODE <= kIntMegakernelPath || depth == 0);
+    const uint32_t prim = traced ? st.prim[i] : kNoHit;
     bool terminate = live && (prim == kNoHit || depth > max_depth || !s4pos(beta));
     Sampler smp{};
     S4 lam = s4(0.f), lpdf = s4(0.f);
@@ -621,14 +676,10 @@ __device__ __forceinline__ void shade_impl(const SceneDev &S, const State &st, c
             } else {
                 start_path<GRAD>(S, st, spd, i, nid, nid, P.gd.lfin, P.gd.pfin, P.gd.adj, P.gd.g, P.gd.ltot);
             }
-        } else {
-            idle_slot(st, i);
         }
-        st.srays[4 * size_t(i)].w = 0.f;
-        st.srays[4 * size_t(i) + 2].w = 0.f;
-        return;
+        return nid < P.total ? kOutLive | kOutRay : 0u;
     }
-    if (!live) return;
+    if (!live) return 0u;
     const float4 r1 = st.rays[2 * size_t(i) + 1];
     const f3 rd = {r1.x, r1.y, r1.z};
     const uint2 info = S.tri_info[prim];
@@ -674,18 +725,15 @@ __device__ __forceinline__ void shade_impl(const SceneDev &S, const State &st, c
                     d.v[q] = spec_eval_uni(S, S.d65_off, S.d65_n, S.d65_uni, S.d65_inv_step, lam.v[q]) * k;
                 st.nee_L[i] = s4f(d);
                 store_ray(st.srays + 4 * size_t(i), offset_ray_origin(ipi, n, wi), __builtin_inff(), wi);
-                st.srays[4 * size_t(i) + 2].w = 0.f;
                 ao = true;
             }
             if (ao) fl |= kFlagNee;
-            else st.srays[4 * size_t(i)].w = 0.f;
         }
-        st.rays[2 * size_t(i)].w = 0.f;
         st.flags[i] = (fl & ~kDepthMask) | ((depth + 1) & kDepthMask);
         st.L[i] = s4f(L);
         st.rng[i] = smp.rng.state;
         st.dim[i] = smp.dim;
-        return;
+        return (fl & kFlagNee) ? kOutLive | kOutShadow : kOutLive;
     }
     const f3 wo_n = norm3(neg3(rd));
     const uint32_t light = info.y & 0x7FFFFFFFu;
@@ -807,10 +855,6 @@ __device__ __forceinline__ void shade_impl(const SceneDev &S, const State &st, c
         }
     }
     if (nee) fl |= kFlagNee;
-    else {
-        st.srays[4 * size_t(i)].w = 0.f;
-        st.srays[4 * size_t(i) + 2].w = 0.f;
-    }
     // BSDF::sample_f (bsdf.cu:57-80)
     const f3 wo = neg3(rd);
     const float uc = smp.get_1d();
@@ -838,6 +882,16 @@ __device__ __forceinline__ void shade_impl(const SceneDev &S, const State &st, c
     st.scal[i] = scal;
     st.rng[i] = smp.rng.state;
     st.dim[i] = smp.dim;
+    return nee ? kOutLive | kOutRay | kOutShadow : kOutLive | kOutRay;
+}
+
+// The live list's entry of this thread in a round of `parity`, kIdle past its end.
+// `none`: the whole workgroup is past it (uniform).
+__device__ __forceinline__ uint32_t live_slot(const State &st, uint32_t parity, bool *none) {
+    const uint32_t n = st.counters[cnt_block(parity) + kCntLive];
+    *none = blockIdx.x * kBlock >= n;
+    const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
+    return k < n ? st.live[parity & 1u][k] : kIdle;
 }
 
 // The path-integrator shading instances need about 172 VGPRs unbounded (2 waves
@@ -846,23 +900,30 @@ __device__ __forceinline__ void shade_impl(const SceneDev &S, const State &st, c
 
 template <uint32_t MODE>
 __global__ __launch_bounds__(kBlock) PBRTM_SHADE_WAVES void shade_kernel(SceneDev S, State st, Params P) {
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    const uint32_t pid = i < P.pool ? st.path_id[i] : kIdle;
-    shade_impl<false, false, MODE>(S, st, P, i, pid, pid, P.spd, P.max_depth, P.round, nullptr, nullptr);
+    bool none;
+    const uint32_t i = live_slot(st, P.round, &none);
+    if (none) return;
+    const uint32_t pid = i != kIdle ? st.path_id[i] : kIdle;
+    const uint32_t out = shade_impl<false, false, MODE>(S, st, P, i, pid, pid, P.spd, P.max_depth, P.round, nullptr,
+                                                        nullptr);
+    append_queues<(MODE > kIntMegakernelPath)>(st, P.round + 1, i, out);
 }
 
 // The gradient replay of one round (same paths as the forward render).
 constexpr uint32_t kMaxGroups = 255;
 __global__ __launch_bounds__(kBlock) void shade_grad_kernel(SceneDev S, State st, Params P) {
     __shared__ double s_acc[kMaxGroups + 1];
+    bool none;
+    const uint32_t i = live_slot(st, P.round, &none);
+    if (none) return;
     for (uint32_t k = threadIdx.x; k <= P.gd.ngroups; k += kBlock) s_acc[k] = 0.0;
     __syncthreads();
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    const uint32_t pid = i < P.pool ? st.path_id[i] : kIdle;
+    const uint32_t pid = i != kIdle ? st.path_id[i] : kIdle;
     float4 grec = make_float4(0.f, 0.f, 0.f, __uint_as_float(kIdle));
     float4 erec[2] = {make_float4(0.f, 0.f, __uint_as_float(kIdle), 0.f),
                       make_float4(0.f, 0.f, __uint_as_float(kIdle), 0.f)};
-    shade_impl<false, true>(S, st, P, i, pid, pid, P.spd, P.max_depth, P.round, erec, &grec);
+    const uint32_t out = shade_impl<false, true>(S, st, P, i, pid, pid, P.spd, P.max_depth, P.round, erec, &grec);
+    append_queues<false>(st, P.round + 1, i, out);
     // Emitter sums: the pmf part over the whole wave, the scale part per emitter
     // (lanes of one emitter summed first), into shared memory.
     {
@@ -927,15 +988,19 @@ __global__ __launch_bounds__(kBlock) void shade_grad_kernel(SceneDev S, State st
 }
 
 // Batched render: each slot reads its job's scene and parameters; the round
-// number comes from the device counter so the round can be replayed in a graph.
+// number comes from the device counter so the round can be replayed in a graph
+// (P.round gives its parity).
 __global__ __launch_bounds__(kBlock) PBRTM_SHADE_WAVES void shade_multi_kernel(State st, Params P) {
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    const uint32_t pid = i < P.pool ? st.path_id[i] : kIdle;
+    bool none;
+    const uint32_t i = live_slot(st, P.round, &none);
+    if (none) return;
+    const uint32_t pid = i != kIdle ? st.path_id[i] : kIdle;
     const uint32_t j = pid != kIdle ? st.job[i] : 0u;
     const JobDev &J = P.jobs[j];
     const uint32_t lid = pid != kIdle ? uint32_t(pid - J.base) : kIdle;
-    shade_impl<true, false>(J.S, st, P, i, pid, lid, J.spd, J.max_depth, st.counters[kCntRound], nullptr,
-                            nullptr);
+    const uint32_t out = shade_impl<true, false>(J.S, st, P, i, pid, lid, J.spd, J.max_depth, st.counters[kCntRound],
+                                                 nullptr, nullptr);
+    append_queues<false>(st, P.round + 1, i, out);
 }
 
 // Sums the kGradShards copies of the coefficient-derivative table into the first.
@@ -947,24 +1012,30 @@ __global__ __launch_bounds__(kBlock) void reduce_shards_kernel(float *d, uint32_
     d[i] = v;
 }
 
-// Start and end of a batched round (kernels, so that a captured graph holds no memset).
-__global__ void round_begin_kernel(uint32_t *counters) {
-    if (threadIdx.x == 0) {
-        for (int k = kCntQueue; k < kCntSQueue + 2; ++k) counters[k] = 0;
-    }
+// End of a round of a single render: its counters go to the host (pinned memory, read
+// after the round's last event), and its parity's block is cleared for the round after
+// the next one to append to.
+__global__ void round_end_kernel(uint32_t *counters, uint32_t parity, uint32_t *host) {
+    const int k = threadIdx.x;
+    if (k >= kCntWords) return;
+    host[k] = counters[k];
+    const int b = cnt_block(parity);
+    if (k >= b && k < b + kCntBlock) counters[k] = 0u;
 }
-// A round that traced no ray had no live path: the render is over and the round
-// does not count.
-__global__ void round_end_kernel(uint32_t *counters) {
+// End of a batched round (a kernel, so that a captured graph holds no memset). A round
+// without a live path means that the render is over, and does not count.
+__global__ void round_end_multi_kernel(uint32_t *counters, uint32_t parity) {
     if (threadIdx.x != 0 || counters[kCntDone]) return;
-    if (counters[kCntQueue] == 0) {
+    uint32_t *c = counters + cnt_block(parity);
+    if (c[kCntLive] == 0) {
         counters[kCntDone] = 1;
         return;
     }
     unsigned long long *acc = reinterpret_cast<unsigned long long *>(counters + kCntAccRays);
-    acc[0] += counters[kCntQueue];
-    acc[1] += counters[kCntSQueue];
+    acc[0] += c[kCntLive];
+    acc[1] += c[kCntShadow];
     counters[kCntRound] += 1;
+    for (int k = 0; k < kCntBlock; ++k) c[k] = 0u;
 }
 
 // The reference's one-by-one pool schedule for one job (one workgroup per
@@ -1232,7 +1303,7 @@ hipError_t film_adjoint(const SceneDev &S, const float *film_rgb, const float *f
 
 namespace {
 
-hipError_t reserve_pool(PathPool &pp, uint32_t pool, uint64_t total, bool batch) {
+hipError_t reserve_pool(PathPool &pp, uint32_t pool, uint64_t total, bool batch, bool separate_rays) {
     hipError_t e;
 #define PT_CK(x)                          \
     do {                                  \
@@ -1251,10 +1322,11 @@ hipError_t reserve_pool(PathPool &pp, uint32_t pool, uint64_t total, bool batch)
         PT_CK(pp.bary.reserve(size_t(pool) * 12));
         PT_CK(pp.srays.reserve(size_t(pool) * 64));
         PT_CK(pp.sprim.reserve(size_t(pool) * 8));
-        PT_CK(pp.queue.reserve(size_t(pool) * 4));
-        PT_CK(pp.squeue.reserve(size_t(pool) * 8));
+        PT_CK(pp.queue.reserve(size_t(pool) * 2 * 4));   // live slots of both parities
+        PT_CK(pp.squeue.reserve(size_t(pool) * 2 * 8));  // shadow rays of both
         pp.cap = pool;
     }
+    if (separate_rays) PT_CK(pp.rayq.reserve(size_t(pool) * 2 * 4));
     if (batch) {
         PT_CK(pp.job.reserve(size_t(pool) * 4));
         PT_CK(pp.sround.reserve(size_t(pool) * 4));
@@ -1264,13 +1336,18 @@ hipError_t reserve_pool(PathPool &pp, uint32_t pool, uint64_t total, bool batch)
         PT_CK(pp.rec_round.reserve(total * 4));
         pp.rec_cap = total;
     }
-    PT_CK(pp.counters.reserve(64));
+    PT_CK(pp.counters.reserve(kCntWords * sizeof(uint32_t)));
     return hipSuccess;
 #undef PT_CK
 }
 
-State make_state(PathPool &pp, uint32_t *err) {
+State make_state(PathPool &pp, uint32_t *err, uint32_t pool, bool separate_rays) {
     State st{};
+    for (uint32_t k = 0; k < 2; ++k) {
+        st.live[k] = pp.queue.as<uint32_t>() + size_t(k) * pool;
+        st.shadowq[k] = pp.squeue.as<uint32_t>() + size_t(k) * 2 * pool;
+        st.rayq[k] = separate_rays ? pp.rayq.as<uint32_t>() + size_t(k) * pool : nullptr;
+    }
     st.path_id = pp.path_id.as<uint32_t>();
     st.flags = pp.flags.as<uint32_t>();
     st.dim = pp.dim.as<uint32_t>();
@@ -1332,15 +1409,16 @@ hipError_t render(const SceneDev &S, const WideTrace &W0, uint32_t spp, uint32_t
     do {                                  \
         if ((e = (x)) != hipSuccess) return e; \
     } while (0)
-    PT_CK(reserve_pool(pp, pool, total, false));
-    PT_CK(reserve_ray_sort(pp.rsort, 2 * pool));  // sized once: no reallocation while rounds are in flight
+    if (uint64_t(pool) > total) pool = uint32_t(total);  // a slot without a first path never gets one
+    const bool separate_rays = integrator > kIntMegakernelPath;
+    PT_CK(reserve_pool(pp, pool, total, false, separate_rays));
     WideTrace W = W0;
     const uint32_t spill_need = W.spill_per_ray;
     if (spill_need) {
         PT_CK(pp.spill.reserve(size_t(pool) * 2 * spill_need * sizeof(uint2)));
         W.spill = pp.spill.as<uint2>();
     }
-    State st = make_state(pp, err);
+    State st = make_state(pp, err, pool, separate_rays);
     st.lfin = lfin;
     st.pfin = pfin;
     Params P{total, spd, spp, max_depth, 0u, pool, nullptr, nullptr, 0u};
@@ -1356,7 +1434,7 @@ hipError_t render(const SceneDev &S, const WideTrace &W0, uint32_t spp, uint32_t
     hipEvent_t ev[kEv];
     for (auto &x : ev) PT_CK(hipEventCreate(&x));
     uint32_t *hc = nullptr;  // pinned: the counters of two rounds
-    PT_CK(hipHostMalloc(reinterpret_cast<void **>(&hc), 2 * 16 * sizeof(uint32_t), hipHostMallocDefault));
+    PT_CK(hipHostMalloc(reinterpret_cast<void **>(&hc), 2 * kCntWords * sizeof(uint32_t), hipHostMallocDefault));
     struct EvGuard {
         hipEvent_t *e;
         uint32_t *h;
@@ -1367,24 +1445,13 @@ hipError_t render(const SceneDev &S, const WideTrace &W0, uint32_t spp, uint32_t
             hipHostFree(h);
         }
     } guard{ev, hc, stream};
-    PT_CK(hipMemsetAsync(st.counters, 0, 64, stream));
-    uint32_t first = uint32_t(std::min<uint64_t>(total, pool));
-    PT_CK(hipMemcpyAsync(st.counters + kCntNextId, &first, 4, hipMemcpyHostToDevice, stream));
-    uint64_t next_before = first;  // paths started before the current round
+    init_counters_kernel<<<1, 64, 0, stream>>>(st.counters, pool);
     PT_CK(hipEventRecord(ev[0], stream));
     if (gd) init_pool_kernel<true><<<grid, kBlock, 0, stream>>>(S, st, P);
     else init_pool_kernel<false><<<grid, kBlock, 0, stream>>>(S, st, P);
     PT_CK(hipGetLastError());
     RenderStats rs;
     float t_trace = 0, t_shadow = 0, t_shade = 0;
-    struct {
-        bool sort_closest = true, sort_shadow = true;
-        double ms[2][2] = {{0, 0}, {0, 0}};
-        uint64_t rays[2][2] = {{0, 0}, {0, 0}};
-        uint32_t quarters = 4;
-        double occ_ms[3] = {0, 0, 0};
-        uint64_t occ_rays[3] = {0, 0, 0};
-    } tune;
     // One round: both traces and the shading kernel, then the counters to the host.
     // Round r + 1 is enqueued before round r's counters are read, so the device
     // does not wait for the host between rounds; when round r turns out to be the
@@ -1393,40 +1460,16 @@ hipError_t render(const SceneDev &S, const WideTrace &W0, uint32_t spp, uint32_t
         hipError_t e;
         hipEvent_t *E = ev + 3 + 5 * (round & 1);
         P.round = round;
-        PT_CK(hipMemsetAsync(st.counters + kCntQueue, 0, 16, stream));
+        const uint32_t par = round & 1u;
+        uint32_t *c = st.counters + cnt_block(par);
         PT_CK(hipEventRecord(E[0], stream));
-        const bool tuning = round >= kTuneFirst && round < kTuneFirst + 4;
-        const bool sort_c = tuning ? ((round - kTuneFirst) % 2 == 0) : tune.sort_closest;
-        const bool sort_s = tuning ? ((round - kTuneFirst) % 2 == 0) : tune.sort_shadow;
-        const bool occ_tuning = round >= kOccFirst && round < kOccFirst + 6;
-        W.grid_quarters = occ_tuning ? kOccQuarters[(round - kOccFirst) % 3] : tune.quarters;
-        if (sort_c) {  // closest-hit rays in (octant, origin Morton code) order
-            uint32_t *q = nullptr;
-            PT_CK(sort_rays(W, reinterpret_cast<const float *>(st.rays), pool, pp.prim.as<uint32_t>(),
-                            pp.thit.as<float>(), pp.bary.as<float>(), err, pp.rsort, st.counters + kCntQueue, &q,
-                            stream));
-            PT_CK(trace_wide_queued(W, reinterpret_cast<const float *>(st.rays), pool, 0, pp.prim.as<uint32_t>(),
-                                    pp.thit.as<float>(), pp.bary.as<float>(), err, q, st.counters + kCntQueue,
-                                    stream, counts));
-        } else {
-            PT_CK(trace_wide(W, reinterpret_cast<const float *>(st.rays), pool, 0, pp.prim.as<uint32_t>(),
-                             pp.thit.as<float>(), pp.bary.as<float>(), err, counts, pp.queue.as<uint32_t>(),
-                             st.counters + kCntQueue, stream));
-        }
+        PT_CK(trace_wide_queued(W, reinterpret_cast<const float *>(st.rays), pool, 0, pp.prim.as<uint32_t>(),
+                                pp.thit.as<float>(), pp.bary.as<float>(), err, separate_rays ? st.rayq[par] : st.live[par],
+                                c + (separate_rays ? kCntRays : kCntLive), stream, counts));
         PT_CK(hipEventRecord(E[1], stream));
-        if (spill_need) W.spill = pp.spill.as<uint2>();
-        if (sort_s) {
-            uint32_t *q = nullptr;
-            PT_CK(sort_rays(W, reinterpret_cast<const float *>(st.srays), 2 * pool, pp.sprim.as<uint32_t>(), nullptr,
-                            nullptr, err, pp.rsort, st.counters + kCntSQueue, &q, stream));
-            PT_CK(trace_wide_queued(W, reinterpret_cast<const float *>(st.srays), 2 * pool, 1,
-                                    pp.sprim.as<uint32_t>(), nullptr, nullptr, err, q, st.counters + kCntSQueue,
-                                    stream, counts ? counts + 3 : nullptr));
-        } else {
-            PT_CK(trace_wide(W, reinterpret_cast<const float *>(st.srays), 2 * pool, 1, pp.sprim.as<uint32_t>(),
-                             nullptr, nullptr, err, counts ? counts + 3 : nullptr, pp.squeue.as<uint32_t>(),
-                             st.counters + kCntSQueue, stream));
-        }
+        PT_CK(trace_wide_queued(W, reinterpret_cast<const float *>(st.srays), 2 * pool, 1, pp.sprim.as<uint32_t>(),
+                                nullptr, nullptr, err, st.shadowq[par], c + kCntShadow, stream,
+                                counts ? counts + 3 : nullptr));
         PT_CK(hipEventRecord(E[2], stream));
         if (gd) shade_grad_kernel<<<grid, kBlock, 0, stream>>>(S, st, P);
         else if (integrator == kIntMegakernelPath) shade_kernel<kIntMegakernelPath><<<grid, kBlock, 0, stream>>>(S, st, P);
@@ -1436,7 +1479,8 @@ hipError_t render(const SceneDev &S, const WideTrace &W0, uint32_t spp, uint32_t
         else shade_kernel<kIntPath><<<grid, kBlock, 0, stream>>>(S, st, P);
         PT_CK(hipGetLastError());
         PT_CK(hipEventRecord(E[3], stream));
-        PT_CK(hipMemcpyAsync(hc + 16 * (round & 1), st.counters, 32, hipMemcpyDeviceToHost, stream));
+        round_end_kernel<<<1, 64, 0, stream>>>(st.counters, par, hc + kCntWords * par);
+        PT_CK(hipGetLastError());
         PT_CK(hipEventRecord(E[4], stream));
         return hipSuccess;
     };
@@ -1446,15 +1490,8 @@ hipError_t render(const SceneDev &S, const WideTrace &W0, uint32_t spp, uint32_t
         PT_CK(enqueue(r + 1));
         hipEvent_t *E = ev + 3 + 5 * (r & 1);
         PT_CK(hipEventSynchronize(E[4]));
-        const uint32_t *host_cnt = hc + 16 * (r & 1);
-        // Done when no ray was traced and no path could start: every live slot then
-        // ended this round. A wavefront path always has a ray, so there this round
-        // had no live path and does not count; the megakernel integrators' single-
-        // vertex paths retire their ray a round before they end, and that last
-        // round's shadow rays and film records do count.
-        const bool done = host_cnt[kCntQueue] == 0 && next_before >= total;
-        if (done && integrator == kIntPath) break;
-        next_before = host_cnt[kCntNextId];
+        const uint32_t *cnt = hc + kCntWords * (r & 1) + cnt_block(r);
+        if (cnt[kCntLive] == 0) break;  // no live path: the render is over, and this round does not count
         float a, b, c;
         hipEventElapsedTime(&a, E[0], E[1]);
         hipEventElapsedTime(&b, E[1], E[2]);
@@ -1462,38 +1499,9 @@ hipError_t render(const SceneDev &S, const WideTrace &W0, uint32_t spp, uint32_t
         t_trace += a;
         t_shadow += b;
         t_shade += c;
-        if (r >= kTuneFirst && r < kTuneFirst + 4) {
-            const int k = (r - kTuneFirst) % 2;  // 0 sorted, 1 unsorted
-            tune.ms[0][k] += a;
-            tune.rays[0][k] += host_cnt[kCntQueue];
-            tune.ms[1][k] += b;
-            tune.rays[1][k] += host_cnt[kCntSQueue];
-            if (r == kTuneFirst + 3) {
-                auto faster_sorted = [&](int q) {
-                    return tune.rays[q][0] && tune.rays[q][1] &&
-                           tune.ms[q][0] / double(tune.rays[q][0]) < tune.ms[q][1] / double(tune.rays[q][1]);
-                };
-                tune.sort_closest = faster_sorted(0);
-                tune.sort_shadow = faster_sorted(1);
-            }
-        }
-        if (r >= kOccFirst && r < kOccFirst + 6) {
-            const int k = (r - kOccFirst) % 3;
-            tune.occ_ms[k] += a + b;
-            tune.occ_rays[k] += uint64_t(host_cnt[kCntQueue]) + host_cnt[kCntSQueue];
-            if (r == kOccFirst + 5) {
-                int best = 0;
-                for (int q = 1; q < 3; ++q)
-                    if (tune.occ_rays[q] && tune.occ_rays[best] &&
-                        tune.occ_ms[q] / double(tune.occ_rays[q]) < tune.occ_ms[best] / double(tune.occ_rays[best]))
-                        best = q;
-                tune.quarters = kOccQuarters[best];
-            }
-        }
-        rs.rays += host_cnt[kCntQueue];
-        rs.shadow_rays += host_cnt[kCntSQueue];
+        rs.rays += cnt[separate_rays ? kCntRays : kCntLive];
+        rs.shadow_rays += cnt[kCntShadow];
         ++r;
-        if (done) break;
         if (r > 100000) return hipErrorUnknown;
     }
     P.round = r;
@@ -1518,8 +1526,6 @@ hipError_t render(const SceneDev &S, const WideTrace &W0, uint32_t spp, uint32_t
     rs.ms_shade = t_shade;
     rs.ms_film = tf;
     rs.rounds = P.round;
-    rs.sorted = (tune.sort_closest ? 1u : 0u) | (tune.sort_shadow ? 2u : 0u);
-    rs.grid_quarters = tune.quarters;
     rs.paths = total;
     if (stats) *stats = rs;
     return hipSuccess;
@@ -1565,8 +1571,8 @@ hipError_t render_shared(const std::vector<BatchJob> &jobs, uint32_t pool, uint3
     do {                                  \
         if ((e = (x)) != hipSuccess) return e; \
     } while (0)
-    PT_CK(reserve_pool(pp, pool, total, true));
-    PT_CK(reserve_ray_sort(pp.rsort, 2 * pool));  // the captured rounds allocate nothing
+    PT_CK(reserve_pool(pp, pool, total, true, false));  // the captured rounds allocate nothing
+    rounds_per_launch += rounds_per_launch & 1u;         // the queues' parity is the round's within a launch
     WideTrace W{};
     W.spill_per_ray = spill_need;
     W.grid_quarters = grid_quarters;
@@ -1587,7 +1593,7 @@ hipError_t render_shared(const std::vector<BatchJob> &jobs, uint32_t pool, uint3
     PT_CK(hipMemcpyAsync(jb, jd.data(), nj * sizeof(JobDev), hipMemcpyHostToDevice, stream));
     PT_CK(hipMemcpyAsync(jb + off_jw, jw.data(), nj * sizeof(WideTrace), hipMemcpyHostToDevice, stream));
     PT_CK(hipMemcpyAsync(jb + off_base, base.data(), (nj + 1) * sizeof(uint64_t), hipMemcpyHostToDevice, stream));
-    const State st = make_state(pp, err);
+    const State st = make_state(pp, err, pool, false);
     Params P{total, 0u, 0u, 0u, 0u, pool, d_jobs, d_base, nj};
     const uint32_t grid = (pool + kBlock - 1) / kBlock;
     hipEvent_t ev[4];
@@ -1604,37 +1610,25 @@ hipError_t render_shared(const std::vector<BatchJob> &jobs, uint32_t pool, uint3
             if (*g) hipGraphDestroy(*g);
         }
     } guard{ev, &graph, &exec};
-    PT_CK(hipMemsetAsync(st.counters, 0, 64, stream));
-    const uint32_t first = pool;
-    PT_CK(hipMemcpyAsync(st.counters + kCntNextId, &first, 4, hipMemcpyHostToDevice, stream));
+    init_counters_kernel<<<1, 64, 0, stream>>>(st.counters, pool);
     PT_CK(hipEventRecord(ev[0], stream));
     init_pool_multi_kernel<<<grid, kBlock, 0, stream>>>(st, P);
     PT_CK(hipGetLastError());
     auto enqueue_rounds = [&]() -> hipError_t {
         hipError_t e2;
         for (uint32_t k = 0; k < rounds_per_launch; ++k) {
-            round_begin_kernel<<<1, 64, 0, stream>>>(st.counters);
-            if ((e2 = hipGetLastError()) != hipSuccess) return e2;
-            // both ray classes in (job, octant, origin Morton code) order
-            uint32_t *q = nullptr;
-            if ((e2 = sort_rays(W, reinterpret_cast<const float *>(st.rays), pool, pp.prim.as<uint32_t>(),
-                                pp.thit.as<float>(), pp.bary.as<float>(), err, pp.rsort, st.counters + kCntQueue, &q,
-                                stream, st.job, 0)) != hipSuccess)
-                return e2;
+            P.round = k;
+            uint32_t *c = st.counters + cnt_block(k);
             if ((e2 = trace_wide_multi_queued(W, d_jw, st.job, 0, reinterpret_cast<const float *>(st.rays), pool, 0,
                                               pp.prim.as<uint32_t>(), pp.thit.as<float>(), pp.bary.as<float>(), err,
-                                              q, st.counters + kCntQueue, stream)) != hipSuccess)
-                return e2;
-            if ((e2 = sort_rays(W, reinterpret_cast<const float *>(st.srays), 2 * pool, pp.sprim.as<uint32_t>(),
-                                nullptr, nullptr, err, pp.rsort, st.counters + kCntSQueue, &q, stream, st.job, 1)) !=
-                hipSuccess)
+                                              st.live[k & 1u], c + kCntLive, stream)) != hipSuccess)
                 return e2;
             if ((e2 = trace_wide_multi_queued(W, d_jw, st.job, 1, reinterpret_cast<const float *>(st.srays),
-                                              2 * pool, 1, pp.sprim.as<uint32_t>(), nullptr, nullptr, err, q,
-                                              st.counters + kCntSQueue, stream)) != hipSuccess)
+                                              2 * pool, 1, pp.sprim.as<uint32_t>(), nullptr, nullptr, err,
+                                              st.shadowq[k & 1u], c + kCntShadow, stream)) != hipSuccess)
                 return e2;
             shade_multi_kernel<<<grid, kBlock, 0, stream>>>(st, P);
-            round_end_kernel<<<1, 64, 0, stream>>>(st.counters);
+            round_end_multi_kernel<<<1, 64, 0, stream>>>(st.counters, k);
             if ((e2 = hipGetLastError()) != hipSuccess) return e2;
         }
         return hipSuccess;
@@ -1649,7 +1643,7 @@ hipError_t render_shared(const std::vector<BatchJob> &jobs, uint32_t pool, uint3
         PT_CK(ee);
         PT_CK(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
     }
-    uint32_t host_cnt[16] = {};
+    uint32_t host_cnt[kCntWords] = {};
     uint32_t launches = 0;
     // Every path ends within max_depth + 2 rounds of its start, so the pool drains in
     // at most (paths / pool + 1) * (max depth + 2) rounds.
@@ -1660,7 +1654,7 @@ hipError_t render_shared(const std::vector<BatchJob> &jobs, uint32_t pool, uint3
         if (use_graph) PT_CK(hipGraphLaunch(exec, stream));
         else PT_CK(enqueue_rounds());
         ++launches;
-        PT_CK(hipMemcpyAsync(host_cnt, st.counters, 64, hipMemcpyDeviceToHost, stream));
+        PT_CK(hipMemcpyAsync(host_cnt, st.counters, sizeof(host_cnt), hipMemcpyDeviceToHost, stream));
         PT_CK(hipStreamSynchronize(stream));
         if (host_cnt[kCntDone]) break;
         if (uint64_t(launches) * rounds_per_launch > round_cap) return hipErrorUnknown;

@@ -182,7 +182,7 @@ __global__ __launch_bounds__(kSortBlock) void onesweep_pass_kernel(
 
 }  // namespace
 
-hipError_t onesweep_reserve(SortScratch &s, uint32_t n) {
+static hipError_t onesweep_reserve(SortScratch &s, uint32_t n) {
     const uint32_t tiles = sort_tiles(n);
     const uint64_t status_words = uint64_t(tiles) * kSortRadix * kSortPasses;
     hipError_t e = s.status.reserve(status_words * sizeof(uint32_t));
@@ -194,13 +194,6 @@ hipError_t onesweep_reserve(SortScratch &s, uint32_t n) {
 hipError_t onesweep_sort_30(uint32_t *keys0, uint32_t *vals0, uint32_t *keys1, uint32_t *vals1,
                             uint32_t n, const uint32_t *hist, uint32_t *err, SortScratch &s,
                             hipStream_t stream, uint32_t **keys_result, uint32_t **vals_result) {
-    return onesweep_sort(keys0, vals0, keys1, vals1, n, hist, err, s, stream, keys_result, vals_result, kSortPasses);
-}
-
-hipError_t onesweep_sort(uint32_t *keys0, uint32_t *vals0, uint32_t *keys1, uint32_t *vals1, uint32_t n,
-                         const uint32_t *hist, uint32_t *err, SortScratch &s, hipStream_t stream,
-                         uint32_t **keys_result, uint32_t **vals_result, uint32_t passes) {
-    if (passes == 0 || passes > kSortPasses) return hipErrorInvalidValue;
     *keys_result = keys0;
     *vals_result = vals0;
     if (n == 0) return hipSuccess;
@@ -215,7 +208,7 @@ hipError_t onesweep_sort(uint32_t *keys0, uint32_t *vals0, uint32_t *keys1, uint
     fill_u32_kernel<<<1, 64, 0, stream>>>(counters, 64, 0u);
     digit_offsets_kernel<<<1, kSortRadix, 0, stream>>>(hist, offsets);
     uint32_t *kin = keys0, *vin = vals0, *kout = keys1, *vout = vals1;
-    for (uint32_t p = 0; p < passes; ++p) {
+    for (uint32_t p = 0; p < kSortPasses; ++p) {
         if (sort_items(n) == kSortItemsLarge)
             onesweep_pass_kernel<kSortItemsLarge><<<tiles, kSortBlock, 0, stream>>>(
                 kin, vin, kout, vout, n, p * kSortRadixBits, offsets + p * kSortRadix,
@@ -227,7 +220,7 @@ hipError_t onesweep_sort(uint32_t *keys0, uint32_t *vals0, uint32_t *keys1, uint
         std::swap(kin, kout);
         std::swap(vin, vout);
     }
-    *keys_result = kin;  // an odd pass count leaves the result in buffer 1, an even one in buffer 0
+    *keys_result = kin;  // three passes: buffer 1
     *vals_result = vin;
     return hipGetLastError();
 }

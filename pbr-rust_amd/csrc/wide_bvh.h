@@ -54,41 +54,21 @@ struct WideTrace {
     uint32_t num_nodes, num_prims, max_depth;
     uint2 *spill;           // per-ray stack overflow area (max_depth - kLdsStack entries per ray), may be null
     uint32_t spill_per_ray;
-    float lo[3], hi[3];     // bounds of the whole tree (ray ordering)
     uint32_t grid_quarters; // persistent traversal grid: this many quarters of the resident maximum (0 = all)
 };
 
 // counts (device, nullable): adds [wide nodes visited, child box tests, triangle tests].
-// queue (device, n entries) and queue_len (device, two words, both zeroed by the
-// caller) hold the compacted active rays: queue_len[0] their number, queue_len[1]
-// the traversal's counter of runs handed out.
+// queue (device, n entries) and queue_len (device, the two words [0] and [kQueueHead]
+// zeroed by the caller) hold the compacted active rays: queue_len[0] their number,
+// queue_len[kQueueHead] the traversal's counter of rows handed out.
+constexpr int kQueueHead = 2;
 hipError_t trace_wide(const WideTrace &B, const float *rays, uint32_t n, int any_hit, uint32_t *prim_out,
                       float *t_out, float *bary_out, uint32_t *err, unsigned long long *counts, uint32_t *queue,
                       uint32_t *queue_len, hipStream_t stream);
 
-// As trace_wide, for rays of several jobs: ray i is traced against jobs[ray_job[i >> job_shift]]
-// (nodes, order, tri_leaf, prim_order, num_nodes, num_prims); B supplies the spill area.
-hipError_t trace_wide_multi(const WideTrace &B, const WideTrace *jobs, const uint32_t *ray_job, uint32_t job_shift,
-                            const float *rays, uint32_t n, int any_hit, uint32_t *prim_out, float *t_out,
-                            float *bary_out, uint32_t *err, uint32_t *queue, uint32_t *queue_len,
-                            hipStream_t stream);
-
-// Orders the active rays of [n] by (direction octant, Morton code of the origin
-// on a 64^3 grid over the tree's box; 20-bit keys, two radix passes) into *queue
-// (a pointer into the scratch, n words) and counts them into *queue_len (two
-// words, zeroed by the caller, as above); inactive rays report a miss. trace_wide_queued then traces that
-// queue.
-struct RaySortScratch {
-    DevBuf keys[2], vals[2], hist;
-    SortScratch sort;
-};
-// ray_job (nullable): rays of a batch, ray i of job ray_job[i >> job_shift]; the
-// job then leads the key (three radix passes). Every step is a kernel (no memset),
-// so that a graph may capture the call once reserve_ray_sort has sized the scratch.
-hipError_t sort_rays(const WideTrace &B, const float *rays, uint32_t n, uint32_t *prim_out, float *t_out,
-                     float *bary_out, uint32_t *err, RaySortScratch &s, uint32_t *queue_len, uint32_t **queue,
-                     hipStream_t stream, const uint32_t *ray_job = nullptr, uint32_t job_shift = 0);
-hipError_t reserve_ray_sort(RaySortScratch &s, uint32_t n);
+// The rays of a queue filled by the caller (queue_len[0] of at most n entries). Ray i of
+// several jobs is traced against jobs[ray_job[i >> job_shift]] (nodes, order, tri_leaf,
+// prim_order, num_nodes, num_prims); B supplies the spill area.
 hipError_t trace_wide_multi_queued(const WideTrace &B, const WideTrace *jobs, const uint32_t *ray_job,
                                    uint32_t job_shift, const float *rays, uint32_t n, int any_hit, uint32_t *prim_out,
                                    float *t_out, float *bary_out, uint32_t *err, const uint32_t *queue,

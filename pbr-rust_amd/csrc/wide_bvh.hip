@@ -744,7 +744,7 @@ __device__ __forceinline__ void add_counts(unsigned long long *counts, uint32_t 
 // kRefill lanes are idle, so that the waves keep most lanes busy instead of waiting
 // for their slowest ray. The first kDealt eighths of the queue are dealt out (wave w
 // takes row w of every `waves` rows); the rest goes row by row to whichever wave asks
-// next (queue_len[1]), so that no wave is left with more work than the others. One
+// next (queue_len[kQueueHead]), so that no wave is left with more work than the others. One
 // counter serves the atomics at some 6 ns each, which is why not all rows go that way
 // and none is shorter (1080p camera rays into 10M triangles: all dealt 1294 us, none
 // 1109, 5/8 1032, 5/8 with rows of 32 at the end 1121; 33M paths of a path-traced
@@ -815,7 +815,7 @@ __device__ __forceinline__ void trace_wide_persistent_body(const WideTrace &B, c
             } else if (left == 0) {  // the next row of the rest
                 rows = 1;
                 uint32_t row = 0;
-                if (lane == 0) row = atomicAdd(&queue_len[1], 1u);
+                if (lane == 0) row = atomicAdd(&queue_len[kQueueHead], 1u);
                 const uint64_t at = dealt + uint64_t(__builtin_amdgcn_readfirstlane(row)) * kWave;
                 more = at < n;
                 if (more) {
@@ -1022,112 +1022,6 @@ hipError_t trace_wide(const WideTrace &B, const float *rays, uint32_t n, int any
                                     stream);
 }
 
-namespace {
-
-__device__ __forceinline__ uint32_t spread3_6(uint32_t v) {  // 6 bits -> every third bit
-    v &= 0x3Fu;
-    v = (v | (v << 16)) & 0x030000FFu;
-    v = (v | (v << 8)) & 0x0300F00Fu;
-    v = (v | (v << 4)) & 0x030C30C3u;
-    v = (v | (v << 2)) & 0x09249249u;
-    return v;
-}
-
-// MULTI: rays of a batch; the ray's job (low 10 bits) leads the key so that a
-// wave's rays share a tree, and the keys take three radix passes.
-template <bool MULTI>
-__global__ __launch_bounds__(256) void ray_keys_kernel(const float4 *__restrict__ rays, uint32_t n, WideTrace B,
-                                                       uint32_t *__restrict__ keys, uint32_t *__restrict__ vals,
-                                                       uint32_t *__restrict__ hist, uint32_t *__restrict__ count,
-                                                       uint32_t *__restrict__ prim_out, float *__restrict__ t_out,
-                                                       float *__restrict__ bary_out,
-                                                       const uint32_t *__restrict__ ray_job, uint32_t job_shift) {
-    __shared__ uint32_t s_hist[kSortPasses * kSortRadix];
-    for (int i = threadIdx.x; i < int(kSortPasses * kSortRadix); i += blockDim.x) s_hist[i] = 0u;
-    __syncthreads();
-    const float sx = B.hi[0] > B.lo[0] ? 64.f / (B.hi[0] - B.lo[0]) : 0.f;
-    const float sy = B.hi[1] > B.lo[1] ? 64.f / (B.hi[1] - B.lo[1]) : 0.f;
-    const float sz = B.hi[2] > B.lo[2] ? 64.f / (B.hi[2] - B.lo[2]) : 0.f;
-    uint32_t mine = 0;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const float4 r0 = rays[2 * size_t(i)];
-        // inactive: after every active ray (active keys are < 2^19, or < 2^30 with jobs)
-        uint32_t key = MULTI ? 0x3FFFFFFFu : 0xFFFFFu;
-        if (r0.w > 0.f) {
-            const float4 r1 = rays[2 * size_t(i) + 1];
-            const uint32_t qx = uint32_t(fminf(63.f, fmaxf(0.f, (r0.x - B.lo[0]) * sx)));
-            const uint32_t qy = uint32_t(fminf(63.f, fmaxf(0.f, (r0.y - B.lo[1]) * sy)));
-            const uint32_t qz = uint32_t(fminf(63.f, fmaxf(0.f, (r0.z - B.lo[2]) * sz)));
-            const uint32_t oct = (r1.x < 0.f ? 1u : 0u) | (r1.y < 0.f ? 2u : 0u) | (r1.z < 0.f ? 4u : 0u);
-            const uint32_t m = (spread3_6(qx) << 2) | (spread3_6(qy) << 1) | spread3_6(qz);  // 18 bits
-            key = (oct << 16) | (m >> 2);  // < 2^19: below the inactive key, two sort passes
-            if (MULTI) key |= (ray_job[i >> job_shift] & 1023u) << 19;
-            ++mine;
-        } else {
-            prim_out[i] = kNoHit;
-            if (t_out) t_out[i] = 0.f;
-            if (bary_out) {
-                bary_out[3 * size_t(i)] = 0.f;
-                bary_out[3 * size_t(i) + 1] = 0.f;
-                bary_out[3 * size_t(i) + 2] = 0.f;
-            }
-        }
-        keys[i] = key;
-        vals[i] = i;
-        atomicAdd(&s_hist[key & 1023u], 1u);
-        atomicAdd(&s_hist[kSortRadix + ((key >> 10) & 1023u)], 1u);
-        if (MULTI) atomicAdd(&s_hist[2 * kSortRadix + ((key >> 20) & 1023u)], 1u);
-    }
-    const uint32_t tot = wave_sum(mine);
-    if (__lane_id() == 0 && tot) atomicAdd(count, tot);
-    __syncthreads();
-    for (int i = threadIdx.x; i < int(kSortPasses * kSortRadix); i += blockDim.x)
-        if (s_hist[i]) atomicAdd(&hist[i], s_hist[i]);
-}
-
-__global__ void zero_hist_kernel(uint32_t *h) {
-    for (uint32_t i = threadIdx.x; i < kSortPasses * kSortRadix; i += blockDim.x) h[i] = 0u;
-}
-
-}  // namespace
-
-hipError_t reserve_ray_sort(RaySortScratch &s, uint32_t n) {
-    hipError_t e = hipSuccess;
-    for (int k = 0; k < 2 && e == hipSuccess; ++k) {
-        e = s.keys[k].reserve(size_t(n) * 4);
-        if (e == hipSuccess) e = s.vals[k].reserve(size_t(n) * 4);
-    }
-    if (e == hipSuccess) e = s.hist.reserve(kSortPasses * kSortRadix * 4);
-    if (e == hipSuccess) e = onesweep_reserve(s.sort, n);
-    return e;
-}
-
-hipError_t sort_rays(const WideTrace &B, const float *rays, uint32_t n, uint32_t *prim_out, float *t_out,
-                     float *bary_out, uint32_t *err, RaySortScratch &s, uint32_t *queue_len, uint32_t **queue,
-                     hipStream_t stream, const uint32_t *ray_job, uint32_t job_shift) {
-    hipError_t e = reserve_ray_sort(s, n);
-    if (e != hipSuccess) return e;
-    *queue = s.vals[0].as<uint32_t>();
-    if (n == 0) return hipSuccess;
-    zero_hist_kernel<<<1, 256, 0, stream>>>(s.hist.as<uint32_t>());  // a kernel, so that a graph may capture it
-    const uint32_t grid = std::min((n + 255) / 256, 1024u);
-    const float4 *r = reinterpret_cast<const float4 *>(rays);
-    if (ray_job)
-        ray_keys_kernel<true><<<grid, 256, 0, stream>>>(r, n, B, s.keys[0].as<uint32_t>(), s.vals[0].as<uint32_t>(),
-                                                        s.hist.as<uint32_t>(), queue_len, prim_out, t_out, bary_out,
-                                                        ray_job, job_shift);
-    else
-        ray_keys_kernel<false><<<grid, 256, 0, stream>>>(r, n, B, s.keys[0].as<uint32_t>(), s.vals[0].as<uint32_t>(),
-                                                         s.hist.as<uint32_t>(), queue_len, prim_out, t_out,
-                                                         bary_out, nullptr, 0);
-    uint32_t *kr = nullptr, *vr = nullptr;
-    e = onesweep_sort(s.keys[0].as<uint32_t>(), s.vals[0].as<uint32_t>(), s.keys[1].as<uint32_t>(),
-                      s.vals[1].as<uint32_t>(), n, s.hist.as<uint32_t>(), err, s.sort, stream, &kr, &vr,
-                      ray_job ? 3u : 2u);
-    *queue = vr;
-    return e;
-}
-
 hipError_t trace_wide_multi_queued(const WideTrace &B, const WideTrace *jobs, const uint32_t *ray_job,
                                    uint32_t job_shift, const float *rays, uint32_t n, int any_hit, uint32_t *prim_out,
                                    float *t_out, float *bary_out, uint32_t *err, const uint32_t *queue,
@@ -1143,18 +1037,6 @@ hipError_t trace_wide_queued(const WideTrace &B, const float *rays, uint32_t n, 
     if (n == 0) return hipSuccess;
     return trace_wide_queued_counts(B, reinterpret_cast<const float4 *>(rays), n, any_hit, prim_out, t_out, bary_out,
                                     err, counts, queue, queue_len, stream);
-}
-
-hipError_t trace_wide_multi(const WideTrace &B, const WideTrace *jobs, const uint32_t *ray_job, uint32_t job_shift,
-                            const float *rays, uint32_t n, int any_hit, uint32_t *prim_out, float *t_out,
-                            float *bary_out, uint32_t *err, uint32_t *queue, uint32_t *queue_len,
-                            hipStream_t stream) {
-    if (n == 0) return hipSuccess;
-    const uint32_t cgrid = (n + kCompactBlock * kCompactItems - 1) / (kCompactBlock * kCompactItems);
-    const float4 *r = reinterpret_cast<const float4 *>(rays);
-    compact_rays_kernel<<<cgrid, kCompactBlock, 0, stream>>>(r, n, queue, queue_len, prim_out, t_out, bary_out);
-    return launch_multi(B, jobs, ray_job, job_shift, r, n, any_hit, prim_out, t_out, bary_out, err, queue, queue_len,
-                        stream);
 }
 
 }  // namespace pbrtm
