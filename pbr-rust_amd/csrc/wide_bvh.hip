@@ -739,8 +739,8 @@ __device__ __forceinline__ void add_counts(unsigned long long *counts, uint32_t 
     }
 }
 
-// Persistent traversal: a grid that fills the GPU once; every wave takes rows of kWave
-// queue slots, and a lane whose ray has finished takes the row's next slot as soon as
+// Persistent traversal: a grid that fills the GPU once; every wave takes rows of up to
+// kWave queue slots (wide_row), and a lane whose ray has finished takes the row's next slot as soon as
 // kRefill lanes are idle, so that the waves keep most lanes busy instead of waiting
 // for their slowest ray. The first kDealt eighths of the queue are dealt out (wave w
 // takes row w of every `waves` rows); the rest goes row by row to whichever wave asks
@@ -754,6 +754,18 @@ __device__ __forceinline__ void add_counts(unsigned long long *counts, uint32_t 
 // tree, jw[ray_job[i >> job_shift]] (jobs of a batched render); the spill area
 // stays the launch's.
 constexpr uint32_t kRefill = 8;
+constexpr uint32_t kWideWaves = kWideBlock / kWave;
+// Slots of a row: a queue with less than kWave rays for each of kSpread waves (one per
+// SIMD) is spread over them in shorter rows. A short launch lasts as long as its
+// longest ray, step by step (1-2 us each), and lanes of a wave wait for each other's
+// node and leaf steps. With twice, four or eight times the waves the steps themselves
+// slow down. 999 rays into 100k triangles 165 -> 140 us, 14,400 into 1M 385 -> 255 us,
+// 153,600 into 1M 507 -> 504 us; 8192 waves 283 and 633 us.
+constexpr uint32_t kSpread = 1024;
+__host__ __device__ constexpr uint32_t wide_row(uint32_t n) {
+    const uint32_t r = n / kSpread + (n % kSpread != 0 ? 1u : 0u);
+    return r < 1u ? 1u : (r > uint32_t(kWave) ? uint32_t(kWave) : r);
+}
 constexpr uint32_t kDealt = 5;
 // A wave steps either its lanes that wait at a node or those that wait at a leaf's
 // primitive, never both paths for a few lanes each: the leaves go when they are at
@@ -778,7 +790,7 @@ __device__ __forceinline__ void trace_wide_persistent_body(const WideTrace &B, c
                                                            uint2 (*s_stack)[kWideBlock]) {
     const uint32_t n = queue_len[0];
     const uint32_t lane = __lane_id();
-    const uint32_t waves = gridDim.x * (kWideBlock / kWave);
+    const uint32_t waves = gridDim.x * kWideWaves;
     WideTree T = tree_of(MULTI ? jw : &B);  // MULTI: the tree of the lane's current ray
     uint32_t visits = 0, boxes = 0, tests = 0;
     WideRay R;
@@ -787,10 +799,11 @@ __device__ __forceinline__ void trace_wide_persistent_body(const WideTrace &B, c
     R.rays = rays;
     // wave-uniform: the slots of the current row not handed out yet, [next, next + left),
     // and the rows dealt to this wave, the current one included
-    uint32_t next = __builtin_amdgcn_readfirstlane(blockIdx.x * kWideBlock + (threadIdx.x & ~uint32_t(kWave - 1)));
-    bool more = next < n;
-    uint32_t left = more ? min(n - next, uint32_t(kWave)) : 0u;
-    const uint64_t row_all = uint64_t(waves) * kWave;  // slots of one row of every wave
+    const uint32_t row = wide_row(n);
+    const uint64_t first = uint64_t(__builtin_amdgcn_readfirstlane(blockIdx.x * kWideWaves + threadIdx.x / kWave)) * row;
+    bool more = first < n;
+    uint32_t next = uint32_t(first), left = more ? min(n - next, row) : 0u;
+    const uint64_t row_all = uint64_t(waves) * row;  // slots of one row of every wave
     uint32_t rows = max(1u, uint32_t(n / row_all * kDealt / 8));
     const uint64_t dealt = rows * row_all;
     while (true) {
@@ -810,17 +823,17 @@ __device__ __forceinline__ void trace_wide_persistent_body(const WideTrace &B, c
             next += taken;
             left -= taken;
             if (left == 0 && --rows != 0) {  // the wave's next dealt row (a whole one: dealt <= n then)
-                next += uint32_t(row_all) - kWave;
-                left = kWave;
+                next += uint32_t(row_all) - row;
+                left = row;
             } else if (left == 0) {  // the next row of the rest
                 rows = 1;
-                uint32_t row = 0;
-                if (lane == 0) row = atomicAdd(&queue_len[kQueueHead], 1u);
-                const uint64_t at = dealt + uint64_t(__builtin_amdgcn_readfirstlane(row)) * kWave;
+                uint32_t k = 0;
+                if (lane == 0) k = atomicAdd(&queue_len[kQueueHead], 1u);
+                const uint64_t at = dealt + uint64_t(__builtin_amdgcn_readfirstlane(k)) * row;
                 more = at < n;
                 if (more) {
                     next = uint32_t(at);
-                    left = min(n - next, uint32_t(kWave));
+                    left = min(n - next, row);
                 }
             }
             continue;
@@ -967,7 +980,8 @@ static uint32_t persistent_grid(Kernel kernel, uint32_t n, uint32_t quarters) {
             }
     }
     if (quarters >= 1 && quarters < 4) blocks = std::max(1u, blocks * quarters / 4);
-    return std::max(1u, std::min(blocks, (n + kWideBlock - 1) / kWideBlock));
+    const uint64_t wave_slots = uint64_t(wide_row(n)) * kWideWaves;
+    return std::max(1u, uint32_t(std::min<uint64_t>(blocks, (n + wave_slots - 1) / wave_slots)));
 }
 
 // The persistent traversal over a compacted queue; the instance with the

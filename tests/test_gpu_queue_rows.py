@@ -1,0 +1,44 @@
+"""Ray queues at the edges of the traversal's rows against the binary traversal: one ray,
+row lengths that change (multiples of the waves the rows are spread over), the first
+queues with full rows, more rays than one row of every wave, inactive rays in between."""
+import numpy as np
+import pytest
+
+import pbrtm
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 1023, 1024, 1025, 2049, 65535, 65537, 400_003, 1_200_001])
+def test_row_edges(ctx, n):
+    print(f"{n} rays", flush=True)
+    bvh = ctx.build(pbrtm.gen_soup(5000, seed=31, mu=-3.0))
+    rng = np.random.default_rng(n)
+    rays = np.zeros((n, 8), np.float32)
+    rays[:, 0:3] = rng.uniform(-0.3, 1.3, (n, 3))
+    rays[:, 4:7] = rng.normal(size=(n, 3))
+    rays[:, 3] = np.where(rng.random(n) < 0.2, 0.0, np.inf)
+    rays[0, 3] = np.inf
+    for any_hit in (False, True):
+        got = bvh.intersect(rays, any_hit=any_hit)
+        want = bvh.intersect(rays, any_hit=any_hit, binary=True)
+        for g, w in zip(got, want):
+            assert np.array_equal(g.view(np.uint32), w.view(np.uint32))
+    bvh.free()
+
+
+@pytest.mark.parametrize("integrator", ["path", "megakernelpath", "ambientocclusion", "surfacenormal"])
+@pytest.mark.parametrize("pool", [1, 255, 257, 5000])
+def test_pool_sizes(ctx, pool, integrator):
+    """Film of a pool that refills many times, in ragged workgroups, against one that never does
+    (the megakernel integrators add samples in sample order, one sample per pixel has no order)."""
+    from pbrtm import scenes
+
+    w, h = (9, 7) if pool == 1 else (53, 37)
+    print(f"{integrator} pool {pool}", flush=True)
+    scene = ctx.scene(scenes.cornell34(w, h))
+    a, aux, st = scene.render(spp=1, max_depth=4, pool_size=pool, integrator=integrator)
+    b, bux, _ = scene.render(spp=1, max_depth=4, integrator=integrator)
+    assert st["paths"] == w * h and np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    assert np.array_equal(aux.view(np.uint32), bux.view(np.uint32))
+    scene.free()
