@@ -835,6 +835,8 @@ int pbrtm_scene_create(pbrtm_ctx *ctx, const pbrtm_scene_desc *desc, pbrtm_scene
     D.inf_dist = H.inf_dist;
     D.shapes = H.shapes.empty() ? nullptr : sc->shapes.as<pbrtm::pt::DShape>();
     D.prim_shape = H.shapes.empty() ? nullptr : sc->prim_shape.as<uint32_t>();
+    D.mixed = 0;
+    for (const auto &m : H.mats) D.mixed |= m.type != H.mats[0].type ? 1u : 0u;
     // The aggregate over the render-space primitives (SceneBuilder::preprocess,
     // scene_builder.cu:829-838): triangles, and analytic primitives through their boxes.
     const int rc = pbrtm_bvh_build(ctx, sc->tri.as<float>(), 3 * desc->num_tris, nullptr, desc->num_tris,

@@ -72,6 +72,7 @@ struct SceneDev {
     float inf_dist;  // 2 x the scene's bounding-sphere radius (UniformInfiniteLight::sample_li)
     const DShape *shapes;        // analytic primitives (spheres, disks, instanced triangles); null if none
     const uint32_t *prim_shape;  // per primitive: index into shapes + 1, 0 = a triangle; null if none
+    uint32_t mixed;              // materials of more than one type
 };
 
 // Integrators render() runs (SceneBuilder::build_integrator, scene_builder.cu:289-313).

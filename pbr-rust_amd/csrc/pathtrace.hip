@@ -457,57 +457,44 @@ __global__ void init_counters_kernel(uint32_t *counters, uint32_t first) {
     counters[k] = (k == kCntNextId || k == b + kCntLive || k == b + kCntRays) ? first : 0u;
 }
 
-// What a slot does after a round of shading.
-constexpr uint32_t kOutLive = 1u, kOutRay = 2u, kOutShadow = 4u;
-
-// Appends the workgroup's slots to the queues of `parity`. Every thread of the workgroup
-// calls this. SEPARATE (the single-vertex integrators): the closest-hit queue is not the
-// live list, and a slot's shadow rays are one instead of two.
-template <bool SEPARATE>
-__device__ __forceinline__ void append_queues(const State &st, uint32_t parity, uint32_t i, uint32_t out) {
-    __shared__ uint32_t s_cnt[3][kBlock / kWave];
-    __shared__ uint32_t s_at[3];
-    const uint32_t wv = threadIdx.x / kWave;
-    const uint64_t live = __ballot((out & kOutLive) != 0u), shadow = __ballot((out & kOutShadow) != 0u);
-    const uint64_t ray = SEPARATE ? __ballot((out & kOutRay) != 0u) : 0ull;
-    if (lane_id() == 0) {
-        s_cnt[0][wv] = uint32_t(__popcll(live));
-        s_cnt[1][wv] = uint32_t(__popcll(shadow));
-        if (SEPARATE) s_cnt[2][wv] = uint32_t(__popcll(ray));
+// The workgroup's slots with shadow rays, gathered as its waves end: the last one to end
+// appends them to the queue of `parity` (two rays per slot, next-event estimation; one
+// for ambient occlusion, SINGLE). The waves end at different times and wait for each
+// other neither here nor on a shared counter, which serves some 6 ns per atomic.
+struct ShadowGather {
+    uint32_t slot[kBlock];
+    uint32_t n, ended;
+};
+// (before a barrier that every thread passes)
+__device__ __forceinline__ void shadow_init(ShadowGather &G) {
+    if (threadIdx.x == 0) G.n = G.ended = 0u;
+}
+template <bool SINGLE>
+__device__ __forceinline__ void append_shadow(const State &st, uint32_t parity, uint32_t i, bool want,
+                                              ShadowGather &G) {
+    constexpr uint32_t kPer = SINGLE ? 1u : 2u;
+    const uint64_t m = __ballot(want);
+    const uint32_t lane = lane_id();
+    uint32_t at = 0;
+    if (lane == 0 && m) at = atomicAdd(&G.n, uint32_t(__popcll(m)));
+    at = __builtin_amdgcn_readfirstlane(at) + uint32_t(__popcll(m & lanemask_lt()));
+    if (want) G.slot[at] = i;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    uint32_t ended = 0;
+    if (lane == 0) ended = atomicAdd(&G.ended, 1u);
+    if (__builtin_amdgcn_readfirstlane(ended) != kBlock / kWave - 1u) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    const uint32_t n = __hip_atomic_load(&G.n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (n == 0) return;
+    uint32_t base = 0;
+    if (lane == 0) base = atomicAdd(st.counters + cnt_block(parity) + kCntShadow, kPer * n);
+    base = __builtin_amdgcn_readfirstlane(base);
+    uint32_t *q = st.shadowq[parity & 1u] + base;
+    for (uint32_t k = lane; k < n; k += kWave) {
+        const uint32_t s = G.slot[k];
+        if (SINGLE) q[k] = 2u * s;
+        else *reinterpret_cast<uint2 *>(q + 2u * k) = make_uint2(2u * s, 2u * s + 1u);
     }
-    __syncthreads();
-    constexpr uint32_t kPer = SEPARATE ? 1u : 2u;  // shadow rays per slot
-    if (threadIdx.x == 0) {
-        uint32_t *c = st.counters + cnt_block(parity);
-        uint32_t n[3] = {0u, 0u, 0u};
-        for (uint32_t k = 0; k < kBlock / kWave; ++k) {
-            n[0] += s_cnt[0][k];
-            n[1] += s_cnt[1][k];
-            if (SEPARATE) n[2] += s_cnt[2][k];
-        }
-        if (n[0]) {
-            const unsigned long long at = atomicAdd(reinterpret_cast<unsigned long long *>(c + kCntLive),
-                                                    (unsigned long long)(n[0]) | ((unsigned long long)(kPer * n[1]) << 32));
-            s_at[0] = uint32_t(at);
-            s_at[1] = uint32_t(at >> 32);
-        }
-        if (SEPARATE) s_at[2] = n[2] ? atomicAdd(c + kCntRays, n[2]) : 0u;
-    }
-    __syncthreads();
-    uint32_t before[3] = {0u, 0u, 0u};
-    for (uint32_t k = 0; k < wv; ++k) {
-        before[0] += s_cnt[0][k];
-        before[1] += s_cnt[1][k];
-        if (SEPARATE) before[2] += s_cnt[2][k];
-    }
-    const uint64_t lt = lanemask_lt();
-    if (out & kOutLive) st.live[parity & 1u][s_at[0] + before[0] + uint32_t(__popcll(live & lt))] = i;
-    if (out & kOutShadow) {
-        const uint32_t at = s_at[1] + kPer * (before[1] + uint32_t(__popcll(shadow & lt)));
-        if (SEPARATE) st.shadowq[parity & 1u][at] = 2u * i;
-        else *reinterpret_cast<uint2 *>(st.shadowq[parity & 1u] + at) = make_uint2(2u * i, 2u * i + 1u);
-    }
-    if (SEPARATE && (out & kOutRay)) st.rayq[parity & 1u][s_at[2] + before[2] + uint32_t(__popcll(ray & lt))] = i;
 }
 
 // One round for slot i: deferred NEE, control_logic, film record, new path,
@@ -528,19 +515,34 @@ __device__ __forceinline__ float dot4(const S4 &a, const S4 &b) {
 // run the megakernel integrators (base/megakernel_integrator.cu:82-147) on the
 // same pool, one round per path vertex.
 template <bool MULTI, bool GRAD, uint32_t MODE = kIntPath>
-__device__ __forceinline__ uint32_t shade_impl(const SceneDev &S, const State &st, const Params &P, uint32_t i,
+__device__ __forceinline__ bool shade_impl(const SceneDev &S, const State &st, const Params &P, uint32_t i,
                                            uint32_t pid, uint32_t lid, uint32_t spd, uint32_t max_depth,
                                            uint32_t round, float4 *erec, float4 *grec) {
     const bool live = pid != kIdle;
-    uint32_t fl = live ? st.flags[i] : 0u;
-    S4 L = live ? f4s(st.L[i]) : s4(0.f), beta = live ? f4s(st.beta[i]) : s4(0.f);
-    S4 gadj = s4(0.f);
-    if (GRAD && live) gadj = f4s(P.gd.g[i]);
+    // the slot's state, all loads at once: a wave here waits for memory most of the time
+    uint32_t fl = 0u, prim_hit = kNoHit, dim = 0u;
+    uint64_t rng = 0u;
+    uint2 blocked = make_uint2(kNoHit, kNoHit);
+    S4 L = s4(0.f), beta = s4(0.f), lam = s4(0.f), lpdf = s4(0.f), gadj = s4(0.f);
+    float4 scal = make_float4(0.f, 0.f, 0.f, 0.f), nee_L = scal;
+    if (live) {
+        fl = st.flags[i];
+        prim_hit = st.prim[i];
+        blocked = *reinterpret_cast<const uint2 *>(st.sprim + 2 * size_t(i));
+        L = f4s(st.L[i]);
+        beta = f4s(st.beta[i]);
+        nee_L = st.nee_L[i];
+        lam = f4s(st.lam[i]);
+        lpdf = f4s(st.lam_pdf[i]);
+        scal = st.scal[i];
+        rng = st.rng[i];
+        dim = st.dim[i];
+        if (GRAD) gadj = f4s(P.gd.g[i]);
+    }
     // 1. the previous round's light sample, if both shadow rays missed
     if (live && (fl & kFlagNee)) {
-        if (st.sprim[2 * size_t(i)] == kNoHit &&
-            (MODE == kIntAmbientOcclusion || st.sprim[2 * size_t(i) + 1] == kNoHit)) {
-            L = s4add(L, f4s(st.nee_L[i]));
+        if (blocked.x == kNoHit && (MODE == kIntAmbientOcclusion || blocked.y == kNoHit)) {
+            L = s4add(L, f4s(nee_L));
             if (GRAD) {
                 // C = beta f cos Le w(pmf p) / (pmf p) with w = g^2 / (g^2 + b^2), g = pmf p:
                 // dC/dpmf = C (1 - 2w) / pmf (the MIS weight's pmf and the light choice's
@@ -554,21 +556,16 @@ __device__ __forceinline__ uint32_t shade_impl(const SceneDev &S, const State &s
     const uint32_t depth = fl & kDepthMask;
     // a single-vertex integrator's second visit has no ray: the path ends
     const bool traced = live && (MODE <= kIntMegakernelPath || depth == 0);
-    const uint32_t prim = traced ? st.prim[i] : kNoHit;
+    const uint32_t prim = traced ? prim_hit : kNoHit;
     bool terminate = live && (prim == kNoHit || depth > max_depth || !s4pos(beta));
     Sampler smp{};
-    S4 lam = s4(0.f), lpdf = s4(0.f);
-    float4 scal = make_float4(0.f, 0.f, 0.f, 0.f);
     if (live) {
         smp.pixel = lid % (S.width * S.height);
         smp.sample = lid / (S.width * S.height);
         smp.spd = spd;
-        smp.rng.state = st.rng[i];
+        smp.rng.state = rng;
         smp.rng.inc = sampler_inc(smp.pixel);
-        smp.dim = st.dim[i];
-        lam = f4s(st.lam[i]);
-        lpdf = f4s(st.lam_pdf[i]);
-        scal = st.scal[i];
+        smp.dim = dim;
     }
     // Russian roulette (wavefront_path.cu:121-138), only past 8 bounces. The
     // wavefront draws its sample always; the megakernel path integrator only
@@ -627,24 +624,41 @@ __device__ __forceinline__ uint32_t shade_impl(const SceneDev &S, const State &s
         terminate = true;
     }
     // 2. finished paths: film record, then a new path in this slot. The new path
-    // ids are reserved once per workgroup (every thread of it gets here): the ids
-    // handed out in a round are one contiguous run whatever the order of the
-    // reservations, and one shared counter serves them one at a time.
-    const uint64_t lanes = __ballot(terminate);
-    __shared__ uint32_t s_new[kBlock / kWave];
-    __shared__ uint32_t s_new_base;
-    const uint32_t wv = threadIdx.x / kWave, nwaves = blockDim.x / kWave;
-    if (lane_id() == 0) s_new[wv] = uint32_t(__popcll(lanes));
+    // ids, and places in the next round's live list, are reserved once per workgroup
+    // (every thread of it gets here): the ids handed out in a round are one contiguous
+    // run whatever the order of the reservations, and one shared counter serves them
+    // one at a time.
+    const uint64_t lanes = __ballot(terminate), keeps = __ballot(live && !terminate);
+    __shared__ uint32_t s_new[kBlock / kWave], s_keep[kBlock / kWave];
+    __shared__ uint32_t s_new_base, s_live_base, s_ray_base;
+    const uint32_t wv = threadIdx.x / kWave;
+    if (lane_id() == 0) {
+        s_new[wv] = uint32_t(__popcll(lanes));
+        s_keep[wv] = uint32_t(__popcll(keeps));
+    }
     __syncthreads();
-    uint32_t before = 0, total_new = 0;
-    for (uint32_t k = 0; k < nwaves; ++k) {
-        const uint32_t t = s_new[k];
+    uint32_t before = 0, total_new = 0, before_keep = 0, total_keep = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kBlock / kWave; ++k) {
+        const uint32_t t = s_new[k], u = s_keep[k];
         before += k < wv ? t : 0u;
         total_new += t;
+        before_keep += k < wv ? u : 0u;
+        total_keep += u;
     }
-    if (threadIdx.x == 0) s_new_base = total_new ? atomicAdd(&st.counters[kCntNextId], total_new) : 0u;
+    if (threadIdx.x == 0) {
+        const uint32_t ids = total_new ? atomicAdd(&st.counters[kCntNextId], total_new) : 0u;
+        const uint32_t started = uint64_t(ids) >= P.total ? 0u : uint32_t(min(uint64_t(total_new), P.total - ids));
+        uint32_t *c = st.counters + cnt_block(round + 1);
+        s_new_base = ids;
+        s_live_base = total_keep + started ? atomicAdd(c + kCntLive, total_keep + started) : 0u;
+        if (MODE > kIntMegakernelPath && started) s_ray_base = atomicAdd(c + kCntRays, started);
+    }
     __syncthreads();
     const uint32_t base = s_new_base + before;
+    const uint32_t new_rank = before + uint32_t(__popcll(lanes & lanemask_lt()));  // of the workgroup's new paths
+    uint32_t *next_live = st.live[(round + 1) & 1u];
+    if (live && !terminate) next_live[s_live_base + before_keep + uint32_t(__popcll(keeps & lanemask_lt()))] = i;
     if (terminate) {
         // Infinite lights (wavefront_path.cu:140-160): every path that ends with a
         // positive beta, escaped or not; the megakernel path integrator only on an
@@ -667,6 +681,8 @@ __device__ __forceinline__ uint32_t shade_impl(const SceneDev &S, const State &s
         }
         const uint64_t nid = uint64_t(base) + __popcll(lanes & lanemask_lt());
         if (nid < P.total) {
+            next_live[s_live_base + total_keep + new_rank] = i;
+            if (MODE > kIntMegakernelPath) st.rayq[(round + 1) & 1u][s_ray_base + new_rank] = i;
             if (MULTI) {
                 const uint32_t j = find_job(P, nid);
                 const JobDev &J = P.jobs[j];
@@ -677,9 +693,9 @@ __device__ __forceinline__ uint32_t shade_impl(const SceneDev &S, const State &s
                 start_path<GRAD>(S, st, spd, i, nid, nid, P.gd.lfin, P.gd.pfin, P.gd.adj, P.gd.g, P.gd.ltot);
             }
         }
-        return nid < P.total ? kOutLive | kOutRay : 0u;
+        return false;
     }
-    if (!live) return 0u;
+    if (!live) return false;
     const float4 r1 = st.rays[2 * size_t(i) + 1];
     const f3 rd = {r1.x, r1.y, r1.z};
     const uint2 info = S.tri_info[prim];
@@ -733,7 +749,7 @@ __device__ __forceinline__ uint32_t shade_impl(const SceneDev &S, const State &s
         st.L[i] = s4f(L);
         st.rng[i] = smp.rng.state;
         st.dim[i] = smp.dim;
-        return (fl & kFlagNee) ? kOutLive | kOutShadow : kOutLive;
+        return (fl & kFlagNee) != 0u;
     }
     const f3 wo_n = norm3(neg3(rd));
     const uint32_t light = info.y & 0x7FFFFFFFu;
@@ -882,7 +898,7 @@ __device__ __forceinline__ uint32_t shade_impl(const SceneDev &S, const State &s
     st.scal[i] = scal;
     st.rng[i] = smp.rng.state;
     st.dim[i] = smp.dim;
-    return nee ? kOutLive | kOutRay | kOutShadow : kOutLive | kOutRay;
+    return nee;
 }
 
 // The live list's entry of this thread in a round of `parity`, kIdle past its end.
@@ -894,19 +910,67 @@ __device__ __forceinline__ uint32_t live_slot(const State &st, uint32_t parity, 
     return k < n ? st.live[parity & 1u][k] : kIdle;
 }
 
+// A workgroup's live slots ordered by what their hit has them do: end the path and start
+// one (a miss, the depth limit), or sample one of the materials; kIdle (past the list's
+// end) last. In list order a wave takes every one of these paths in turn with a quarter
+// of its lanes (VALU lane use 25 % at 81 % VALU busy); ordered over the whole pool the
+// slots' state, an array per field, is fetched four times over (L2 misses x 4.7, and no
+// gain), so a workgroup orders its own slots, which stay neighbours: instructions x 0.6,
+// lane use 44 %. Single renders of one material type (SceneDev::mixed 0) are not
+// ordered: ended and going paths alone are not worth it there (shading of a diffuse
+// room 382 -> 405 us a round), while in a batch, where a new path reads its job's tables
+// lane by lane, they are (110 -> 57 us a round of 16 small jobs). The order is all that
+// the class decides: each slot finds out by itself what to do.
+template <bool MULTI>
+__device__ __forceinline__ uint32_t order_slots(const SceneDev &S, const State &st, const Params &P, uint32_t i) {
+    constexpr uint32_t kClasses = 5, kWaves = kBlock / kWave;
+    __shared__ uint32_t s_cnt[kClasses][kWaves];
+    __shared__ uint32_t s_slot[kBlock];
+    uint32_t cls = kClasses - 1u;
+    if (i != kIdle) {
+        const uint32_t prim = st.prim[i], depth = st.flags[i] & kDepthMask;
+        const uint32_t j = MULTI ? st.job[i] : 0u;
+        const SceneDev &D = MULTI ? P.jobs[j].S : S;
+        const uint32_t max_depth = MULTI ? P.jobs[j].max_depth : P.max_depth;
+        cls = prim == kNoHit || depth > max_depth ? 0u : 1u + min(D.mats[D.tri_info[prim].x].type, 2u);
+    }
+    const uint32_t wv = threadIdx.x / kWave;
+    uint32_t at = 0;
+#pragma unroll
+    for (uint32_t c = 0; c < kClasses; ++c) {
+        const uint64_t m = __ballot(cls == c);
+        if (cls == c) at = uint32_t(__popcll(m & lanemask_lt()));
+        if (lane_id() == 0) s_cnt[c][wv] = uint32_t(__popcll(m));
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t c = 0; c < kClasses; ++c)
+#pragma unroll
+        for (uint32_t k = 0; k < kWaves; ++k) at += (c < cls || (c == cls && k < wv)) ? s_cnt[c][k] : 0u;
+    s_slot[at] = i;
+    __syncthreads();
+    return s_slot[threadIdx.x];
+}
+
 // The path-integrator shading instances need about 172 VGPRs unbounded (2 waves
-// per SIMD); held to 168 (3 waves) they spill 8 bytes per lane, which is faster.
+// per SIMD); held to 168 (3 waves) they spill 24 bytes per lane, which is faster; held
+// to 128 (4 waves) they lose what the waves gain (1080p x 16 path tracing 107.0 against
+// 109.1 ms). With ordered slots they wait for memory 70 % of the time.
 #define PBRTM_SHADE_WAVES __attribute__((amdgpu_waves_per_eu(3)))
 
 template <uint32_t MODE>
 __global__ __launch_bounds__(kBlock) PBRTM_SHADE_WAVES void shade_kernel(SceneDev S, State st, Params P) {
     bool none;
-    const uint32_t i = live_slot(st, P.round, &none);
+    uint32_t i = live_slot(st, P.round, &none);
     if (none) return;
+    __shared__ ShadowGather s_shadow;
+    shadow_init(s_shadow);
+    if (MODE <= kIntMegakernelPath && S.mixed) i = order_slots<false>(S, st, P, i);
+    else __syncthreads();
     const uint32_t pid = i != kIdle ? st.path_id[i] : kIdle;
-    const uint32_t out = shade_impl<false, false, MODE>(S, st, P, i, pid, pid, P.spd, P.max_depth, P.round, nullptr,
+    const bool shadow = shade_impl<false, false, MODE>(S, st, P, i, pid, pid, P.spd, P.max_depth, P.round, nullptr,
                                                         nullptr);
-    append_queues<(MODE > kIntMegakernelPath)>(st, P.round + 1, i, out);
+    append_shadow<(MODE > kIntMegakernelPath)>(st, P.round + 1, i, shadow, s_shadow);
 }
 
 // The gradient replay of one round (same paths as the forward render).
@@ -914,16 +978,19 @@ constexpr uint32_t kMaxGroups = 255;
 __global__ __launch_bounds__(kBlock) void shade_grad_kernel(SceneDev S, State st, Params P) {
     __shared__ double s_acc[kMaxGroups + 1];
     bool none;
-    const uint32_t i = live_slot(st, P.round, &none);
+    uint32_t i = live_slot(st, P.round, &none);
     if (none) return;
+    __shared__ ShadowGather s_shadow;
+    shadow_init(s_shadow);
+    if (S.mixed) i = order_slots<false>(S, st, P, i);
     for (uint32_t k = threadIdx.x; k <= P.gd.ngroups; k += kBlock) s_acc[k] = 0.0;
     __syncthreads();
     const uint32_t pid = i != kIdle ? st.path_id[i] : kIdle;
     float4 grec = make_float4(0.f, 0.f, 0.f, __uint_as_float(kIdle));
     float4 erec[2] = {make_float4(0.f, 0.f, __uint_as_float(kIdle), 0.f),
                       make_float4(0.f, 0.f, __uint_as_float(kIdle), 0.f)};
-    const uint32_t out = shade_impl<false, true>(S, st, P, i, pid, pid, P.spd, P.max_depth, P.round, erec, &grec);
-    append_queues<false>(st, P.round + 1, i, out);
+    const bool shadow = shade_impl<false, true>(S, st, P, i, pid, pid, P.spd, P.max_depth, P.round, erec, &grec);
+    append_shadow<false>(st, P.round + 1, i, shadow, s_shadow);
     // Emitter sums: the pmf part over the whole wave, the scale part per emitter
     // (lanes of one emitter summed first), into shared memory.
     {
@@ -992,15 +1059,18 @@ __global__ __launch_bounds__(kBlock) void shade_grad_kernel(SceneDev S, State st
 // (P.round gives its parity).
 __global__ __launch_bounds__(kBlock) PBRTM_SHADE_WAVES void shade_multi_kernel(State st, Params P) {
     bool none;
-    const uint32_t i = live_slot(st, P.round, &none);
+    uint32_t i = live_slot(st, P.round, &none);
     if (none) return;
+    __shared__ ShadowGather s_shadow;
+    shadow_init(s_shadow);
+    i = order_slots<true>(P.jobs[0].S, st, P, i);
     const uint32_t pid = i != kIdle ? st.path_id[i] : kIdle;
     const uint32_t j = pid != kIdle ? st.job[i] : 0u;
     const JobDev &J = P.jobs[j];
     const uint32_t lid = pid != kIdle ? uint32_t(pid - J.base) : kIdle;
-    const uint32_t out = shade_impl<true, false>(J.S, st, P, i, pid, lid, J.spd, J.max_depth, st.counters[kCntRound],
+    const bool shadow = shade_impl<true, false>(J.S, st, P, i, pid, lid, J.spd, J.max_depth, st.counters[kCntRound],
                                                  nullptr, nullptr);
-    append_queues<false>(st, P.round + 1, i, out);
+    append_shadow<false>(st, P.round + 1, i, shadow, s_shadow);
 }
 
 // Sums the kGradShards copies of the coefficient-derivative table into the first.
