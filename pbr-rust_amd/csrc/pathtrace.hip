@@ -1314,13 +1314,82 @@ __global__ __launch_bounds__(kBlock) void film_lane_kernel(SceneDev S, const flo
     }
 }
 
-// The film of one render: a lane per pixel up to kLaneFilm samples, else a wave.
+// film_kernel for kLaneFilm < spp <= kSortFilm: one lane per pixel, so that neighbouring
+// pixels' records are read together and every lane adds. Each lane keeps its pixel's
+// samples in (round, sample) order in a column of LDS, by insertion: a pixel's samples
+// mostly finish in order. 1080p x 16 samples 1.53 -> 0.15 ms (663 MB of records,
+// 4.6 TB/s), x 64 samples 3.9 -> 0.82 ms.
+constexpr uint32_t kSortFilm = 64;
+constexpr uint32_t kSortRounds = 1u << 22;  // rounds fit 22 bits above the 10 of a sample
+
+__global__ __launch_bounds__(kWave) void film_sort_kernel(SceneDev S, const float4 *__restrict__ rec,
+                                                          const uint32_t *__restrict__ rec_round, uint32_t spp,
+                                                          float *film_rgb, float *film_aux) {
+    extern __shared__ uint32_t s_col[];  // [spp][kWave]
+    const uint32_t wh = S.width * S.height, lane = threadIdx.x;
+    const uint32_t px = blockIdx.x * kWave + lane;
+    if (px >= wh) return;
+    uint32_t last = 0;
+    for (uint32_t s0 = 0; s0 < spp; s0 += 8) {
+        uint32_t key[8];
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k) key[k] = s0 + k < spp ? rec_round[size_t(s0 + k) * wh + px] : 0u;
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k) {
+            const uint32_t s = s0 + k;
+            if (s >= spp) break;
+            const uint32_t v = (key[k] << 10) | s;
+            uint32_t at = s;
+            if (s > 0 && v < last) {
+                while (at > 0) {
+                    const uint32_t u = s_col[(at - 1) * kWave + lane];
+                    if (u < v) break;
+                    s_col[at * kWave + lane] = u;
+                    --at;
+                }
+            } else {
+                last = v;
+            }
+            s_col[at * kWave + lane] = v;
+        }
+    }
+    float sum[3] = {0.f, 0.f, 0.f}, wsum = 0.f;
+    for (uint32_t p0 = 0; p0 < spp; p0 += 8) {
+        float4 r[8];
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k)
+            r[k] = p0 + k < spp ? rec[size_t(s_col[(p0 + k) * kWave + lane] & 1023u) * wh + px]
+                                : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k) {
+            if (r[k].w == 0) continue;
+            sum[0] += r[k].w * r[k].x;
+            sum[1] += r[k].w * r[k].y;
+            sum[2] += r[k].w * r[k].z;
+            wsum += r[k].w;
+        }
+    }
+    float rgb[3] = {sum[0], sum[1], sum[2]};
+    if (wsum != 0)
+        for (int c = 0; c < 3; ++c) rgb[c] /= wsum;
+    for (int c = 0; c < 3; ++c) film_rgb[3 * size_t(px) + c] = ip3(S.out_from_sensor + 3 * c, rgb);
+    if (film_aux) {
+        for (int c = 0; c < 3; ++c) film_aux[4 * size_t(px) + c] = sum[c];
+        film_aux[4 * size_t(px) + 3] = wsum;
+    }
+}
+
+// The film of one render of `rounds` rounds: a lane per pixel up to kSortFilm samples,
+// else a wave.
 static void launch_film(const SceneDev &S, const float4 *rec, const uint32_t *rec_round, uint32_t spp,
-                        float *film_rgb, float *film_aux, hipStream_t stream) {
+                        uint64_t rounds, float *film_rgb, float *film_aux, hipStream_t stream) {
     const uint32_t wh = S.width * S.height;
     if (spp <= kLaneFilm)
         film_lane_kernel<<<(wh + kBlock - 1) / kBlock, kBlock, 0, stream>>>(S, rec, rec_round, spp, film_rgb,
                                                                             film_aux);
+    else if (spp <= kSortFilm && rounds <= kSortRounds)
+        film_sort_kernel<<<(wh + kWave - 1) / kWave, kWave, spp * kWave * sizeof(uint32_t), stream>>>(
+            S, rec, rec_round, spp, film_rgb, film_aux);
     else
         film_kernel<<<(wh + kFilmWaves - 1) / kFilmWaves, kFilmWaves * kWave, 0, stream>>>(S, rec, rec_round, spp,
                                                                                          film_rgb, film_aux);
@@ -1372,6 +1441,10 @@ hipError_t film_adjoint(const SceneDev &S, const float *film_rgb, const float *f
 }
 
 namespace {
+
+// Rounds of a job's one-by-one render are fewer than this: every slot's paths end within
+// max_depth + 2 rounds each, and each of the vpool slots starts its share of them.
+uint64_t round_bound(const JobDev &J) { return (J.total / J.vpool + 2) * (uint64_t(J.max_depth) + 3); }
 
 hipError_t reserve_pool(PathPool &pp, uint32_t pool, uint64_t total, bool batch, bool separate_rays) {
     hipError_t e;
@@ -1582,7 +1655,7 @@ hipError_t render(const SceneDev &S, const WideTrace &W0, uint32_t spp, uint32_t
         PT_CK(hipGetLastError());
     }
     if (film_rgb) {
-        launch_film(S, st.rec, st.rec_round, spp, film_rgb, film_aux, stream);
+        launch_film(S, st.rec, st.rec_round, spp, r, film_rgb, film_aux, stream);
         PT_CK(hipGetLastError());
     }
     PT_CK(hipEventRecord(ev[2], stream));
@@ -1734,8 +1807,8 @@ hipError_t render_shared(const std::vector<BatchJob> &jobs, uint32_t pool, uint3
     PT_CK(hipGetLastError());
     PT_CK(hipEventRecord(ev[2], stream));
     for (uint32_t j = 0; j < nj; ++j) {
-        launch_film(jd[j].S, st.rec + jd[j].base, st.rec_round + jd[j].base, jd[j].spp, jobs[j].film_rgb,
-                    jobs[j].film_aux, stream);
+        launch_film(jd[j].S, st.rec + jd[j].base, st.rec_round + jd[j].base, jd[j].spp, round_bound(jd[j]),
+                    jobs[j].film_rgb, jobs[j].film_aux, stream);
         PT_CK(hipGetLastError());
     }
     PT_CK(hipEventRecord(ev[3], stream));

@@ -42,3 +42,21 @@ def test_pool_sizes(ctx, pool, integrator):
     assert st["paths"] == w * h and np.array_equal(a.view(np.uint32), b.view(np.uint32))
     assert np.array_equal(aux.view(np.uint32), bux.view(np.uint32))
     scene.free()
+
+
+@pytest.mark.parametrize("spp,pool", [(9, 0), (9, 700), (16, 1), (49, 300), (64, 0), (64, 97), (81, 300)])
+def test_film_order(ctx, spp, pool):
+    """Film sums in (round, sample) order on both sides of the per-lane film's sample limit, with
+    pools that finish a pixel's samples in and out of order, against the oracle."""
+    import oracle as O
+    from pbrtm import scenes
+
+    w, h = (5, 3) if pool == 1 else (13, 7)
+    print(f"{spp} spp, pool {pool}", flush=True)
+    sc = scenes.cornell34(w, h, spp=spp, max_depth=6)
+    scene = ctx.scene(sc)
+    rgb, aux, _ = scene.render(spp=spp, max_depth=6, pool_size=pool)
+    orgb, oaux, _ = O.render(sc, threads=8, pool_size=pool) if pool else O.render(sc, threads=8)
+    assert np.array_equal(rgb.view(np.uint32), orgb.view(np.uint32))
+    assert np.array_equal(aux.view(np.uint32), oaux.view(np.uint32))
+    scene.free()
