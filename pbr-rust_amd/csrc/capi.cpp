@@ -60,6 +60,8 @@ struct pbrtm_ctx {
     std::string error;
     std::vector<BatchTune> batch_tune;
     SpareBvh spare;
+    DevBuf sig_cols;        // the RGB-to-spectrum table for gradients: its columns, then the z nodes
+    size_t sig_count = 0;   // columns it held when it was uploaded
 };
 
 struct pbrtm_bvh {
@@ -264,6 +266,7 @@ void pbrtm_destroy(pbrtm_ctx *ctx) {
     ctx->spill.release();
     ctx->collapse.release();
     ctx->queue.release();
+    ctx->sig_cols.release();
     auto &p = ctx->batch_pool;
     for (DevBuf *b : {&p.path_id, &p.flags, &p.rng, &p.dim, &p.lam, &p.lam_pdf, &p.L, &p.beta, &p.nee_L, &p.scal,
                       &p.prev, &p.rays, &p.prim, &p.thit, &p.bary, &p.srays, &p.sprim, &p.rec, &p.rec_round,
@@ -732,6 +735,7 @@ struct pbrtm_scene {
     pbrtm::pt::PathPool pool;
     pbrtm::DevBuf film_rgb, film_aux;
     pbrtm::DevBuf g_lfin, g_pfin, g_target, g_adj, g_coef, g_acc, g_slot;  // gradient replay
+    pbrtm::DevBuf g_rgb, g_albedo;  // the materials' albedo RGB (uploaded once) and their derivatives
 };
 
 extern "C" {
@@ -743,7 +747,7 @@ void pbrtm_scene_free(pbrtm_scene *sc) {
     for (pbrtm::DevBuf *b : {&sc->tri, &sc->tri_info, &sc->mats, &sc->lights, &sc->pmf, &sc->cdf, &sc->spec_lam,
                              &sc->spec_val, &sc->filt, &sc->shapes, &sc->prim_shape, &sc->film_rgb, &sc->film_aux,
                              &sc->g_lfin, &sc->g_pfin,
-                             &sc->g_target, &sc->g_adj, &sc->g_coef, &sc->g_acc, &sc->g_slot})
+                             &sc->g_target, &sc->g_adj, &sc->g_coef, &sc->g_acc, &sc->g_slot, &sc->g_rgb, &sc->g_albedo})
         b->release();
     auto &p = sc->pool;
     for (pbrtm::DevBuf *b : {&p.path_id, &p.flags, &p.rng, &p.dim, &p.lam, &p.lam_pdf, &p.L, &p.beta, &p.nee_L,
@@ -1048,22 +1052,50 @@ int pbrtm_render_grad(pbrtm_ctx *ctx, pbrtm_scene *sc, const pbrtm_render_params
     CK(ctx, pbrtm::pt::render(sc->dev, W, spp, params->max_depth, pool, sc->pool, nullptr, nullptr, err, &rep, st,
                               nullptr, nullptr, &gd), "replay");
     const auto t3 = std::chrono::steady_clock::now();
-    std::vector<float> coef(size_t(nm) * 3);
     std::vector<double> hacc(ng + 2);
     uint32_t derr = 0;
+    if (d_albedo && nm) {  // J^T through the RGB-to-spectrum table (non-diffuse materials: zero)
+        if (!sc->g_rgb.ptr) {
+            CK(ctx, sc->g_rgb.reserve(size_t(nm) * 12), "alloc");
+            CK(ctx, hipMemcpyAsync(sc->g_rgb.ptr, H.mat_rgb.data(), size_t(nm) * 12, hipMemcpyHostToDevice, st), "upload");
+        }
+        CK(ctx, sc->g_albedo.reserve(size_t(nm) * 12), "alloc");
+        for (int pass = 0; pass < 2; ++pass) {
+            uint32_t missing = 0;
+            try {
+                const size_t have = pbrtm::pt::sigmoid_columns();
+                if (!ctx->sig_cols.ptr || ctx->sig_count != have) {
+                    std::vector<float> cols;
+                    std::vector<double> z;
+                    pbrtm::pt::sigmoid_snapshot(cols, z);
+                    CK(ctx, ctx->sig_cols.reserve(cols.size() * 4 + z.size() * 8), "alloc");
+                    CK(ctx, hipMemcpyAsync(ctx->sig_cols.ptr, cols.data(), cols.size() * 4, hipMemcpyHostToDevice, st), "upload");
+                    CK(ctx, hipMemcpyAsync(ctx->sig_cols.as<uint8_t>() + cols.size() * 4, z.data(), z.size() * 8,
+                                           hipMemcpyHostToDevice, st), "upload");
+                    CK(ctx, hipStreamSynchronize(st), "upload");  // the vectors end here
+                    ctx->sig_count = have;
+                }
+            } catch (const std::bad_alloc &) {
+                return fail(ctx, PBRTM_ERR_NOMEM, "RGB-to-spectrum table");
+            }
+            constexpr size_t kCols = size_t(3) * pbrtm::pt::kSigmoidRes * pbrtm::pt::kSigmoidRes * pbrtm::pt::kSigmoidRes * 3;
+            CK(ctx, hipMemsetAsync(err + 1, 0, 4, st), "memset");
+            CK(ctx, pbrtm::pt::albedo_gradient(sc->g_rgb.as<float>(), sc->dev.mats, gd.d_coef, ctx->sig_cols.as<float>(),
+                                               reinterpret_cast<const double *>(ctx->sig_cols.as<float>() + kCols), nm,
+                                               sc->g_albedo.as<float>(), err + 1, st), "albedo gradient");
+            CK(ctx, hipMemcpyAsync(&missing, err + 1, 4, hipMemcpyDeviceToHost, st), "download");
+            CK(ctx, hipMemcpyAsync(d_albedo, sc->g_albedo.ptr, size_t(nm) * 12, hipMemcpyDeviceToHost, st), "download");
+            CK(ctx, hipStreamSynchronize(st), "sync");
+            if (!missing) break;
+            pbrtm::pt::sigmoid_compute(H.mat_rgb.data(), nm);  // columns that no lookup needed (grey albedos)
+        }
+    }
     CK(ctx, hipMemcpyAsync(&derr, err, 4, hipMemcpyDeviceToHost, st), "download");
-    if (nm) CK(ctx, hipMemcpyAsync(coef.data(), gd.d_coef, coef.size() * 4, hipMemcpyDeviceToHost, st), "download");
     CK(ctx, hipMemcpyAsync(hacc.data(), acc, hacc.size() * 8, hipMemcpyDeviceToHost, st), "download");
     if (film_rgb) CK(ctx, hipMemcpyAsync(film_rgb, film, wh * 12, hipMemcpyDeviceToHost, st), "download");
     CK(ctx, hipStreamSynchronize(st), "sync");
     if (derr) return fail(ctx, PBRTM_ERR_DEVICE, device_error_text(derr));
     *loss = hacc[ng + 1];
-    if (d_albedo) {  // J^T through the RGB-to-spectrum table (non-diffuse materials accumulate nothing)
-        if (nm) pbrtm::pt::rgb_to_sigmoid_jacobian_transpose(H.mat_rgb.data(), coef.data(), nm, d_albedo);
-        for (uint32_t m = 0; m < nm; ++m)
-            if (H.mats[m].type != pbrtm::pt::kDiffuse) d_albedo[3 * size_t(m)] = d_albedo[3 * size_t(m) + 1] =
-                d_albedo[3 * size_t(m) + 2] = 0.f;
-    }
     if (d_scale) {  // dLoss/ds_m = (a_m - k P_m) / s_m, P_m = the emitter's total pmf
         std::vector<double> P(ng, 0.0);
         for (size_t t = 0; t < H.lights.size(); ++t) P[H.lights[t].group] += double(H.light_pmf[t]);

@@ -133,10 +133,18 @@ std::string build_scene_host(const void *desc, SceneHost &out);
 
 // RGB-to-spectrum sigmoid coefficients of an albedo RGB, and the sRGB matrices (for tests).
 void rgb_to_sigmoid(const float rgb[3], float out[3]);
-// d(c0, c1, c2) / d(r, g, b) of rgb_to_sigmoid, row-major [q][k].
-void rgb_to_sigmoid_jacobian(const float rgb[3], double J[9]);
-// out[m] = J(rgb[m])^T coef[m] for n RGBs (multi-threaded).
-void rgb_to_sigmoid_jacobian_transpose(const float *rgb, const float *coef, size_t n, float *out);
+// The RGB-to-spectrum table for albedo_gradient: how many columns are computed, all of
+// them as floats ([3][64][64][64][3], NaN where there is none yet) with the 64 z nodes, and
+// the columns that n RGBs need, computed now.
+constexpr uint32_t kSigmoidRes = 64;
+size_t sigmoid_columns();
+void sigmoid_snapshot(std::vector<float> &cols, std::vector<double> &z);
+void sigmoid_compute(const float *rgb, size_t n);
+// out[m] = J(rgb[m])^T coef[m] for n materials, J = d(c0, c1, c2) / d(r, g, b) of
+// rgb_to_sigmoid, zero for materials that are not diffuse; *missing is set if a column
+// is not in cols. All device pointers.
+hipError_t albedo_gradient(const float *rgb, const DMat *mats, const float *coef, const float *cols, const double *z,
+                           uint32_t n, float *out, uint32_t *missing, hipStream_t stream);
 void srgb_matrices(float xyz_from_rgb[9], float rgb_from_xyz[9], float white_xy[2]);
 // SquareMatrix<4>::inverse (euclidean_space/squared_matrix.cu), row-major; false if singular.
 bool mat4_inverse_ref(const float in[16], float out[16]);

@@ -272,68 +272,20 @@ class SpectrumTable {
         return out;
     }
 
-    // J[q][k] = d c_q / d rgb_k of lookup(): the trilinear interpolation's
-    // derivative times that of the cell coordinates x = rgb[(m+1)%3] (res-1) / z,
-    // y = rgb[(m+2)%3] (res-1) / z, z = rgb[m] (grey inputs take this general branch).
-    void jacobian(const float rgb[3], double J[3][3]) { jacobian_impl(rgb, J, true); }
-
-    // out[m][k] = sum_q J_m[q][k] coef[m][q] for n RGBs, on all host threads (the
-    // columns are computed first, so the threads only read the cache).
-    void jacobian_transpose(const float *rgb, const float *coef, size_t n, float *out) {
-        prefetch(rgb, n, true);
-        const unsigned nt = std::max(1u, std::min<unsigned>(std::thread::hardware_concurrency(), 64u));
-        std::vector<std::thread> ts;
-        for (unsigned t = 0; t < nt; ++t)
-            ts.emplace_back([&, t] {
-                for (size_t m = t; m < n; m += nt) {
-                    double J[3][3];
-                    jacobian_impl(rgb + 3 * m, J, false);
-                    for (int k = 0; k < 3; ++k) {
-                        double v = 0;
-                        for (int q = 0; q < 3; ++q) v += J[q][k] * double(coef[3 * m + q]);
-                        out[3 * m + k] = float(v);
-                    }
-                }
-            });
-        for (auto &th : ts) th.join();
+    // The columns computed so far, and all of them as the floats that lookups and
+    // Jacobians read ([3][kRes][kRes][kRes][3], NaN where there is no column yet).
+    size_t count() {
+        std::lock_guard<std::mutex> g(mu_);
+        return cols_.size();
     }
-
-  private:
-    void jacobian_impl(const float rgb[3], double J[3][3], bool locked) {
-        const int mc = (rgb[0] > rgb[1]) ? ((rgb[0] > rgb[2]) ? 0 : 2) : ((rgb[1] > rgb[2]) ? 1 : 2);
-        const double z = rgb[mc];
-        if (!(z > 0) || rgb[0] < 0 || rgb[1] < 0 || rgb[2] < 0) {  // black: no general-branch cell
-            for (int q = 0; q < 9; ++q) J[q / 3][q % 3] = 0;
-            return;
-        }
-        const double x = double(rgb[(mc + 1) % 3] * (kRes - 1)) / z;
-        const double y = double(rgb[(mc + 2) % 3] * (kRes - 1)) / z;
-        const int xi = std::min((int)x, kRes - 2), yi = std::min((int)y, kRes - 2);
-        int zi = 0;
-        while (zi < kRes - 2 && z_[zi + 1] < z) ++zi;
-        const double dx = x - xi, dy = y - yi, h = z_[zi + 1] - z_[zi], dz = (z - z_[zi]) / h;
-        auto get = [&](int l, int j, int i) -> const Column & {
-            return locked ? column(l, j, i) : cols_.find((l * kRes + j) * kRes + i)->second;
-        };
-        const Column &a = get(mc, yi, xi), &b = get(mc, yi, xi + 1);
-        const Column &c = get(mc, yi + 1, xi), &d = get(mc, yi + 1, xi + 1);
-        auto mix = [](double t, double u, double v) { return u + t * (v - u); };
-        for (int q = 0; q < 3; ++q) {
-            auto f = [&](const Column &col, int dk) { return double(float(col[zi + dk][q])); };
-            double gx[2], gy[2], v[2];
-            for (int k = 0; k < 2; ++k) {
-                gx[k] = mix(dy, f(b, k) - f(a, k), f(d, k) - f(c, k));
-                gy[k] = mix(dx, f(c, k) - f(a, k), f(d, k) - f(b, k));
-                v[k] = mix(dy, mix(dx, f(a, k), f(b, k)), mix(dx, f(c, k), f(d, k)));
-            }
-            const double ddx = mix(dz, gx[0], gx[1]), ddy = mix(dz, gy[0], gy[1]), ddz = v[1] - v[0];
-            J[q][mc] = -ddx * x / z - ddy * y / z + ddz / h;
-            J[q][(mc + 1) % 3] = ddx * (kRes - 1) / z;
-            J[q][(mc + 2) % 3] = ddy * (kRes - 1) / z;
-        }
+    void snapshot(std::vector<float> &cols, std::vector<double> &z) {
+        std::lock_guard<std::mutex> g(mu_);
+        cols.assign(size_t(3) * kRes * kRes * kRes * 3, std::nanf(""));
+        for (const auto &c : cols_)
+            for (int k = 0; k < kRes; ++k)
+                for (int q = 0; q < 3; ++q) cols[(size_t(c.first) * kRes + k) * 3 + q] = float(c.second[k][q]);
+        z.assign(z_, z_ + kRes);
     }
-
-  public:
 
   private:
     using Column = std::array<std::array<double, 3>, kRes>;
@@ -573,15 +525,9 @@ float pc1d(const float *f, size_t n, float mn, float mx, float *func, float *cdf
 
 }  // namespace
 
-void rgb_to_sigmoid_jacobian_transpose(const float *rgb, const float *coef, size_t n, float *out) {
-    globals().table.jacobian_transpose(rgb, coef, n, out);
-}
-
-void rgb_to_sigmoid_jacobian(const float rgb[3], double J[9]) {
-    double m[3][3];
-    globals().table.jacobian(rgb, m);
-    for (int q = 0; q < 9; ++q) J[q] = m[q / 3][q % 3];
-}
+size_t sigmoid_columns() { return globals().table.count(); }
+void sigmoid_snapshot(std::vector<float> &cols, std::vector<double> &z) { globals().table.snapshot(cols, z); }
+void sigmoid_compute(const float *rgb, size_t n) { globals().table.prefetch(rgb, n, true); }
 
 void rgb_to_sigmoid(const float rgb[3], float out[3]) {
     auto c = globals().table.lookup(rgb);
