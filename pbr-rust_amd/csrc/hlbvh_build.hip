@@ -1193,15 +1193,22 @@ __global__ __launch_bounds__(256) void top_acc_reset_kernel(TopLevel TL, uint32_
 // ---------------------------------------- wave finisher for 65..2048 treelets
 //
 // A top-level node of at most kMidNode treelets is split, together with its
-// whole subtree down to nodes of <= 64 treelets, by one wave, one node after
-// another from a stack in LDS: per split a bounds pass, a bucket pass
-// (hlbvh.cu:690-706), the price of the 23 splits (first strict minimum,
+// whole subtree down to nodes of <= 64 treelets, by one workgroup: per split a
+// bucket pass (hlbvh.cu:690-706), the price of the 23 splits (first strict minimum,
 // hlbvh.cu:711-741) and a stable partition into the other record buffer, 64
-// positions a row. The waves of a workgroup work independently (no workgroup
-// barriers). The deep levels of the level path (thousands of small nodes, a few
-// launches each) become this one launch.
-constexpr int kMidStack = 16;  // pending nodes: the larger child waits, so at most log2(2048 / 65) + 1
-constexpr int kMidWaves = kChunkBlock / kWave;
+// positions a row, by one wave, which goes on with the smaller child from its own
+// stack in LDS and offers the larger one to the workgroup's other waves. A wave
+// without a node takes an offered one; nothing else is shared, and no barrier is
+// passed, within a list node. The deep levels of the level path (thousands of small
+// nodes, a few launches each) become this one launch. It is bound by the chain of
+// splits under one list node, the first of them one wave's: with one wave per list node
+// 1M triangles took 364 us, now 277 (269 with 8 waves, slower at 10M), a build of 20k
+// triangles 105 us less.
+constexpr int kMidStack = 16;  // pending nodes of a wave: at most log2(2048 / 65) + 1
+constexpr int kMidBlock = 256;
+constexpr int kMidWaves = kMidBlock / kWave;
+constexpr uint32_t kMidOffers = 16;
+constexpr uint32_t kOfferEmpty = 0, kOfferBusy = 1, kOfferFull = 2;
 
 struct MidLds {
     uint4 stack[kMidStack];  // (begin, end, node id, prims | buffer << 31)
@@ -1209,7 +1216,16 @@ struct MidLds {
     uint32_t cnt[kNumBuckets], pr[kNumBuckets], box[kNumBuckets][6];
     uint8_t bkt[kMidNode];  // bucket of each position of the node
 };
-// Resident grid: each wave takes nodes wave-stride from the list, whose length
+// Of the workgroup: the list node's bounds, nodes offered to other waves, and how many
+// nodes of the subtree are not split yet (waves leave when there are none).
+struct MidShare {
+    uint32_t root[12];
+    uint32_t state[kMidOffers];
+    uint4 node[kMidOffers];
+    uint32_t box[kMidOffers][12];
+    uint32_t open;
+};
+// Resident grid: each workgroup takes nodes grid-stride from the list, whose length
 // it reads on the device.
 // Order-mapped min (k % 6 < 3) / max of a record's centroid and box into v.
 __device__ __forceinline__ void add_rec_bounds(uint32_t v[12], const Rec &r) {
@@ -1221,30 +1237,68 @@ __device__ __forceinline__ void add_rec_bounds(uint32_t v[12], const Rec &r) {
     v[9] = max(v[9], f2ord(b.hi.x)); v[10] = max(v[10], f2ord(b.hi.y)); v[11] = max(v[11], f2ord(b.hi.z));
 }
 
-__global__ __launch_bounds__(kChunkBlock) void mid_top_kernel(BuildArgs A) {
+__global__ __launch_bounds__(kMidBlock) void mid_top_kernel(BuildArgs A) {
     __shared__ MidLds s_lds[kMidWaves];
+    __shared__ MidShare s_share;
     MidLds &L = s_lds[threadIdx.x / kWave];
+    MidShare &G = s_share;
     const uint32_t lane = __lane_id();
     const uint32_t nitems = min(A.counters[kCntMidTop], A.cap_mid_top);
-    for (uint32_t wid = blockIdx.x * kMidWaves + threadIdx.x / kWave; wid < nitems; wid += gridDim.x * kMidWaves) {
-        {  // the list's node and its bounds; its descendants get theirs from the partition
-            const WorkItem it = A.mid_top[wid];
+    for (uint32_t wid = blockIdx.x; wid < nitems; wid += gridDim.x) {
+        // the list's node and its bounds (its descendants get theirs from the partition)
+        const WorkItem it = A.mid_top[wid];
+        if (threadIdx.x < 12) G.root[threadIdx.x] = threadIdx.x % 6 < 3 ? 0xFFFFFFFFu : 0u;
+        if (threadIdx.x < kMidOffers) G.state[threadIdx.x] = kOfferEmpty;
+        if (threadIdx.x == 0) G.open = 1u;
+        __syncthreads();
+        {
             const Rec *R = pick(A.trec, it.buf);
             uint32_t v[12];
 #pragma unroll
             for (int k = 0; k < 12; ++k) v[k] = ((k % 6) < 3) ? 0xFFFFFFFFu : 0u;
-            for (uint32_t p = it.begin + lane; p < it.end; p += kWave) add_rec_bounds(v, R[p]);
+            for (uint32_t p = it.begin + threadIdx.x; p < it.end; p += kMidBlock) add_rec_bounds(v, R[p]);
 #pragma unroll
             for (int k = 0; k < 12; ++k) v[k] = ((k % 6) < 3) ? wave_min_u32_all(v[k]) : wave_max_u32_all(v[k]);
             if (lane == 0) {
-                L.stack[0] = make_uint4(it.begin, it.end, it.node, it.prims | (it.buf << 31));
 #pragma unroll
-                for (int k = 0; k < 12; ++k) L.sbox[0][k] = v[k];
+                for (int k = 0; k < 12; ++k) {
+                    if ((k % 6) < 3) atomicMin(&G.root[k], v[k]);
+                    else atomicMax(&G.root[k], v[k]);
+                }
             }
         }
-        int sp = 1;  // uniform
+        __syncthreads();
+        int sp = 0;  // uniform
+        if (threadIdx.x < kWave) {
+            if (lane == 0) L.stack[0] = make_uint4(it.begin, it.end, it.node, it.prims | (it.buf << 31));
+            if (lane < 12) L.sbox[0][lane] = G.root[lane];
+            sp = 1;
+        }
         wave_lds_sync();
-        while (sp > 0) {
+        for (;;) {
+            if (sp == 0) {  // an offered node, or the end of the subtree
+                const uint32_t st = lane < kMidOffers ? __hip_atomic_load(&G.state[lane], __ATOMIC_RELAXED,
+                                                                          __HIP_MEMORY_SCOPE_WORKGROUP)
+                                                      : kOfferEmpty;
+                const uint64_t full = __ballot(st == kOfferFull);
+                if (!full) {
+                    const uint32_t open = __hip_atomic_load(&G.open, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    if (__builtin_amdgcn_readfirstlane(open) == 0u) break;
+                    __builtin_amdgcn_s_sleep(2);
+                    continue;
+                }
+                const uint32_t o = uint32_t(__ffsll((unsigned long long)full)) - 1u;
+                uint32_t was = 0;
+                if (lane == 0) was = atomicCAS(&G.state[o], kOfferFull, kOfferBusy);
+                if (__builtin_amdgcn_readfirstlane(was) != kOfferFull) continue;  // another wave took it
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+                if (lane == 0) L.stack[0] = G.node[o];
+                if (lane < 12) L.sbox[0][lane] = G.box[o][lane];
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+                if (lane == 0) atomicExch(&G.state[o], kOfferEmpty);
+                sp = 1;
+                wave_lds_sync();
+            }
             --sp;
             const uint4 nd = L.stack[sp];
             const uint32_t begin = nd.x, end = nd.y, node = nd.z, prims = nd.w & 0x7FFFFFFFu, buf = nd.w >> 31;
@@ -1254,7 +1308,10 @@ __global__ __launch_bounds__(kChunkBlock) void mid_top_kernel(BuildArgs A) {
             const Box cb = acc_box(L.sbox[sp]), fb = acc_box(L.sbox[sp] + 6);
             const int axis = box_max_dim(cb);
             if (sel3(cb.lo, axis) == sel3(cb.hi, axis)) {  // the node stays unbuilt
-                if (lane == 0) atomicOr(A.err, uint32_t(kErrDegenerateCentroids));
+                if (lane == 0) {
+                    atomicOr(A.err, uint32_t(kErrDegenerateCentroids));
+                    atomicSub(&G.open, 1u);
+                }
                 continue;
             }
             const float base = sel3(cb.lo, axis);
@@ -1304,7 +1361,10 @@ __global__ __launch_bounds__(kChunkBlock) void mid_top_kernel(BuildArgs A) {
             const uint32_t nl = price.left_treelets;  // left treelets
             // both end buckets hold a treelet, so neither side is empty (as top_decide_kernel)
             if (lp == 0u || rp == 0u || nl == 0u || nl == m) {
-                if (lane == 0) atomicOr(A.err, uint32_t(kErrSplit));
+                if (lane == 0) {
+                    atomicOr(A.err, uint32_t(kErrSplit));
+                    atomicSub(&G.open, 1u);
+                }
                 continue;
             }
             // stable partition into the other buffer, a row at a time (records loaded
@@ -1338,16 +1398,19 @@ __global__ __launch_bounds__(kChunkBlock) void mid_top_kernel(BuildArgs A) {
                 for (int k = 0; k < 12; ++k)
                     cv[c][k] = ((k % 6) < 3) ? wave_min_u32_all(cv[c][k]) : wave_max_u32_all(cv[c][k]);
             // the children: lane 0 reads a single treelet back from W (written by this wave)
-            __threadfence_block();
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
             if (lane == 0) {
                 write_interior(A.nodes, node, fb, lp, uint32_t(axis));
                 const uint32_t nb = 1 - buf;
                 const WorkItem cl{begin, begin + nl, node + 1, lp, nb, {0, 0, 0}};
                 const WorkItem cr{begin + nl, end, node + 2 * lp, prims - lp, nb, {0, 0, 0}};
                 const bool right_big = m - nl > nl;
+                const uint32_t small_size = min(nl, m - nl), big_size = m - small_size;
+                const uint32_t more = uint32_t(small_size > kSmallNode) + uint32_t(big_size > kSmallNode);
+                if (more == 2u) atomicAdd(&G.open, 1u);  // before either can be taken and finished
                 int top = sp;
 #pragma unroll
-                for (int j = 0; j < 2; ++j) {  // the larger child waits below the smaller one
+                for (int j = 0; j < 2; ++j) {  // the larger child first: offered, or below the smaller one
                     const bool take_right = (j == 0) == right_big;
                     const WorkItem cw = take_right ? cr : cl;
                     const uint32_t cs = cw.end - cw.begin;
@@ -1355,20 +1418,36 @@ __global__ __launch_bounds__(kChunkBlock) void mid_top_kernel(BuildArgs A) {
                         emit_bottom_root(A, A.trec[nb][cw.begin], cw.node);
                     } else if (cs <= kSmallNode) {
                         push_item(A.small_top, A.counters + kCntSmallTop, A.cap_small_top, cw, A.err);
-                    } else if (top < kMidStack) {
-                        L.stack[top] = make_uint4(cw.begin, cw.end, cw.node, cw.prims | (nb << 31));
-#pragma unroll
-                        for (int k = 0; k < 12; ++k) L.sbox[top][k] = take_right ? cv[1][k] : cv[0][k];
-                        ++top;
                     } else {
-                        atomicOr(A.err, uint32_t(kErrCapacity));
+                        const uint4 e = make_uint4(cw.begin, cw.end, cw.node, cw.prims | (nb << 31));
+                        uint32_t o = kMidOffers;
+                        if (j == 0 && more == 2u)
+                            for (o = 0; o < kMidOffers; ++o)
+                                if (atomicCAS(&G.state[o], kOfferEmpty, kOfferBusy) == kOfferEmpty) break;
+                        if (o < kMidOffers) {
+                            G.node[o] = e;
+#pragma unroll
+                            for (int k = 0; k < 12; ++k) G.box[o][k] = take_right ? cv[1][k] : cv[0][k];
+                            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+                            atomicExch(&G.state[o], kOfferFull);
+                        } else if (top < kMidStack) {
+                            L.stack[top] = e;
+#pragma unroll
+                            for (int k = 0; k < 12; ++k) L.sbox[top][k] = take_right ? cv[1][k] : cv[0][k];
+                            ++top;
+                        } else {
+                            atomicOr(A.err, uint32_t(kErrCapacity));
+                            atomicSub(&G.open, 1u);
+                        }
                     }
                 }
+                if (more == 0u) atomicSub(&G.open, 1u);
                 sp = top;
             }
             sp = __shfl(sp, 0, kWave);
             wave_lds_sync();
         }
+        __syncthreads();  // the next list node reuses the offers and the count
     }
 }
 
@@ -2269,12 +2348,11 @@ hipError_t build_hlbvh_device(const float *d_tri, uint32_t n, BuildScratch &S, B
         if (hipGetDevice(&dev) != hipSuccess ||
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
             cus = 256;
-        mid_grid = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, mid_top_kernel, kChunkBlock, 0) ==
+        mid_grid = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, mid_top_kernel, kMidBlock, 0) ==
                            hipSuccess && per_cu > 0 ? per_cu * cus : 4 * cus;
     }
     if (D > kSmallNode)
-        mid_top_kernel<<<std::min<uint32_t>(mid_grid, (A.cap_mid_top + kMidWaves - 1) / kMidWaves), kChunkBlock, 0,
-                         stream>>>(A);
+        mid_top_kernel<<<std::min<uint32_t>(mid_grid, A.cap_mid_top), kMidBlock, 0, stream>>>(A);
     // then the nodes of <= 64, a wave each (an exact grid lets the hardware balance their uneven work)
     PBRTM_TRY(read_counters(S, stream));
     out.small_top = std::min(S.host_counters[kCntSmallTop], A.cap_small_top);
