@@ -54,8 +54,8 @@ FILM_RECORD_BYTES = 16 + 4  # per path: sensor RGB + filter weight, finishing ro
 # with --calibrate-copy), for the default workload. Taken from the profile named
 # beside it, not measured by this run.
 TRAFFIC = {
-    "trace_wide_kernel": (2_014_720_512, "profiles/trace_wide_hlbvh10m_1080p_pmc_traffic.md"),
-    "build": (13_166_864_448, "profiles/trace_wide_hlbvh10m_1080p_pmc_traffic.md"),
+    "trace_wide_kernel": (2_275_583_424, "profiles/trace_wide_hlbvh10m_1080p_pmc_traffic.md"),
+    "build": (13_289_255_040, "profiles/trace_wide_hlbvh10m_1080p_pmc_traffic.md"),
 }
 
 
@@ -538,7 +538,7 @@ def main():
             "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(trace_gbs / HBM_PEAK_GBS, 4),
             "traffic": traffic if default_workload else None,
             "traffic_source": traffic_src if default_workload else None,
-            "limiter": "latency of dependent node fetches (VALU lane use and waves per SIMD in the profile)",
+            "limiter": "VALU issue at 35-38 % lane use (counters in the profile)",
             "bytes_per_launch": int((bytes1 + bytes2) / 2),
             "algorithmic_bytes": "32 B ray + 20/8 B hit + 132 B per 8-wide node visit + 48 B per triangle test"}
     # The headline: the whole build priced at 216 algorithmic bytes per triangle

@@ -858,10 +858,11 @@ __device__ __forceinline__ void trace_wide_persistent_body(const WideTrace &B, c
     add_counts<COUNT>(counts, visits, boxes, tests);
 }
 
-// The occupancy targets and the refill threshold come from measurement: the
-// persistent single-tree traversal runs fastest at 5 waves per SIMD with refills
-// at 8 idle lanes (6 waves: -10 %; 16 lanes: -4 %), the per-ray-tree one at 5;
-// the LDS stack (24 KiB per block) allows 6.
+// The occupancy floor of 5 waves per SIMD keeps the registers of the per-ray-tree and the
+// analytic instances within 96 without spills; the single-tree triangle instance needs 78
+// and runs at the 6 that the LDS stack (24 KiB per block) allows. Held to 6, the
+// per-ray-tree one spills four registers: 16 mixed jobs 5.46 -> 5.62 ms. Refills at 8 idle
+// lanes (16 lanes: -4 %).
 // SHAPES: trees with analytic primitives (a leaf position whose pad word holds a
 // shape index + 1); triangle-only trees take the instance without that branch.
 template <bool COUNT, bool SHAPES>
