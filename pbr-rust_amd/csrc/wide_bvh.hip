@@ -753,7 +753,7 @@ __device__ __forceinline__ void add_counts(unsigned long long *counts, uint32_t 
 // finished, wide_ray_finish), so which lane or wave takes it changes nothing. MULTI: every ray selects its own
 // tree, jw[ray_job[i >> job_shift]] (jobs of a batched render); the spill area
 // stays the launch's.
-constexpr uint32_t kRefill = 8;
+constexpr uint32_t kRefill = 16;
 constexpr uint32_t kWideWaves = kWideBlock / kWave;
 // Slots of a row: a queue with less than kWave rays for each of kSpread waves (one per
 // SIMD) is spread over them in shorter rows. A short launch lasts as long as its
@@ -769,13 +769,13 @@ __host__ __device__ constexpr uint32_t wide_row(uint32_t n) {
 constexpr uint32_t kDealt = 5;
 // A wave steps either its lanes that wait at a node or those that wait at a leaf's
 // primitive, never both paths for a few lanes each: the leaves go when they are at
-// least a quarter of the others. Waiting longer fills the leaf steps but idles more
-// lanes (and delays a wave's last rays): 1/4 against 1/6, 1/8, 1/12 or a fixed count
-// of 8 lanes was fastest or within 1 % on camera, bounce and shadow queues and path
-// tracing. Against testing every leaf where a lane met it: 1080p camera rays into 10M
+// least a third of the others. Waiting longer fills the leaf steps but idles more
+// lanes (and delays a wave's last rays): 33M path-traced paths 105.8 ms at 1/4, 105.1 at
+// 1/3, 107.1 at 1/6; 1/2 slows short queues (16 mixed jobs +1 %); 1/8, 1/12 and a fixed
+// count of 8 lanes are slower still. Against testing every leaf where a lane met it: 1080p camera rays into 10M
 // triangles 1780 -> 1246 us, shadow rays into 1M 909 -> 701 us, 999 rays 209 -> 178 us
 // (and 96 -> 75 VGPRs, 6 waves per SIMD).
-constexpr uint32_t kLeafShare = 4;
+constexpr uint32_t kLeafShare = 3;
 
 template <bool COUNT, bool MULTI, bool SHAPES>
 __device__ __forceinline__ void trace_wide_persistent_body(const WideTrace &B, const float4 *__restrict__ rays,
@@ -861,8 +861,10 @@ __device__ __forceinline__ void trace_wide_persistent_body(const WideTrace &B, c
 // The occupancy floor of 5 waves per SIMD keeps the registers of the per-ray-tree and the
 // analytic instances within 96 without spills; the single-tree triangle instance needs 78
 // and runs at the 6 that the LDS stack (24 KiB per block) allows. Held to 6, the
-// per-ray-tree one spills four registers: 16 mixed jobs 5.46 -> 5.62 ms. Refills at 8 idle
-// lanes (16 lanes: -4 %).
+// per-ray-tree one spills four registers: 16 mixed jobs 5.46 -> 5.62 ms. A refill
+// waits for 16 idle lanes: the rays' start (two loads, reciprocals, shear) costs a step of
+// the whole wave. With 4, 8 and 16 the path-traced paths above take 107.3, 105.8 and 105.0
+// ms, with the third above 104.4; 24 gains nothing there and slows camera rays by 2 %.
 // SHAPES: trees with analytic primitives (a leaf position whose pad word holds a
 // shape index + 1); triangle-only trees take the instance without that branch.
 template <bool COUNT, bool SHAPES>
