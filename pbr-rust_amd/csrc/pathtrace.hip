@@ -1747,6 +1747,8 @@ hipError_t render(const SceneDev &S, const WideTrace &W0, uint32_t spp, uint32_t
 
 namespace {
 
+constexpr uint32_t kMaxLaunchRounds = 1024;
+
 // Every job of `jobs` in one shared pool (the batched wavefront).
 hipError_t render_shared(const std::vector<BatchJob> &jobs, uint32_t pool, uint32_t rounds_per_launch, bool use_graph,
                          PathPool &pp, DevBuf &jobbuf, uint32_t *err, BatchStats *stats, hipStream_t stream,
@@ -1785,7 +1787,9 @@ hipError_t render_shared(const std::vector<BatchJob> &jobs, uint32_t pool, uint3
         if ((e = (x)) != hipSuccess) return e; \
     } while (0)
     PT_CK(reserve_pool(pp, pool, total, true, false));  // the captured rounds allocate nothing
-    rounds_per_launch += rounds_per_launch & 1u;         // the queues' parity is the round's within a launch
+    // the queues' parity is the round's within a launch, so a launch holds an even number;
+    // more than kMaxLaunchRounds (2048 traces and as many kernels more) save nothing
+    rounds_per_launch = (std::min(rounds_per_launch, kMaxLaunchRounds) + 1u) & ~1u;
     WideTrace W{};
     W.spill_per_ray = spill_need;
     W.grid_quarters = grid_quarters;
