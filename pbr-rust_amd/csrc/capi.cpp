@@ -1084,11 +1084,12 @@ int pbrtm_render_grad(pbrtm_ctx *ctx, pbrtm_scene *sc, const pbrtm_render_params
                                                reinterpret_cast<const double *>(ctx->sig_cols.as<float>() + kCols), nm,
                                                sc->g_albedo.as<float>(), err + 1, st), "albedo gradient");
             CK(ctx, hipMemcpyAsync(&missing, err + 1, 4, hipMemcpyDeviceToHost, st), "download");
-            CK(ctx, hipMemcpyAsync(d_albedo, sc->g_albedo.ptr, size_t(nm) * 12, hipMemcpyDeviceToHost, st), "download");
             CK(ctx, hipStreamSynchronize(st), "sync");
             if (!missing) break;
+            if (pass == 1) return fail(ctx, PBRTM_ERR_DEVICE, "RGB-to-spectrum table: a column of an albedo is missing");
             pbrtm::pt::sigmoid_compute(H.mat_rgb.data(), nm);  // columns that no lookup needed (grey albedos)
         }
+        CK(ctx, hipMemcpyAsync(d_albedo, sc->g_albedo.ptr, size_t(nm) * 12, hipMemcpyDeviceToHost, st), "download");
     }
     CK(ctx, hipMemcpyAsync(&derr, err, 4, hipMemcpyDeviceToHost, st), "download");
     CK(ctx, hipMemcpyAsync(hacc.data(), acc, hacc.size() * 8, hipMemcpyDeviceToHost, st), "download");

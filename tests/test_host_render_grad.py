@@ -1,0 +1,67 @@
+"""pbrtm_render_grad's host path on a runtime without a device: what a call that fails leaves
+behind, and what it returns."""
+import ctypes
+import os
+import sys
+
+import numpy as np
+
+sys.path[:0] = [os.path.dirname(os.path.abspath(__file__)),
+                os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "pbr-rust_amd")]
+import fake_hip  # noqa: E402
+
+SENTINEL = -7.0
+
+
+def grad(ctx, scene, materials, d_scale=None):
+    """(return code, loss, d_albedo) with outputs that start as sentinels."""
+    import pbrtm
+
+    target = np.zeros((scene.height, scene.width, 3), np.float32)
+    d_albedo = np.full((materials, 3), SENTINEL, np.float32)
+    loss = ctypes.c_double(SENTINEL)
+    params = pbrtm.RenderParams(4, 2, 0, 0)
+    rc = ctx.lib.pbrtm_render_grad(ctx.h, scene.h, ctypes.byref(params), pbrtm._ptr(target), None,
+                                   ctypes.byref(loss), pbrtm._ptr(d_albedo), None, None)
+    return rc, loss.value, d_albedo
+
+
+def room():
+    """A small all-diffuse room of grey albedos, whose table columns no lookup has computed."""
+    from pbrtm import scenes
+
+    sc = scenes.grad_room(20, 4, 4, spp=4, max_depth=2)
+    sc["albedo"] = np.full_like(sc["albedo"], 0.5)
+    return sc
+
+
+def columns_stay_missing():
+    calls = []
+
+    def launch(kernel, blocks, threads, captured, args):
+        if "albedo_gradient" in kernel:  # (rgb, mats, coef, cols, z, n, out, missing)
+            calls.append(kernel)
+            fake_hip.poke_u32(fake_hip.pointer(args, 7), 1)
+
+    fake_hip.install(launch)
+    import pbrtm
+
+    with pbrtm.Context(0) as ctx:
+        sc = room()
+        scene = ctx.scene(sc)
+        rc, _, d_albedo = grad(ctx, scene, len(sc["albedo"]))
+        assert len(calls) == 2  # once more after the missing columns were computed
+        assert rc == pbrtm.ERR_DEVICE, rc
+        assert b"RGB-to-spectrum" in ctx.lib.pbrtm_last_error(ctx.h)
+        assert (d_albedo == SENTINEL).all()
+        scene.free()
+
+
+@fake_hip.needs_compiler
+def test_columns_that_stay_missing_are_an_error(tmp_path):
+    """Never gradients of NaN columns."""
+    fake_hip.isolated(__file__, "columns_stay_missing", tmp_path)
+
+
+if __name__ == "__main__":
+    fake_hip.main(globals())
