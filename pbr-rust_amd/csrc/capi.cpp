@@ -1052,8 +1052,11 @@ int pbrtm_render_grad(pbrtm_ctx *ctx, pbrtm_scene *sc, const pbrtm_render_params
     CK(ctx, pbrtm::pt::render(sc->dev, W, spp, params->max_depth, pool, sc->pool, nullptr, nullptr, err, &rep, st,
                               nullptr, nullptr, &gd), "replay");
     const auto t3 = std::chrono::steady_clock::now();
-    std::vector<double> hacc(ng + 2);
     uint32_t derr = 0;
+    CK(ctx, hipMemcpyAsync(&derr, err, 4, hipMemcpyDeviceToHost, st), "download");
+    CK(ctx, hipStreamSynchronize(st), "sync");
+    if (derr) return fail(ctx, PBRTM_ERR_DEVICE, device_error_text(derr));  // before any output is written
+    std::vector<double> hacc(ng + 2);
     if (d_albedo && nm) {  // J^T through the RGB-to-spectrum table (non-diffuse materials: zero)
         if (!sc->g_rgb.ptr) {
             CK(ctx, sc->g_rgb.reserve(size_t(nm) * 12), "alloc");
@@ -1091,11 +1094,9 @@ int pbrtm_render_grad(pbrtm_ctx *ctx, pbrtm_scene *sc, const pbrtm_render_params
         }
         CK(ctx, hipMemcpyAsync(d_albedo, sc->g_albedo.ptr, size_t(nm) * 12, hipMemcpyDeviceToHost, st), "download");
     }
-    CK(ctx, hipMemcpyAsync(&derr, err, 4, hipMemcpyDeviceToHost, st), "download");
     CK(ctx, hipMemcpyAsync(hacc.data(), acc, hacc.size() * 8, hipMemcpyDeviceToHost, st), "download");
     if (film_rgb) CK(ctx, hipMemcpyAsync(film_rgb, film, wh * 12, hipMemcpyDeviceToHost, st), "download");
     CK(ctx, hipStreamSynchronize(st), "sync");
-    if (derr) return fail(ctx, PBRTM_ERR_DEVICE, device_error_text(derr));
     *loss = hacc[ng + 1];
     if (d_scale) {  // dLoss/ds_m = (a_m - k P_m) / s_m, P_m = the emitter's total pmf
         std::vector<double> P(ng, 0.0);

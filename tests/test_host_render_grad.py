@@ -57,6 +57,29 @@ def columns_stay_missing():
         scene.free()
 
 
+def device_error():
+    def launch(kernel, blocks, threads, captured, args):
+        if "trace_wide_kernel" in kernel:  # (tree, rays, queue, length, any_hit, prim, t, bary, err, counts)
+            fake_hip.poke_u32(fake_hip.pointer(args, 8), 8)  # a traversal stack overflow
+
+    fake_hip.install(launch)
+    import pbrtm
+
+    with pbrtm.Context(0) as ctx:
+        sc = room()
+        scene = ctx.scene(sc)
+        rc, loss, d_albedo = grad(ctx, scene, len(sc["albedo"]))
+        assert rc == pbrtm.ERR_DEVICE, rc
+        assert b"traversal stack" in ctx.lib.pbrtm_last_error(ctx.h)
+        assert loss == SENTINEL and (d_albedo == SENTINEL).all()
+        scene.free()
+
+
+@fake_hip.needs_compiler
+def test_device_error_leaves_the_outputs_alone(tmp_path):
+    fake_hip.isolated(__file__, "device_error", tmp_path)
+
+
 @fake_hip.needs_compiler
 def test_columns_that_stay_missing_are_an_error(tmp_path):
     """Never gradients of NaN columns."""
