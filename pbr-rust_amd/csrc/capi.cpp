@@ -1057,7 +1057,7 @@ int pbrtm_render_grad(pbrtm_ctx *ctx, pbrtm_scene *sc, const pbrtm_render_params
     CK(ctx, hipStreamSynchronize(st), "sync");
     if (derr) return fail(ctx, PBRTM_ERR_DEVICE, device_error_text(derr));  // before any output is written
     std::vector<double> hacc(ng + 2);
-    if (d_albedo && nm) {  // J^T through the RGB-to-spectrum table (non-diffuse materials: zero)
+    if (d_albedo && nm) try {  // J^T through the RGB-to-spectrum table (non-diffuse materials: zero)
         if (!sc->g_rgb.ptr) {
             CK(ctx, sc->g_rgb.reserve(size_t(nm) * 12), "alloc");
             CK(ctx, hipMemcpyAsync(sc->g_rgb.ptr, H.mat_rgb.data(), size_t(nm) * 12, hipMemcpyHostToDevice, st), "upload");
@@ -1065,21 +1065,17 @@ int pbrtm_render_grad(pbrtm_ctx *ctx, pbrtm_scene *sc, const pbrtm_render_params
         CK(ctx, sc->g_albedo.reserve(size_t(nm) * 12), "alloc");
         for (int pass = 0; pass < 2; ++pass) {
             uint32_t missing = 0;
-            try {
-                const size_t have = pbrtm::pt::sigmoid_columns();
-                if (!ctx->sig_cols.ptr || ctx->sig_count != have) {
-                    std::vector<float> cols;
-                    std::vector<double> z;
-                    pbrtm::pt::sigmoid_snapshot(cols, z);
-                    CK(ctx, ctx->sig_cols.reserve(cols.size() * 4 + z.size() * 8), "alloc");
-                    CK(ctx, hipMemcpyAsync(ctx->sig_cols.ptr, cols.data(), cols.size() * 4, hipMemcpyHostToDevice, st), "upload");
-                    CK(ctx, hipMemcpyAsync(ctx->sig_cols.as<uint8_t>() + cols.size() * 4, z.data(), z.size() * 8,
-                                           hipMemcpyHostToDevice, st), "upload");
-                    CK(ctx, hipStreamSynchronize(st), "upload");  // the vectors end here
-                    ctx->sig_count = have;
-                }
-            } catch (const std::bad_alloc &) {
-                return fail(ctx, PBRTM_ERR_NOMEM, "RGB-to-spectrum table");
+            const size_t have = pbrtm::pt::sigmoid_columns();
+            if (!ctx->sig_cols.ptr || ctx->sig_count != have) {
+                std::vector<float> cols;
+                std::vector<double> z;
+                pbrtm::pt::sigmoid_snapshot(cols, z);
+                CK(ctx, ctx->sig_cols.reserve(cols.size() * 4 + z.size() * 8), "alloc");
+                CK(ctx, hipMemcpyAsync(ctx->sig_cols.ptr, cols.data(), cols.size() * 4, hipMemcpyHostToDevice, st), "upload");
+                CK(ctx, hipMemcpyAsync(ctx->sig_cols.as<uint8_t>() + cols.size() * 4, z.data(), z.size() * 8,
+                                       hipMemcpyHostToDevice, st), "upload");
+                CK(ctx, hipStreamSynchronize(st), "upload");  // the vectors end here
+                ctx->sig_count = have;
             }
             constexpr size_t kCols = size_t(3) * pbrtm::pt::kSigmoidRes * pbrtm::pt::kSigmoidRes * pbrtm::pt::kSigmoidRes * 3;
             CK(ctx, hipMemsetAsync(err + 1, 0, 4, st), "memset");
@@ -1093,6 +1089,10 @@ int pbrtm_render_grad(pbrtm_ctx *ctx, pbrtm_scene *sc, const pbrtm_render_params
             pbrtm::pt::sigmoid_compute(H.mat_rgb.data(), nm);  // columns that no lookup needed (grey albedos)
         }
         CK(ctx, hipMemcpyAsync(d_albedo, sc->g_albedo.ptr, size_t(nm) * 12, hipMemcpyDeviceToHost, st), "download");
+    } catch (const std::bad_alloc &) {
+        return fail(ctx, PBRTM_ERR_NOMEM, "RGB-to-spectrum table");
+    } catch (const std::exception &x) {
+        return fail(ctx, PBRTM_ERR_INVALID, x.what());
     }
     CK(ctx, hipMemcpyAsync(hacc.data(), acc, hacc.size() * 8, hipMemcpyDeviceToHost, st), "download");
     if (film_rgb) CK(ctx, hipMemcpyAsync(film_rgb, film, wh * 12, hipMemcpyDeviceToHost, st), "download");

@@ -6,13 +6,16 @@
 // per scene.
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <cmath>
 #include <cstring>
+#include <exception>
 #include <limits>
 #include <map>
 #include <mutex>
 #include <stdexcept>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -407,14 +410,29 @@ class SpectrumTable {
         }
         if (keys.empty()) return;
         std::vector<Column> out(keys.size());
-        const unsigned nt = std::max(1u, std::min<unsigned>(std::thread::hardware_concurrency(), 64u));
-        std::vector<std::thread> ts;
-        for (unsigned t = 0; t < nt; ++t)
-            ts.emplace_back([&, t] {
-                for (size_t k = t; k < keys.size(); k += nt)
+        // The threads that can be started, and this one, take columns in turn; what one of
+        // them throws is thrown here once all have ended.
+        std::atomic<size_t> next{0};
+        std::exception_ptr thrown;
+        auto work = [&] {
+            try {
+                for (size_t k; (k = next.fetch_add(1)) < keys.size();)
                     out[k] = compute(keys[k] / (kRes * kRes), (keys[k] / kRes) % kRes, keys[k] % kRes);
-            });
+            } catch (...) {
+                std::lock_guard<std::mutex> g(mu_);
+                thrown = std::current_exception();
+            }
+        };
+        const size_t nt = std::max(1u, std::min<unsigned>(std::thread::hardware_concurrency(), 64u));
+        std::vector<std::thread> ts;
+        ts.reserve(nt);
+        try {
+            while (ts.size() + 1 < std::min(nt, keys.size())) ts.emplace_back(work);
+        } catch (const std::system_error &) {  // no more threads
+        }
+        work();
         for (auto &th : ts) th.join();
+        if (thrown) std::rethrow_exception(thrown);
         std::lock_guard<std::mutex> g(mu_);
         for (size_t k = 0; k < keys.size(); ++k) cols_.emplace(keys[k], out[k]);
     }

@@ -75,6 +75,39 @@ def device_error():
         scene.free()
 
 
+def no_threads():
+    """Missing columns where no thread can be started and little can be allocated (an address
+    space limit a few MB above what is in use)."""
+    import resource
+
+    old = resource.getrlimit(resource.RLIMIT_AS)
+
+    def launch(kernel, blocks, threads, captured, args):
+        if "albedo_gradient" in kernel:
+            used = 4096 * int(open("/proc/self/statm").read().split()[0])
+            resource.setrlimit(resource.RLIMIT_AS, (used + (4 << 20), old[1]))
+            fake_hip.poke_u32(fake_hip.pointer(args, 7), 1)
+
+    fake_hip.install(launch)
+    import pbrtm
+
+    with pbrtm.Context(0) as ctx:
+        sc = room()
+        scene = ctx.scene(sc)
+        rc, _, d_albedo = grad(ctx, scene, len(sc["albedo"]))
+        resource.setrlimit(resource.RLIMIT_AS, old)
+        # the columns are computed without threads; then the table's copy does not fit, or the
+        # second run reports the albedos missing again
+        assert rc in (pbrtm.ERR_NOMEM, pbrtm.ERR_DEVICE), rc
+        assert (d_albedo == SENTINEL).all()
+        scene.free()
+
+
+@fake_hip.needs_compiler
+def test_no_exception_leaves_the_call(tmp_path):
+    fake_hip.isolated(__file__, "no_threads", tmp_path)
+
+
 @fake_hip.needs_compiler
 def test_device_error_leaves_the_outputs_alone(tmp_path):
     fake_hip.isolated(__file__, "device_error", tmp_path)
