@@ -1060,7 +1060,10 @@ int pbrtm_render_grad(pbrtm_ctx *ctx, pbrtm_scene *sc, const pbrtm_render_params
     if (d_albedo && nm) try {  // J^T through the RGB-to-spectrum table (non-diffuse materials: zero)
         if (!sc->g_rgb.ptr) {
             CK(ctx, sc->g_rgb.reserve(size_t(nm) * 12), "alloc");
-            CK(ctx, hipMemcpyAsync(sc->g_rgb.ptr, H.mat_rgb.data(), size_t(nm) * 12, hipMemcpyHostToDevice, st), "upload");
+            const hipError_t e =
+                hipMemcpyAsync(sc->g_rgb.ptr, H.mat_rgb.data(), size_t(nm) * 12, hipMemcpyHostToDevice, st);
+            if (e != hipSuccess) sc->g_rgb.release();
+            CK(ctx, e, "upload");
         }
         CK(ctx, sc->g_albedo.reserve(size_t(nm) * 12), "alloc");
         for (int pass = 0; pass < 2; ++pass) {

@@ -75,6 +75,37 @@ def device_error():
         scene.free()
 
 
+def failed_upload():
+    """The first gradient's upload of the albedos fails; the next one has to upload them."""
+    rgb = []
+
+    def launch(kernel, blocks, threads, captured, args):
+        if "albedo_gradient" in kernel:
+            raw = (ctypes.c_float * (3 * n)).from_address(fake_hip.pointer(args, 0))
+            rgb.append(np.array(raw, np.float32).reshape(n, 3))
+
+    lib = fake_hip.install(launch)
+    import pbrtm
+
+    sc = room()
+    sc["albedo"] = np.random.default_rng(1).uniform(0.1, 0.9, sc["albedo"].shape).astype(np.float32)
+    n = len(sc["albedo"])
+    with pbrtm.Context(0) as ctx:
+        scene = ctx.scene(sc)
+        lib.fake_hip_fail_copy(ctypes.c_uint64(12 * n))
+        rc, _, d_albedo = grad(ctx, scene, n)
+        assert rc == pbrtm.ERR_HIP and not rgb and (d_albedo == SENTINEL).all(), rc
+        rc, _, _ = grad(ctx, scene, n)
+        assert rc == pbrtm.OK and len(rgb) == 1
+        assert np.array_equal(rgb[0], sc["albedo"])
+        scene.free()
+
+
+@fake_hip.needs_compiler
+def test_albedos_are_uploaded_after_a_failed_upload(tmp_path):
+    fake_hip.isolated(__file__, "failed_upload", tmp_path)
+
+
 def no_threads():
     """Missing columns where no thread can be started and little can be allocated (an address
     space limit a few MB above what is in use)."""
