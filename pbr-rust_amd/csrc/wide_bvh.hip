@@ -414,9 +414,9 @@ __global__ __launch_bounds__(kCompactBlock) void compact_rays_kernel(const float
 }
 
 // Traversal state of one ray. binv / berr: the box tests' reciprocal direction
-// (clamped, finite) and per-axis constant error term (wide_ray_start). Instead of the
-// direction it holds the triangle test's shear; ray_dir fetches the direction again
-// where an unusual case needs it.
+// (clamped, finite; unclamped for a ray that starts as kRayGeneric) and per-axis constant
+// error term (wide_ray_start). Instead of the direction it holds the triangle test's
+// shear; ray_dir fetches the direction again where an unusual case needs it.
 struct WideRay {
     f3 o, binv, berr;
     RayShear sh;
@@ -528,7 +528,10 @@ __device__ __forceinline__ bool wide_ray_start(WideRay &R, const float4 *__restr
     R.berr = {box_err_const(R.o.x, inv.x, R.binv.x, least), box_err_const(R.o.y, inv.y, R.binv.y, least),
               box_err_const(R.o.z, inv.z, R.binv.z, least)};
     const float span = fabsf(R.o.x) + fabsf(R.o.y) + fabsf(R.o.z) + fabsf(d.x) + fabsf(d.y) + fabsf(d.z);
-    if (!(least <= 0x1p20f && span <= 0x1p60f)) R.oct |= kRayGeneric;
+    if (!(least <= 0x1p20f && span <= 0x1p60f)) {
+        R.oct |= kRayGeneric;
+        R.binv = inv;
+    }
     R.node = 0;
     R.pmask = 0xFFu;
     R.sp = 0;
@@ -548,22 +551,30 @@ __device__ __forceinline__ void wide_ray_finish(const WideRay &R, uint32_t *__re
     }
 }
 
-// Hit mask of a node's slots for a ray outside box_axis' range: each slot's decoded
-// planes through the reference's slab test.
-__device__ __forceinline__ uint32_t wide_box_generic(const WNode *W, const WideRay &R) {
-    const int neg[3] = {int(R.oct & 1u), int((R.oct >> 1) & 1u), int((R.oct >> 2) & 1u)};
-    const f3 d = ray_dir(R), inv = {1.0f / d.x, 1.0f / d.y, 1.0f / d.z};
+// Hit mask of a node's slots for a ray outside box_axis' range (WideRay::binv is its
+// unclamped reciprocal): each slot's decoded planes through the reference's slab test,
+// near and far already chosen by the direction's signs. Bound by instruction issue like
+// the test it stands in for, so it decodes the words at hand, all slots in line; slot by
+// slot (the scheduling barrier), because all decodes at once spill registers in every
+// instance of the kernel. 2M rays with directions of length 2^-24 into 1M triangles: 5.0
+// ms; as a loop over byte loads of the node 22.9 ms; in halves of four slots 8.7 ms.
+__device__ __forceinline__ uint32_t wide_box_generic(uint4 hd, const uint32_t nw[3][2], const uint32_t fw[3][2],
+                                                     const WideRay &R) {
+    const float org[3] = {__uint_as_float(hd.x), __uint_as_float(hd.y), __uint_as_float(hd.z)};
+    const float step[3] = {pow2f(int(int8_t(hd.w & 0xFFu))), pow2f(int(int8_t((hd.w >> 8) & 0xFFu))),
+                           pow2f(int(int8_t((hd.w >> 16) & 0xFFu)))};
+    const int no_neg[3] = {0, 0, 0};
     uint32_t hs = 0;
-#pragma unroll 1
+#pragma unroll
     for (int s = 0; s < kWide; ++s) {
-        float lo[3], hi[3];
+        float np[3], fp[3];
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
-            const float step = pow2f(W->exp[a]);
-            lo[a] = fmaf(float(W->q[a][s]), step, W->org[a]);
-            hi[a] = fmaf(float(W->q[a + 3][s]), step, W->org[a]);
+            np[a] = fmaf(float((nw[a][s / 4] >> (8 * (s % 4))) & 0xFFu), step[a], org[a]);
+            fp[a] = fmaf(float((fw[a][s / 4] >> (8 * (s % 4))) & 0xFFu), step[a], org[a]);
         }
-        hs |= box_hit(lo, hi, R.o, inv, neg, R.best_t) ? 1u << s : 0u;
+        hs |= box_hit(np, fp, R.o, R.binv, no_neg, R.best_t) ? 1u << s : 0u;
+        __builtin_amdgcn_sched_barrier(0);
     }
     return hs;
 }
@@ -633,10 +644,6 @@ __device__ __forceinline__ bool wide_node(WideRay &R, const WideTree &T, uint32_
     // bytes), hit mask in slot order
     const uint4 *q = reinterpret_cast<const uint4 *>(W);
     const uint4 hd = q[0];
-    const BoxAxis ax[3] = {
-        box_axis(__uint_as_float(hd.x), pow2f(int(int8_t(hd.w & 0xFFu))), R.o.x, R.binv.x, R.berr.x),
-        box_axis(__uint_as_float(hd.y), pow2f(int(int8_t((hd.w >> 8) & 0xFFu))), R.o.y, R.binv.y, R.berr.y),
-        box_axis(__uint_as_float(hd.z), pow2f(int(int8_t((hd.w >> 16) & 0xFFu))), R.o.z, R.binv.z, R.berr.z)};
     uint32_t qw[12];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
@@ -660,22 +667,30 @@ __device__ __forceinline__ bool wide_node(WideRay &R, const WideTree &T, uint32_
             fw[a][h] = (lo & m) | (hi & ~m);
         }
     }
-    // a miss is a negative (far - near), its sign bit shifted into place
-    uint32_t miss = 0;
+    uint32_t hs;
+    if (R.oct & kRayGeneric) {
+        hs = wide_box_generic(hd, nw, fw, R);
+    } else {
+        const BoxAxis ax[3] = {
+            box_axis(__uint_as_float(hd.x), pow2f(int(int8_t(hd.w & 0xFFu))), R.o.x, R.binv.x, R.berr.x),
+            box_axis(__uint_as_float(hd.y), pow2f(int(int8_t((hd.w >> 8) & 0xFFu))), R.o.y, R.binv.y, R.berr.y),
+            box_axis(__uint_as_float(hd.z), pow2f(int(int8_t((hd.w >> 16) & 0xFFu))), R.o.z, R.binv.z, R.berr.z)};
+        // a miss is a negative (far - near), its sign bit shifted into place
+        uint32_t miss = 0;
 #pragma unroll
-    for (int s = kWide - 1; s >= 0; --s) {
-        float tn[3], tf[3];
+        for (int s = kWide - 1; s >= 0; --s) {
+            float tn[3], tf[3];
 #pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            tn[a] = fmaf(float((nw[a][s / 4] >> (8 * (s % 4))) & 0xFFu), ax[a].a, ax[a].bn);
-            tf[a] = fmaf(float((fw[a][s / 4] >> (8 * (s % 4))) & 0xFFu), ax[a].a, ax[a].bf);
+            for (int a = 0; a < 3; ++a) {
+                tn[a] = fmaf(float((nw[a][s / 4] >> (8 * (s % 4))) & 0xFFu), ax[a].a, ax[a].bn);
+                tf[a] = fmaf(float((fw[a][s / 4] >> (8 * (s % 4))) & 0xFFu), ax[a].a, ax[a].bf);
+            }
+            const float lo = fmaxf(fmaxf(fmaxf(tn[0], tn[1]), tn[2]), 0.0f);
+            const float hi = fminf(fminf(fminf(tf[0], tf[1]), tf[2]), R.best_t);
+            miss = __builtin_amdgcn_alignbit(miss, __float_as_uint(hi - lo), 31);
         }
-        const float lo = fmaxf(fmaxf(fmaxf(tn[0], tn[1]), tn[2]), 0.0f);
-        const float hi = fminf(fminf(fminf(tf[0], tf[1]), tf[2]), R.best_t);
-        miss = __builtin_amdgcn_alignbit(miss, __float_as_uint(hi - lo), 31);
+        hs = ~miss & 0xFFu;
     }
-    uint32_t hs = ~miss & 0xFFu;
-    if (R.oct & kRayGeneric) hs = wide_box_generic(W, R);
     // ... then in depth-first position order: hm bit p = hs bit (slot at position p).
     // The hit bits become bytes (slot s -> byte s of {d1, d0}), a byte permute
     // gathers them by the position's slot code (an unused position's code 12
@@ -774,7 +789,7 @@ constexpr uint32_t kDealt = 5;
 // 1/3, 107.1 at 1/6; 1/2 slows short queues (16 mixed jobs +1 %); 1/8, 1/12 and a fixed
 // count of 8 lanes are slower still. Against testing every leaf where a lane met it: 1080p camera rays into 10M
 // triangles 1780 -> 1246 us, shadow rays into 1M 909 -> 701 us, 999 rays 209 -> 178 us
-// (and 96 -> 75 VGPRs, 6 waves per SIMD).
+// (and 96 -> 74 VGPRs, 6 waves per SIMD).
 constexpr uint32_t kLeafShare = 3;
 
 template <bool COUNT, bool MULTI, bool SHAPES>
@@ -859,7 +874,7 @@ __device__ __forceinline__ void trace_wide_persistent_body(const WideTrace &B, c
 }
 
 // The occupancy floor of 5 waves per SIMD keeps the registers of the per-ray-tree and the
-// analytic instances within 96 without spills; the single-tree triangle instance needs 78
+// analytic instances within 96 without spills; the single-tree triangle instance needs 74
 // and runs at the 6 that the LDS stack (24 KiB per block) allows. Held to 6, the
 // per-ray-tree one spills four registers: 16 mixed jobs 5.46 -> 5.62 ms. A refill
 // waits for 16 idle lanes: the rays' start (two loads, reciprocals, shear) costs a step of

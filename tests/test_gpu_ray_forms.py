@@ -108,3 +108,34 @@ def test_ray_forms(ctx, scene, form):
                     assert _same(t[hit], ot[hit])
                     assert _same(bary[hit], ob[hit])
     bvh.free()
+
+
+def test_short_directions_take_as_long_as_others(ctx):
+    """Rays on both sides of the range of the conservative box test (directions shorter than
+    2^-20 take the reference's own test): a queue of them takes at most twice the time."""
+    import time
+
+    from test_zz_no_alloc import DeviceArray
+
+    n = 230_400
+    bvh = ctx.build(pbrtm.gen_soup(1_000_000, seed=41))
+    rng = np.random.default_rng(41)
+    d = rng.normal(size=(n, 3))
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    prim, took = DeviceArray((n,), np.uint32), {}
+    for length in (2.0 ** -18, 2.0 ** -24):
+        rays = np.zeros((n, 8), np.float32)
+        rays[:, 0:3] = np.random.default_rng(42).uniform(size=(n, 3))
+        rays[:, 3] = np.inf
+        rays[:, 4:7] = d * length
+        dev, times = DeviceArray(rays.shape, np.float32, rays), []
+        for _ in range(12):
+            t0 = time.perf_counter()
+            bvh.intersect(dev, device_ptrs=True, prim=prim)
+            times.append(time.perf_counter() - t0)
+        took[length] = float(np.median(times[2:]))
+        print(f"directions of length {length:.3g}: {took[length] * 1e6:.0f} us", flush=True)
+        dev.free()
+    prim.free()
+    bvh.free()
+    assert took[2.0 ** -24] <= 2 * took[2.0 ** -18], took
