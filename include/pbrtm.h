@@ -117,7 +117,8 @@ int pbrtm_bvh_export_canonical(const pbrtm_bvh *bvh, uint8_t *buf, uint64_t *len
  * The 8-wide traversal tests triangles in exactly the reference's order, so hits
  * (ties included) equal the binary traversal's. stats_out (host, may be NULL)
  * receives [nodes visited, box tests, triangle tests] summed over the rays; it
- * selects a counting instance of the same traversal. */
+ * selects a counting instance of the same traversal. A node whose boxes are tested
+ * again after a hit in one of its leaves adds 8 box tests and no visit. */
 int pbrtm_bvh_intersect(pbrtm_bvh *bvh, const float *rays, uint64_t n, int any_hit, uint32_t flags,
                         uint32_t *prim_out, float *t_out, float *bary_out, uint64_t *stats_out);
 

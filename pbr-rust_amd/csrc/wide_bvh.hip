@@ -859,9 +859,12 @@ __device__ __forceinline__ void trace_wide_persistent_body(const WideTrace &B, c
         if (uint32_t(__popcll(leaves)) * kLeafShare >= uint32_t(__popcll(~(leaves | idle)))) {
             if (in_leaf) {
                 live = wide_leaf<COUNT, SHAPES>(R, T, any_hit, tests);
-                // a leaf that shortened the ray: the node's other boxes are tested again
-                if (live && R.k == R.kend && (R.pmask == 0 || R.best_t == R.t_leaf))
-                    live = wide_advance(R, T, B, qi, err, s_stack);
+                if (live && R.k == R.kend) {
+                    if (R.pmask == 0 || R.best_t == R.t_leaf)
+                        live = wide_advance(R, T, B, qi, err, s_stack);
+                    else if (COUNT)
+                        --visits;  // the leaf shortened the ray: the same node's boxes are tested again
+                }
                 if (!live) wide_ray_finish(R, prim_out, t_out, bary_out);
             }
         } else if (live && !in_leaf) {
