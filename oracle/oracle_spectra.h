@@ -377,10 +377,15 @@ class Table {
     // d(c0, c1, c2)/d(r, g, b) of lookup(): J[q][k] = dc_q / drgb_k, from the
     // derivative of the trilinear interpolation and of the cell coordinates
     // x = rgb[(m+1)%3] (res-1) / z, y = rgb[(m+2)%3] (res-1) / z, z = rgb[m].
-    // Grey inputs take the general branch (the closed form holds only on the diagonal).
+    // Grey inputs take the general branch (the closed form holds only on the diagonal);
+    // black has no cell there: its derivative is taken as zero.
     void jacobian(const float rgb[3], double J[3][3]) {
         int mc = (rgb[0] > rgb[1]) ? ((rgb[0] > rgb[2]) ? 0 : 2) : ((rgb[1] > rgb[2]) ? 1 : 2);
         double z = rgb[mc];
+        if (!(z > 0)) {
+            for (int q = 0; q < 9; ++q) J[q / 3][q % 3] = 0;
+            return;
+        }
         double x = double(rgb[(mc + 1) % 3] * (kRes - 1)) / z;
         double y = double(rgb[(mc + 2) % 3] * (kRes - 1)) / z;
         int xi = std::min((int)x, kRes - 2), yi = std::min((int)y, kRes - 2);

@@ -144,6 +144,43 @@ def test_device_error_leaves_the_outputs_alone(tmp_path):
     fake_hip.isolated(__file__, "device_error", tmp_path)
 
 
+def missing_columns():
+    """The four columns that grey albedos read, in the table of each albedo_gradient launch."""
+    seen = []
+
+    def launch(kernel, blocks, threads, captured, args):
+        if "albedo_gradient" in kernel:
+            cols = np.ctypeslib.as_array((ctypes.c_float * (3 * 64 * 64 * 64 * 3)).from_address(fake_hip.pointer(args, 3)))
+            grey = cols.reshape(3, 64, 64, 64, 3)[2, 62:, 62:].copy()  # [component][y][x][z][coefficient]
+            seen.append(grey)
+            if np.isnan(grey).any():
+                fake_hip.poke_u32(fake_hip.pointer(args, 7), 1)
+
+    fake_hip.install(launch)
+    import pbrtm
+
+    with pbrtm.Context(0) as ctx:
+        sc = room()
+        scene = ctx.scene(sc)
+        rc, _, d_albedo = grad(ctx, scene, len(sc["albedo"]))
+        assert rc == pbrtm.OK and (d_albedo != SENTINEL).all()
+        assert len(seen) == 2 and np.isnan(seen[0]).all() and np.isfinite(seen[1]).all()
+        # a node of the table: column x = y = 62, z = smoothstep(smoothstep(40 / 63))
+        x = 40 / 63
+        x = x * x * (3 - 2 * x)
+        z = x * x * (3 - 2 * x)
+        want = pbrtm.rgb_to_sigmoid(np.array([z * 62 / 63, z * 62 / 63, z], np.float32))
+        assert np.allclose(seen[1][0, 0, 40], want, rtol=1e-4)
+        rc, _, _ = grad(ctx, scene, len(sc["albedo"]))  # nothing is missing any more
+        assert rc == pbrtm.OK and len(seen) == 3
+        scene.free()
+
+
+@fake_hip.needs_compiler
+def test_missing_columns_are_computed_and_uploaded(tmp_path):
+    fake_hip.isolated(__file__, "missing_columns", tmp_path)
+
+
 @fake_hip.needs_compiler
 def test_columns_that_stay_missing_are_an_error(tmp_path):
     """Never gradients of NaN columns."""
