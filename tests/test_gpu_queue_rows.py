@@ -1,6 +1,9 @@
 """Ray queues at the edges of the traversal's rows against the binary traversal: one ray,
-row lengths that change (multiples of the waves the rows are spread over), the first
-queues with full rows, more rays than one row of every wave, inactive rays in between."""
+row lengths that change (multiples of the 1024 waves the rows are spread over), the first
+queues with full rows, more rays than one row of every wave, inactive rays in between. On
+256 compute units with 6 workgroups of 4 waves, one row of every wave is 393,216 rays; with
+four of them or more a wave is dealt a second row before it asks for others, which takes
+1,572,864 active rays: the last size has about 1,967,000."""
 import numpy as np
 import pytest
 
@@ -9,7 +12,7 @@ import pbrtm
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 1023, 1024, 1025, 2049, 65535, 65537, 400_003, 1_200_001])
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 1023, 1024, 1025, 2049, 65535, 65537, 400_003, 1_200_001, 2_458_765])
 def test_row_edges(ctx, n):
     print(f"{n} rays", flush=True)
     bvh = ctx.build(pbrtm.gen_soup(5000, seed=31, mu=-3.0))

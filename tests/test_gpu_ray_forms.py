@@ -110,6 +110,31 @@ def test_ray_forms(ctx, scene, form):
     bvh.free()
 
 
+@pytest.mark.parametrize("form", ["axis", "tiny", "far", "none"])
+def test_ray_forms_noalloc(ctx, form):
+    """The same rays through the entry point without allocation."""
+    from test_zz_no_alloc import DeviceArray
+
+    tri = SCENES["grid"]()
+    bvh = ctx.build(tri)
+    n = 4001
+    rays = _rays(form, tri, n, np.random.default_rng(len(form)))
+    print(f"noalloc {form}", flush=True)
+    dev = DeviceArray(rays.shape, np.float32, rays)
+    out = [DeviceArray((n,), np.uint32), DeviceArray((n,), np.float32), DeviceArray((n, 3), np.float32)]
+    for any_hit in (False, True):
+        bvh.intersect_noalloc(dev, *out, any_hit=any_hit)
+        prim, t, bary = (a.numpy() for a in out)
+        op, ot, ob = bvh.intersect(rays, any_hit=any_hit, binary=True)
+        assert np.array_equal(prim, op)
+        if not any_hit:
+            hit = op != pbrtm.NO_HIT
+            assert _same(t[hit], ot[hit]) and _same(bary[hit], ob[hit])
+    for a in (dev, *out):
+        a.free()
+    bvh.free()
+
+
 def test_short_directions_take_as_long_as_others(ctx):
     """Rays on both sides of the range of the conservative box test (directions shorter than
     2^-20 take the reference's own test): a queue of them takes at most twice the time."""
