@@ -173,7 +173,7 @@ def render_roofline(b, runs):
         stages[k] = {"bytes": int(b[k]), "ms": round(t, 2), "gbs": round(gbs, 1),
                      "frac": round(gbs / HBM_PEAK_GBS, 4)}
     gbs = total / (ms * 1e-3) / 1e9
-    return {"kernel": "whole render (trace_wide_kernel, shade_kernel, compaction, film)", "bound": "hbm",
+    return {"kernel": "whole render (trace_wide_kernel, shade_kernel, film)", "bound": "hbm",
             "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(gbs / HBM_PEAK_GBS, 4),
             "traffic": None, "bytes_per_render": int(total), "stages": stages,
             "algorithmic_bytes": f"per closest ray: {2 * PATH_STATE_BYTES} B path state + {PATH_HIT_BYTES} B hit "
@@ -222,8 +222,6 @@ def pathtracer(args, ctx, pbrtm, host):
         "stages_ms": {k: round(float(np.mean([r[k] for r in runs])), 2)
                       for k in ("ms_trace", "ms_shadow", "ms_shade", "ms_film")},
         "rounds": last["rounds"], "rays": last["rays"], "shadow_rays": last["shadow_rays"],
-        "ray_order": {"closest_sorted": bool(last["ray_order"] & 1), "shadow_sorted": bool(last["ray_order"] & 2)},
-        "grid_quarters": last["grid_quarters"],
         "mrays_per_s": round((last["rays"] + last["shadow_rays"]) / (ms * 1e3), 1),
         "pool_4m": {"value": round(W * H * spp / (ms_big * 1e3), 2), "ms_per_image": round(ms_big, 2),
                     "note": "2^22 path slots instead of the reference's 2^21: each pixel sums the same samples in another order"},

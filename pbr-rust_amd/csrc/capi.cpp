@@ -155,7 +155,8 @@ double event_ms(hipEvent_t a, hipEvent_t b) {
 
 // Scratch of pbrtm_bvh_intersect_noalloc: a file-scope device array, so that the
 // entry point allocates nothing. Layout: a 256-byte header (word 0: device
-// error bits, word 1: ray queue length; cleared by a kernel on every call),
+// error bits, word 1: ray queue length, word 3: rows handed out; cleared by a kernel on
+// every call),
 // the ray queue (one word per ray), then the traversal's stack spill area.
 // Each device holds its own copy for the life of the process; every call on a
 // device shares it, so calls that overlap on one device race.
@@ -578,7 +579,7 @@ int pbrtm_bvh_intersect_noalloc(pbrtm_bvh *bvh, const float *rays, uint64_t n, i
     CK(ctx, hipSetDevice(ctx->device), "hipSetDevice");
     uint8_t *base = noalloc_scratch_of(ctx->device);
     if (!base) return fail(ctx, PBRTM_ERR_HIP, "pbrtm_bvh_intersect_noalloc: scratch symbol address unavailable");
-    uint32_t *words = reinterpret_cast<uint32_t *>(base);  // [0] device error bits, [1] queue length
+    uint32_t *words = reinterpret_cast<uint32_t *>(base);  // [0] device error bits, [1] queue length, [3] its head
     uint32_t *queue = reinterpret_cast<uint32_t *>(base + kNoAllocHeader);
     uint2 *spill = reinterpret_cast<uint2 *>(base + kNoAllocHeader + kNoAllocMaxRays * sizeof(uint32_t));
     zero_words_kernel<<<1, 64, 0, ctx->stream>>>(words, kNoAllocHeader / sizeof(uint32_t));

@@ -1198,8 +1198,9 @@ __global__ __launch_bounds__(256) void top_acc_reset_kernel(TopLevel TL, uint32_
 // hlbvh.cu:711-741) and a stable partition into the other record buffer, 64
 // positions a row, by one wave, which goes on with the smaller child from its own
 // stack in LDS and offers the larger one to the workgroup's other waves. A wave
-// without a node takes an offered one; nothing else is shared, and no barrier is
-// passed, within a list node. The deep levels of the level path (thousands of small
+// without a node takes an offered one. The waves share the list node's bounds first, with a
+// barrier on either side; from there to its end they pass none and share only the offers
+// and the count of nodes left to split. The deep levels of the level path (thousands of small
 // nodes, a few launches each) become this one launch. It is bound by the chain of
 // splits under one list node, the first of them one wave's: with one wave per list node
 // 1M triangles took 364 us, now 277 (269 with 8 waves, slower at 10M), a build of 20k

@@ -38,10 +38,9 @@ constexpr uint32_t kIdle = 0xFFFFFFFFu;
 // 60 % of small renders and batches; ordering the rays by octant and cell saved 2-5 %
 // of the traversal and cost more than that.)
 // counters[] layout (u32 words): per parity a block of kCntBlock words, [kCntLive,
-// kCntShadow] the lengths of the live list and the shadow queue (one u64 for the
-// appends), [kCntRays] the closest-hit queue's where it is a queue of its own, and each
-// length's traversal counter kQueueHead words after it; kCntAccRays: u64 accumulators
-// of a batched render.
+// kCntShadow] the lengths of the live list and the shadow queue, [kCntRays] the
+// closest-hit queue's where it is a queue of its own, and each length's traversal counter
+// kQueueHead words after it; kCntAccRays: u64 accumulators of a batched render.
 constexpr int kCntNextId = 0, kCntRound = 1, kCntDone = 2, kCntAccRays = 4;
 constexpr int kCntBlock = 8, kCntLive = 0, kCntShadow = 1, kCntRays = 4;
 constexpr int kCntWords = 32;

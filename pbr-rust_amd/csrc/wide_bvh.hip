@@ -444,14 +444,14 @@ __device__ __forceinline__ WideTree tree_of(const WideTrace *B) {
     return WideTree{B->nodes, B->order, B->num_nodes, B};
 }
 
-// The exact box of the binary leaf at positions [first, first + cnt) (the union of
-// its primitives' boxes: the leaf-ordered vertices, or an analytic primitive's
-// box stored as the corners lo, hi, lo) against the ray with t_max (bounds3.h:146-195).
 __device__ __forceinline__ f3 ray_dir(const WideRay &R) {
     const float4 r1 = R.rays[2 * size_t(R.id) + 1];
     return {r1.x, r1.y, r1.z};
 }
 
+// The exact box of the binary leaf at positions [first, first + cnt) (the union of
+// its primitives' boxes: the leaf-ordered vertices, or an analytic primitive's
+// box stored as the corners lo, hi, lo) against the ray with t_max (bounds3.h:146-195).
 __device__ __forceinline__ bool leaf_box_hit(const WideTree &T, uint32_t first, uint32_t cnt,
                                                         const WideRay &R, float t_max) {
     Box b = box_empty();
@@ -771,11 +771,13 @@ __device__ __forceinline__ void add_counts(unsigned long long *counts, uint32_t 
 constexpr uint32_t kRefill = 16;
 constexpr uint32_t kWideWaves = kWideBlock / kWave;
 // Slots of a row: a queue with less than kWave rays for each of kSpread waves (one per
-// SIMD) is spread over them in shorter rows. A short launch lasts as long as its
-// longest ray, step by step (1-2 us each), and lanes of a wave wait for each other's
-// node and leaf steps. With twice, four or eight times the waves the steps themselves
-// slow down. 999 rays into 100k triangles 165 -> 140 us, 14,400 into 1M 385 -> 255 us,
-// 153,600 into 1M 507 -> 504 us; 8192 waves 283 and 633 us.
+// SIMD of 256 compute units, where it was measured; a constant, since the host's grid and
+// the device's rows both follow from it) is spread over them in shorter rows. A short
+// launch lasts as long as its longest ray, step by step (1-2 us each), and lanes of a wave
+// wait for each other's node and leaf steps; with eight times the waves the steps
+// themselves slow down. Calls of 999 camera rays into 100k triangles, 14,400 and 153,600
+// into 1M, with rows of 64: 174, 455 and 540 us; now 141, 386 and 535; spread over 8192
+// waves 138, 410 and 706.
 constexpr uint32_t kSpread = 1024;
 __host__ __device__ constexpr uint32_t wide_row(uint32_t n) {
     const uint32_t r = n / kSpread + (n % kSpread != 0 ? 1u : 0u);
@@ -969,8 +971,8 @@ hipError_t collapse_wide(const BNode *bnodes, uint32_t n, WideBvh &out, DevBuf &
 }
 
 // Workgroups of a persistent traversal kernel: as many as are resident on the
-// device at once (quarters/4 of them when quarters is 1..3), at most one per 256
-// rays. The resident count is computed once per (kernel, device).
+// device at once (quarters/4 of them when quarters is 1..3), at most one per kWideWaves
+// rows of the longest queue (wide_row). The resident count is computed once per (kernel, device).
 template <typename Kernel>
 static uint32_t persistent_grid(Kernel kernel, uint32_t n, uint32_t quarters) {
     struct Entry {
