@@ -1697,7 +1697,7 @@ hipError_t render(const SceneDev &S, const WideTrace &W0, uint32_t spp, uint32_t
         return hipSuccess;
     };
     PT_CK(enqueue(0));
-    uint32_t r = 0;
+    uint32_t r = 0, last_rays = 0;
     for (;;) {
         PT_CK(enqueue(r + 1));
         hipEvent_t *E = ev + 3 + 5 * (r & 1);
@@ -1711,7 +1711,8 @@ hipError_t render(const SceneDev &S, const WideTrace &W0, uint32_t spp, uint32_t
         t_trace += a;
         t_shadow += b;
         t_shade += c;
-        rs.rays += cnt[separate_rays ? kCntRays : kCntLive];
+        last_rays = cnt[separate_rays ? kCntRays : kCntLive];
+        rs.rays += last_rays;
         rs.shadow_rays += cnt[kCntShadow];
         ++r;
         if (r > 100000) return hipErrorUnknown;
@@ -1737,7 +1738,10 @@ hipError_t render(const SceneDev &S, const WideTrace &W0, uint32_t spp, uint32_t
     rs.ms_shadow = t_shadow;
     rs.ms_shade = t_shade;
     rs.ms_film = tf;
-    rs.rounds = P.round;
+    // The megakernel integrators' count goes up to the first round without a closest-hit
+    // ray: that is the last one with live paths if those wait for their shadow rays alone,
+    // else the empty round after it.
+    rs.rounds = P.round + (integrator != kIntPath && last_rays != 0 ? 1 : 0);
     rs.paths = total;
     if (stats) *stats = rs;
     return hipSuccess;

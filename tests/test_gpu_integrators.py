@@ -115,3 +115,25 @@ def test_cli_integrator_option(tmp_path):
     img = np.asarray(Image.open(out).convert("RGBA"))
     orgb, _, _ = O.render_megakernel(scenes.cornell34(64, 64), "ambientocclusion", threads=16)
     assert np.array_equal(img, O.srgb8(orgb))
+
+
+@pytest.mark.parametrize("scene,integrator,spp,depth,pool,rounds", [
+    ("cornell", "path", 4, 5, 100, 61), ("cornell", "megakernelpath", 1, 0, 0, 2),
+    ("cornell", "megakernelpath", 4, 5, 100, 57), ("cornell", "megakernelpath", 4, 200, 50, 140),
+    ("cornell", "ambientocclusion", 4, 5, 100, 28), ("cornell", "ambientocclusion", 4, 200, 50, 56),
+    ("cornell", "surfacenormal", 1, 0, 0, 2), ("grid", "surfacenormal", 1, 0, 100, 6),
+    ("grid", "ambientocclusion", 4, 1, 100, 20)])
+def test_round_counts(ctx, scene, integrator, spp, depth, pool, rounds):
+    """stats.rounds: for the wavefront integrator the rounds with live paths, for the megakernel
+    integrators the rounds up to the first one without a closest-hit ray, whether the last paths
+    end on a miss or wait for a shadow ray in it (values of renders recorded when each round
+    scanned the pool for its rays)."""
+    from pbrtm.scenes import cornell34, sphere_grid
+
+    s = ctx.scene(cornell34(23, 17) if scene == "cornell" else sphere_grid(width=24, height=18, n=3))
+    try:
+        _, _, st = s.render(spp=spp, max_depth=depth, pool_size=pool, integrator=integrator)
+    finally:
+        s.free()
+    log(f"{scene} {integrator} spp {spp} depth {depth} pool {pool}: {st['rounds']} rounds")
+    assert st["rounds"] == rounds
