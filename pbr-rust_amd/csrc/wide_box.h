@@ -1,0 +1,111 @@
+// The quantized boxes of the 8-wide tree and the conservative test of a ray against
+// them: plain FP32 / FP64 arithmetic that the collapse and the traversal share, and that
+// a host program can run against the reference's slab test (box_hit).
+#pragma once
+
+#include "pbrtm_geometry.h"
+
+namespace pbrtm {
+
+// 2^e for e in [-126, 127], exactly.
+PBRTM_HD float pow2f(int e) { return __builtin_bit_cast(float, uint32_t(e + 127) << 23); }
+
+// Exponent of a node's step along an axis of extent ext: the smallest power of two with
+// ext / step <= 253.
+PBRTM_HD int box_step_exp(float ext) {
+    int e = -126;
+    if (ext > 0.f) {
+        int e2;
+        frexpf(ext / 253.0f, &e2);
+        e = e2;
+        if (ldexpf(1.0f, e2 - 1) * 253.0f >= ext) e = e2 - 1;
+    }
+    return e < -126 ? -126 : (e > 126 ? 126 : e);
+}
+
+// Quantized lower / upper plane of a coordinate in a node of origin org and step 2^e
+// (inv_step = 2^-e, so the divisions are exact products). The plane lies outside the
+// coordinate as a real number, org + q * step, not only after rounding, so that a
+// traversal which does not round planes to FP32 needs no allowance for it: far from the
+// world's origin such an allowance outgrows the boxes. The comparison in FP64 holds that
+// sum exactly, or, where 255 steps are more than the origin, to 2^-52 of them.
+PBRTM_HD int box_quant_lo(float v, float org, float step, float inv_step) {
+    int q = int(fminf(255.f, fmaxf(0.f, floorf((v - org) * inv_step))));
+    while (q > 0 && double(org) + double(q) * double(step) > double(v)) --q;
+    return q;
+}
+PBRTM_HD int box_quant_hi(float v, float org, float step, float inv_step) {
+    int q = int(fminf(255.f, fmaxf(0.f, ceilf((v - org) * inv_step))));
+    while (q < 255 && double(org) + double(q) * double(step) < double(v)) ++q;
+    return q;
+}
+
+// Conservative slab test of the quantized boxes. In a node, the distance to the
+// plane with byte q is q * A + B, A = step * inv and B = (org - o) * inv: one
+// conversion and one fmaf per plane instead of decoding the plane, subtracting the
+// origin and multiplying. It must never miss a box whose exact box the reference's
+// test (box_hit) enters, so the near distances are lowered and the far ones raised
+// by err = 16u (|B| + 255 |A|), u = 2^-24. In units of u (|B| + 255 |A|), which bounds
+// the distance to every plane of the node, what separates the two is at most 13.01:
+//   - box_hit's difference and product: 2.01, and its widening of the far distances,
+//     2 gamma(3) + u: 7.01 (the near distances are not widened);
+//   - the roundings of B (2.01), of B -+ err (1.01) and of the fmaf (1.01);
+//   - the quantized planes contain the exact ones as real numbers and A is exact (a power
+//     of two times inv): nothing. In particular nothing here grows with the distance of
+//     the scene from the world's origin.
+// A component of d that is zero or tiny has a reciprocal that is infinite or very large:
+// it is clamped to 2^32 times the least |inv| of the ray, and err of that axis raised by
+// four times the distance at which the axis of the least |inv| has left the tree's box.
+// That covers every distance that the other axes can hold against it (a plane that
+// touches o has t = 0 or NaN in the reference), and moves its planes outwards by 2^-30
+// of the size of the tree and the ray's distance from it, whatever their scale.
+// Rays without a direction, with NaNs or far outside any scene (BoxRay::generic) take
+// the reference's own test on the decoded planes.
+constexpr float kBoxErr = 16.0f * 5.9604644775390625e-08f;
+
+// A ray's reciprocal direction for the box tests (clamped; as it is if generic) and its
+// clamped axes' constant error term (else 0).
+struct BoxRay {
+    f3 inv, err;
+    bool generic;
+};
+// size(): the largest distance along an axis from o to the far side of the tree's box;
+// asked for rays with a clamped axis only.
+template <typename Size>
+PBRTM_HD BoxRay box_ray(f3 o, f3 d, f3 inv, Size size) {
+    const f3 a = abs3(inv);
+    const float least = fminf(fminf(a.x, a.y), a.z), cap = least * 0x1p32f;
+    BoxRay r{inv, {0.f, 0.f, 0.f}, false};
+    const float span = fabsf(o.x) + fabsf(o.y) + fabsf(o.z) + fabsf(d.x) + fabsf(d.y) + fabsf(d.z);
+    if (!(least <= 0x1p20f && span <= 0x1p60f)) {
+        r.generic = true;
+    } else if (!(fmaxf(fmaxf(a.x, a.y), a.z) <= cap)) {
+        const float err = 4.0f * size() * least;
+        if (!(a.x <= cap)) r.inv.x = copysignf(cap, inv.x), r.err.x = err;
+        if (!(a.y <= cap)) r.inv.y = copysignf(cap, inv.y), r.err.y = err;
+        if (!(a.z <= cap)) r.inv.z = copysignf(cap, inv.z), r.err.z = err;
+    }
+    return r;
+}
+
+// One axis of a node for a ray: near distance fmaf(q, a, bn), far distance fmaf(q, a, bf).
+struct BoxAxis {
+    float a, bn, bf;
+};
+PBRTM_HD BoxAxis box_axis(float org, float step, float o, float inv, float ray_err) {
+    const float a = step * inv, b = (org - o) * inv;
+    const float err = fmaf(fabsf(a), 255.0f * kBoxErr, fmaf(fabsf(b), kBoxErr, ray_err));
+    return {a, b - err, b + err};
+}
+// Negative when the box of near bytes qn and far bytes qf is missed up to t_max.
+PBRTM_HD float box_gap(const BoxAxis ax[3], const uint32_t qn[3], const uint32_t qf[3], float t_max) {
+    const float lo = fmaxf(fmaxf(fmaxf(fmaf(float(qn[0]), ax[0].a, ax[0].bn), fmaf(float(qn[1]), ax[1].a, ax[1].bn)),
+                                 fmaf(float(qn[2]), ax[2].a, ax[2].bn)),
+                           0.0f);
+    const float hi = fminf(fminf(fminf(fmaf(float(qf[0]), ax[0].a, ax[0].bf), fmaf(float(qf[1]), ax[1].a, ax[1].bf)),
+                                 fmaf(float(qf[2]), ax[2].a, ax[2].bf)),
+                           t_max);
+    return hi - lo;
+}
+
+}  // namespace pbrtm

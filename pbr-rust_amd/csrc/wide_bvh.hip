@@ -23,7 +23,7 @@
 // boxes) passes the slab test with the t at which the leaf was entered, exactly
 // as the binary traversal tests it. Each visit costs one 128-byte node instead
 // of up to seven dependent 32-byte fetches.
-#include "pbrtm_geometry.h"
+#include "wide_box.h"
 #include "wave_ops.h"
 #include "pbrtm_shapes.h"
 #include "wide_bvh.h"
@@ -38,28 +38,16 @@ struct Job {
     uint32_t bnode, wnode, depth, prims;  // prims: primitives under the binary node
 };
 
-// 2^e for e in [-126, 127], exactly.
-__device__ __forceinline__ float pow2f(int e) { return __uint_as_float(uint32_t(e + 127) << 23); }
-
 // Encodes n (<= 8) child boxes into w's origin, exponents and quantized planes;
 // unused slots get the inverted box (lo 255, hi 0). ulo / uhi: the union of the
-// child boxes (the collapsed binary node's own box); box(s, lo, hi) fetches child
-// s. Steps are powers of two, so the divisions below are exact products.
+// child boxes (the collapsed binary node's own box); box(s, lo, hi) fetches child s.
 template <typename BoxOf>
 __device__ __forceinline__ void encode_node(WNode *w, const float ulo[3], const float uhi[3], BoxOf box, int n) {
     float sc[3], inv[3];
     uint32_t ex = 0u;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-        const float ext = uhi[a] - ulo[a];
-        int e = -126;
-        if (ext > 0.f) {  // smallest power-of-two step with ext / step <= 253
-            int e2;
-            frexpf(ext / 253.0f, &e2);
-            e = e2;
-            if (ldexpf(1.0f, e2 - 1) * 253.0f >= ext) e = e2 - 1;
-        }
-        e = max(-126, min(126, e));
+        const int e = box_step_exp(uhi[a] - ulo[a]);
         sc[a] = pow2f(e);
         inv[a] = pow2f(-e);
         ex |= (uint32_t(e) & 0xFFu) << (8 * a);
@@ -73,10 +61,8 @@ __device__ __forceinline__ void encode_node(WNode *w, const float ulo[3], const 
         for (int a = 0; a < 3; ++a) {
             int ql = 255, qh = 0;
             if (s < n) {
-                ql = int(fminf(255.f, fmaxf(0.f, floorf((l[a] - ulo[a]) * inv[a]))));
-                while (ql > 0 && fmaf(float(ql), sc[a], ulo[a]) > l[a]) --ql;
-                qh = int(fminf(255.f, fmaxf(0.f, ceilf((h[a] - ulo[a]) * inv[a]))));
-                while (qh < 255 && fmaf(float(qh), sc[a], ulo[a]) < h[a]) ++qh;
+                ql = box_quant_lo(l[a], ulo[a], sc[a], inv[a]);
+                qh = box_quant_hi(h[a], ulo[a], sc[a], inv[a]);
             }
             plo[a] |= uint64_t(ql) << (8 * s);
             phi[a] |= uint64_t(qh) << (8 * s);
@@ -414,9 +400,9 @@ __global__ __launch_bounds__(kCompactBlock) void compact_rays_kernel(const float
 }
 
 // Traversal state of one ray. binv / berr: the box tests' reciprocal direction
-// (clamped, finite; unclamped for a ray that starts as kRayGeneric) and per-axis constant
-// error term (wide_ray_start). Instead of the direction it holds the triangle test's
-// shear; ray_dir fetches the direction again where an unusual case needs it.
+// (clamped, finite; unclamped for a ray that starts as kRayGeneric) and a clamped axis'
+// constant error term, else 0 (box_ray). Instead of the direction it holds the triangle
+// test's shear; ray_dir fetches the direction again where an unusual case needs it.
 struct WideRay {
     f3 o, binv, berr;
     RayShear sh;
@@ -466,53 +452,21 @@ __device__ __forceinline__ bool leaf_box_hit(const WideTree &T, uint32_t first, 
     return box_hit(lo, hi, R.o, inv, neg, t_max);
 }
 
-// Conservative slab test of the quantized boxes. In a node, the distance to the
-// plane with byte q is q * A + B, A = step * inv and B = (org - o) * inv: one
-// conversion and one fmaf per plane instead of decoding the plane, subtracting the
-// origin and multiplying. It must never miss a box whose exact box the reference's
-// test (box_hit) enters, so the near distances are lowered and the far ones raised
-// by err = 64u (|B| + 255 |A|) + 8u |o inv|, u = 2^-24, which is more than twice the
-// sum of what separates the two in either direction:
-//   - the decoded plane fmaf(q, step, org), which bounds the exact one, is within
-//     u |plane| of org + q step: u |plane inv| <= 1.01 u (|B| + 255 |A| + |o inv|);
-//   - box_hit's difference and product: 2.01 u |plane - o| |inv| <= 2.1 u (|B| + 255 |A|);
-//   - the roundings of B (2.01 u |B|), of the fmaf and of B -+ err (2.1 u each);
-//   - box_hit's widening of the far distances, 2 gamma(3) + u <= 7.1 u (|B| + 255 |A|).
-// A is exact (a power of two times inv). A component of d that is zero or tiny has a
-// reciprocal that is infinite or very large: it is clamped to 2^100 times the least
-// |inv| of the ray, and err of that axis raised by 2^70 times it, which moves its
-// planes outwards by 2^-30 and covers every distance t < 2^70 least |inv| that the
-// other axes can hold against it (a plane that touches o has t = 0 or NaN in the
-// reference). Rays without a direction, with NaNs or far outside any scene take the
-// reference's own test on the decoded planes (kRayGeneric, wide_box_generic). The
-// hits do not depend on any of this: a triangle hit counts only if its leaf's exact
-// box passes box_hit (wide_leaf).
 // The traversal is bound by instruction issue (VALU busy 62-76 %), and decoding each
-// plane to test it with box_hit's operations took about twice the instructions:
-// 1080p camera rays into 10M triangles 1995 -> 1780 us, their bounce 1490 -> 1327 us,
-// 919,601 shadow rays into 1M triangles 1080 -> 909 us a call.
-constexpr float kBoxErrAB = 64.0f * 5.9604644775390625e-08f;
-constexpr float kBoxErrO = 8.0f * 5.9604644775390625e-08f;
-struct BoxAxis {
-    float a, bn, bf;  // near distance fmaf(q, a, bn), far distance fmaf(q, a, bf)
-};
-__device__ __forceinline__ BoxAxis box_axis(float org, float step, float o, float inv, float berr) {
-    const float a = step * inv, b = (org - o) * inv;
-    const float err = fmaf(fabsf(a), 255.0f * kBoxErrAB, fmaf(fabsf(b), kBoxErrAB, berr));
-    return {a, b - err, b + err};
-}
-__device__ __forceinline__ float box_clamp_inv(float inv, float least) {
-    const float cap = least * 0x1p100f;
-    return fabsf(inv) <= cap ? inv : copysignf(cap, inv);
-}
+// plane to test it with box_hit's operations took about twice the instructions of the
+// conservative test (wide_box.h): 1080p camera rays into 10M triangles 1995 -> 1780 us,
+// their bounce 1490 -> 1327 us, 919,601 shadow rays into 1M triangles 1080 -> 909 us a call.
+// A ray along an axis reads the root's node to know the tree's size; with a constant in its
+// place 524,288 of them take 0.65 ms through a scene of extent 1 (300k triangles) and 1.9
+// seconds through one of extent 2^40 or 2^-30, now 0.64 ms through all of them. With an
+// allowance for rounding planes to FP32, as many random rays through that scene 4,096,
+// 16,384 and 65,536 times its extent from the world's origin took 1.12, 2.36 and 13.9 ms,
+// now 0.85, 0.81 and 0.80.
 constexpr uint32_t kRayGeneric = 8u;  // WideRay::oct, above the octant's three bits
-__device__ __forceinline__ float box_err_const(float o, float inv, float binv, float least) {
-    const float e = kBoxErrO * fabsf(o * binv);
-    return inv == binv ? e : e + least * 0x1p70f;
-}
 
 // Loads ray i; true when it has an interval to trace (t_max > 0).
-__device__ __forceinline__ bool wide_ray_start(WideRay &R, const float4 *__restrict__ rays, uint32_t i) {
+__device__ __forceinline__ bool wide_ray_start(WideRay &R, const float4 *__restrict__ rays, uint32_t i,
+                                               const WideTree &T) {
     const float4 r0 = rays[2 * size_t(i)], r1 = rays[2 * size_t(i) + 1];
     R.o = {r0.x, r0.y, r0.z};
     const f3 d = {r1.x, r1.y, r1.z};
@@ -523,15 +477,15 @@ __device__ __forceinline__ bool wide_ray_start(WideRay &R, const float4 *__restr
     R.hit = TriHit{0.f, 0.f, 0.f, 0.f};
     const f3 inv = {1.0f / d.x, 1.0f / d.y, 1.0f / d.z};
     R.oct = uint32_t(inv.x < 0.f) | (uint32_t(inv.y < 0.f) << 1) | (uint32_t(inv.z < 0.f) << 2);
-    const float least = fminf(fminf(fabsf(inv.x), fabsf(inv.y)), fabsf(inv.z));
-    R.binv = {box_clamp_inv(inv.x, least), box_clamp_inv(inv.y, least), box_clamp_inv(inv.z, least)};
-    R.berr = {box_err_const(R.o.x, inv.x, R.binv.x, least), box_err_const(R.o.y, inv.y, R.binv.y, least),
-              box_err_const(R.o.z, inv.z, R.binv.z, least)};
-    const float span = fabsf(R.o.x) + fabsf(R.o.y) + fabsf(R.o.z) + fabsf(d.x) + fabsf(d.y) + fabsf(d.z);
-    if (!(least <= 0x1p20f && span <= 0x1p60f)) {
-        R.oct |= kRayGeneric;
-        R.binv = inv;
-    }
+    const BoxRay box = box_ray(R.o, d, inv, [&] {
+        const uint4 hd = *reinterpret_cast<const uint4 *>(T.nodes);  // the root's origin and steps
+        return fmaxf(fmaxf(fabsf(__uint_as_float(hd.x) - R.o.x) + 255.f * pow2f(int(int8_t(hd.w & 0xFFu))),
+                           fabsf(__uint_as_float(hd.y) - R.o.y) + 255.f * pow2f(int(int8_t((hd.w >> 8) & 0xFFu)))),
+                     fabsf(__uint_as_float(hd.z) - R.o.z) + 255.f * pow2f(int(int8_t((hd.w >> 16) & 0xFFu))));
+    });
+    R.binv = box.inv;
+    R.berr = box.err;
+    if (box.generic) R.oct |= kRayGeneric;
     R.node = 0;
     R.pmask = 0xFFu;
     R.sp = 0;
@@ -551,8 +505,8 @@ __device__ __forceinline__ void wide_ray_finish(const WideRay &R, uint32_t *__re
     }
 }
 
-// Hit mask of a node's slots for a ray outside box_axis' range (WideRay::binv is its
-// unclamped reciprocal): each slot's decoded planes through the reference's slab test,
+// Hit mask of a node's slots for a ray outside the conservative test's range (WideRay::binv
+// is its unclamped reciprocal): each slot's decoded planes through the reference's slab test,
 // near and far already chosen by the direction's signs. Bound by instruction issue like
 // the test it stands in for, so it decodes the words at hand, all slots in line; slot by
 // slot (the scheduling barrier), because all decodes at once spill registers in every
@@ -679,15 +633,13 @@ __device__ __forceinline__ bool wide_node(WideRay &R, const WideTree &T, uint32_
         uint32_t miss = 0;
 #pragma unroll
         for (int s = kWide - 1; s >= 0; --s) {
-            float tn[3], tf[3];
+            uint32_t qn[3], qf[3];
 #pragma unroll
             for (int a = 0; a < 3; ++a) {
-                tn[a] = fmaf(float((nw[a][s / 4] >> (8 * (s % 4))) & 0xFFu), ax[a].a, ax[a].bn);
-                tf[a] = fmaf(float((fw[a][s / 4] >> (8 * (s % 4))) & 0xFFu), ax[a].a, ax[a].bf);
+                qn[a] = (nw[a][s / 4] >> (8 * (s % 4))) & 0xFFu;
+                qf[a] = (fw[a][s / 4] >> (8 * (s % 4))) & 0xFFu;
             }
-            const float lo = fmaxf(fmaxf(fmaxf(tn[0], tn[1]), tn[2]), 0.0f);
-            const float hi = fminf(fminf(fminf(tf[0], tf[1]), tf[2]), R.best_t);
-            miss = __builtin_amdgcn_alignbit(miss, __float_as_uint(hi - lo), 31);
+            miss = __builtin_amdgcn_alignbit(miss, __float_as_uint(box_gap(ax, qn, qf, R.best_t)), 31);
         }
         hs = ~miss & 0xFFu;
     }
@@ -791,7 +743,7 @@ constexpr uint32_t kDealt = 5;
 // 1/3, 107.1 at 1/6; 1/2 slows short queues (16 mixed jobs +1 %); 1/8, 1/12 and a fixed
 // count of 8 lanes are slower still. Against testing every leaf where a lane met it: 1080p camera rays into 10M
 // triangles 1780 -> 1246 us, shadow rays into 1M 909 -> 701 us, 999 rays 209 -> 178 us
-// (and 96 -> 74 VGPRs, 6 waves per SIMD).
+// (and 96 -> 73 VGPRs, 6 waves per SIMD).
 constexpr uint32_t kLeafShare = 3;
 
 template <bool COUNT, bool MULTI, bool SHAPES>
@@ -832,7 +784,7 @@ __device__ __forceinline__ void trace_wide_persistent_body(const WideTrace &B, c
                     qi = next + pos;
                     const uint32_t i = queue[qi];
                     if (MULTI) T = tree_of(jw + ray_job[i >> job_shift]);
-                    live = wide_ray_start(R, rays, i);
+                    live = wide_ray_start(R, rays, i, T);
                     if (!live) wide_ray_finish(R, prim_out, t_out, bary_out);
                 }
             }
@@ -879,7 +831,7 @@ __device__ __forceinline__ void trace_wide_persistent_body(const WideTrace &B, c
 }
 
 // The occupancy floor of 5 waves per SIMD keeps the registers of the per-ray-tree and the
-// analytic instances within 96 without spills; the single-tree triangle instance needs 74
+// analytic instances within 96 without spills; the single-tree triangle instance needs 73
 // and runs at the 6 that the LDS stack (24 KiB per block) allows. Held to 6, the
 // per-ray-tree one spills four registers: 16 mixed jobs 5.46 -> 5.62 ms. A refill
 // waits for 16 idle lanes: the rays' start (two loads, reciprocals, shear) costs a step of

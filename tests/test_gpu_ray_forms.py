@@ -164,3 +164,26 @@ def test_short_directions_take_as_long_as_others(ctx):
     prim.free()
     bvh.free()
     assert took[2.0 ** -24] <= 2 * took[2.0 ** -18], took
+
+
+@pytest.mark.parametrize("form,scale,offset", [
+    ("axis", 2.0 ** -30, 0), ("axis", 2.0 ** 40, 0), ("axis", 1, 4096), ("short", 2.0 ** -30, 0),
+    ("short", 2.0 ** 40, 0), ("short", 1, 4096), ("short", 1, 16384)])
+def test_work_does_not_depend_on_the_scene_s_place(ctx, form, scale, offset):
+    """The same rays into the same triangles, scaled or moved: a ray visits as many nodes and
+    tests as many triangles. (In small and large scenes rays along an axis once entered every
+    box, far from the world's origin all rays the boxes around their own.)"""
+    base = pbrtm.gen_soup(100_000, seed=51, mu=-5.0)
+    counts = []
+    for s, o in ((1.0, 0.0), (scale, offset)):
+        tri = (base.astype(np.float64) * s + o).astype(np.float32)
+        bvh = ctx.build(tri)
+        rays = _rays(form, base, 2000, np.random.default_rng(52))
+        rays[:, 0:3] = (rays[:, 0:3].astype(np.float64) * s + o).astype(np.float32)
+        rays[:, 3] *= np.float32(s)
+        stats = np.zeros(3, np.uint64)
+        bvh.intersect(rays, stats=stats)
+        counts.append(stats[[0, 2]] / len(rays))
+        bvh.free()
+    print(f"{form} scale {scale} offset {offset}: visits and tests per ray {counts[0]} -> {counts[1]}", flush=True)
+    assert counts[1][0] <= 1.1 * counts[0][0] and counts[1][1] <= 1.3 * counts[0][1]
