@@ -154,14 +154,14 @@ double event_ms(hipEvent_t a, hipEvent_t b) {
 }
 
 // Scratch of pbrtm_bvh_intersect_noalloc: a file-scope device array, so that the
-// entry point allocates nothing. Layout: a 256-byte header (word 0: device
-// error bits, word 1: ray queue length, word 3: rows handed out; cleared by a kernel on
-// every call),
+// entry point allocates nothing. Layout: a 4096-byte header (word 0: device error bits,
+// word 1: ray queue length, from word 16: rows handed out; cleared by a kernel on every call),
 // the ray queue (one word per ray), then the traversal's stack spill area.
 // Each device holds its own copy for the life of the process; every call on a
 // device shares it, so calls that overlap on one device race.
 constexpr uint64_t kNoAllocMaxRays = 1ull << 22;
-constexpr uint64_t kNoAllocHeader = 256;
+constexpr uint64_t kNoAllocHeader = 4096;
+static_assert(kNoAllocHeader >= 64 + kHeadWords * 4);
 constexpr uint64_t kNoAllocSpillBytes = 16ull << 20;
 constexpr uint64_t kNoAllocBytes = kNoAllocHeader + kNoAllocMaxRays * 4 + kNoAllocSpillBytes;
 static __device__ __align__(256) uint8_t scratch[kNoAllocBytes];
@@ -520,8 +520,9 @@ int pbrtm_bvh_intersect(pbrtm_bvh *bvh, const float *rays, uint64_t n, int any_h
         d_t = t_out ? ctx->stage_b.as<float>() : nullptr;
         d_b = bary_out ? ctx->stage_c.as<float>() : nullptr;
     }
-    CK(ctx, ctx->dev_err.reserve(64), "alloc");
-    CK(ctx, hipMemsetAsync(ctx->dev_err.ptr, 0, 64, ctx->stream), "memset");
+    // word 0: device error bits, 1: queue length, 4 .. 9: counts, 16 on: rows handed out
+    CK(ctx, ctx->dev_err.reserve(64 + kHeadWords * 4), "alloc");
+    CK(ctx, hipMemsetAsync(ctx->dev_err.ptr, 0, 64 + kHeadWords * 4, ctx->stream), "memset");
     unsigned long long *d_counts = stats_out ? (unsigned long long *)(ctx->dev_err.as<uint8_t>() + 16) : nullptr;
     const bool binary = (flags & PBRTM_TRACE_BINARY) != 0;
     if (bvh->n == 0) {
@@ -551,7 +552,8 @@ int pbrtm_bvh_intersect(pbrtm_bvh *bvh, const float *rays, uint64_t n, int any_h
             CK(ctx, ctx->queue.reserve(size_t(n) * 4), "alloc ray queue");
             CK(ctx, trace_wide(W, (const float *)d_rays, uint32_t(n), any_hit, d_prim, d_t, d_b,
                                ctx->dev_err.as<uint32_t>(), d_counts, ctx->queue.as<uint32_t>(),
-                               ctx->dev_err.as<uint32_t>() + 1, ctx->stream), "trace");
+                               ctx->dev_err.as<uint32_t>() + 1, ctx->dev_err.as<uint32_t>() + 16, ctx->stream),
+               "trace");
         }
     }
     if (!dev) {
@@ -579,10 +581,10 @@ int pbrtm_bvh_intersect_noalloc(pbrtm_bvh *bvh, const float *rays, uint64_t n, i
     CK(ctx, hipSetDevice(ctx->device), "hipSetDevice");
     uint8_t *base = noalloc_scratch_of(ctx->device);
     if (!base) return fail(ctx, PBRTM_ERR_HIP, "pbrtm_bvh_intersect_noalloc: scratch symbol address unavailable");
-    uint32_t *words = reinterpret_cast<uint32_t *>(base);  // [0] device error bits, [1] queue length, [3] its head
+    uint32_t *words = reinterpret_cast<uint32_t *>(base);  // [0] device error bits, [1] queue length, [16] heads
     uint32_t *queue = reinterpret_cast<uint32_t *>(base + kNoAllocHeader);
     uint2 *spill = reinterpret_cast<uint2 *>(base + kNoAllocHeader + kNoAllocMaxRays * sizeof(uint32_t));
-    zero_words_kernel<<<1, 64, 0, ctx->stream>>>(words, kNoAllocHeader / sizeof(uint32_t));
+    zero_words_kernel<<<1, 256, 0, ctx->stream>>>(words, 16 + kHeadWords);
     CK(ctx, hipGetLastError(), "clear scratch");
     if (bvh->n == 0) {
         fill_miss_kernel<<<uint32_t((n + 255) / 256), 256, 0, ctx->stream>>>(uint32_t(n), prim_out, t_out, bary_out);
@@ -604,7 +606,7 @@ int pbrtm_bvh_intersect_noalloc(pbrtm_bvh *bvh, const float *rays, uint64_t n, i
                             std::to_string(kNoAllocSpillBytes) + "-byte scratch for " + std::to_string(n) + " rays");
         W.spill = W.spill_per_ray ? spill : nullptr;
         CK(ctx, trace_wide(W, rays, uint32_t(n), any_hit, prim_out, t_out, bary_out, words, nullptr, queue,
-                           words + 1, ctx->stream), "trace");
+                           words + 1, words + 16, ctx->stream), "trace");
     }
     uint32_t derr = 0;
     CK(ctx, hipMemcpyAsync(&derr, words, 4, hipMemcpyDeviceToHost, ctx->stream), "download");

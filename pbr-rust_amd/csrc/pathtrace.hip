@@ -39,12 +39,18 @@ constexpr uint32_t kIdle = 0xFFFFFFFFu;
 // of the traversal and cost more than that.)
 // counters[] layout (u32 words): per parity a block of kCntBlock words, [kCntLive,
 // kCntShadow] the lengths of the live list and the shadow queue, [kCntRays] the
-// closest-hit queue's where it is a queue of its own, and each length's traversal counter
-// kQueueHead words after it; kCntAccRays: u64 accumulators of a batched render.
+// closest-hit queue's where it is a queue of its own; kCntAccRays: u64 accumulators of a
+// batched render; after these kCntWords words, per parity the traversals' heads of the
+// closest-hit and of the shadow queue.
 constexpr int kCntNextId = 0, kCntRound = 1, kCntDone = 2, kCntAccRays = 4;
-constexpr int kCntBlock = 8, kCntLive = 0, kCntShadow = 1, kCntRays = 4;
+constexpr int kCntBlock = 8, kCntLive = 0, kCntShadow = 1, kCntRays = 2;
 constexpr int kCntWords = 32;
+constexpr int kHeadBlock = 2 * int(kHeadWords);  // a parity's heads
+constexpr int kCntAll = kCntWords + 2 * kHeadBlock;
 __host__ __device__ constexpr int cnt_block(uint32_t parity) { return kCntBlock * (1 + int(parity & 1u)); }
+__host__ __device__ constexpr int cnt_heads(uint32_t parity, bool shadow) {
+    return kCntWords + int(parity & 1u) * kHeadBlock + (shadow ? int(kHeadWords) : 0);
+}
 
 struct State {
     uint32_t *path_id, *flags, *dim;
@@ -450,10 +456,9 @@ __global__ __launch_bounds__(kBlock) void init_pool_multi_kernel(State st, Param
 
 // The counters before round 0: `first` slots hold paths.
 __global__ void init_counters_kernel(uint32_t *counters, uint32_t first) {
-    const int k = threadIdx.x;
-    if (k >= kCntWords) return;
     const int b = cnt_block(0);
-    counters[k] = (k == kCntNextId || k == b + kCntLive || k == b + kCntRays) ? first : 0u;
+    for (int k = threadIdx.x; k < kCntAll; k += blockDim.x)
+        counters[k] = (k == kCntNextId || k == b + kCntLive || k == b + kCntRays) ? first : 0u;
 }
 
 // The workgroup's slots with shadow rays, gathered as its waves end: the last one to end
@@ -1085,15 +1090,16 @@ __global__ __launch_bounds__(kBlock) void reduce_shards_kernel(float *d, uint32_
 // after the round's last event), and its parity's block is cleared for the round after
 // the next one to append to.
 __global__ void round_end_kernel(uint32_t *counters, uint32_t parity, uint32_t *host) {
-    const int k = threadIdx.x;
+    const int k = threadIdx.x, b = cnt_block(parity);
+    for (int h = k; h < kHeadBlock; h += blockDim.x) counters[cnt_heads(parity, false) + h] = 0u;
     if (k >= kCntWords) return;
     host[k] = counters[k];
-    const int b = cnt_block(parity);
     if (k >= b && k < b + kCntBlock) counters[k] = 0u;
 }
 // End of a batched round (a kernel, so that a captured graph holds no memset). A round
 // without a live path means that the render is over, and does not count.
 __global__ void round_end_multi_kernel(uint32_t *counters, uint32_t parity) {
+    for (int h = threadIdx.x; h < kHeadBlock; h += blockDim.x) counters[cnt_heads(parity, false) + h] = 0u;
     if (threadIdx.x != 0 || counters[kCntDone]) return;
     uint32_t *c = counters + cnt_block(parity);
     if (c[kCntLive] == 0) {
@@ -1548,7 +1554,7 @@ hipError_t reserve_pool(PathPool &pp, uint32_t pool, uint64_t total, bool batch,
         PT_CK(pp.rec_round.reserve(total * 4));
         pp.rec_cap = total;
     }
-    PT_CK(pp.counters.reserve(kCntWords * sizeof(uint32_t)));
+    PT_CK(pp.counters.reserve(kCntAll * sizeof(uint32_t)));
     return hipSuccess;
 #undef PT_CK
 }
@@ -1657,7 +1663,7 @@ hipError_t render(const SceneDev &S, const WideTrace &W0, uint32_t spp, uint32_t
             hipHostFree(h);
         }
     } guard{ev, hc, stream};
-    init_counters_kernel<<<1, 64, 0, stream>>>(st.counters, pool);
+    init_counters_kernel<<<1, kBlock, 0, stream>>>(st.counters, pool);
     PT_CK(hipEventRecord(ev[0], stream));
     if (gd) init_pool_kernel<true><<<grid, kBlock, 0, stream>>>(S, st, P);
     else init_pool_kernel<false><<<grid, kBlock, 0, stream>>>(S, st, P);
@@ -1677,11 +1683,12 @@ hipError_t render(const SceneDev &S, const WideTrace &W0, uint32_t spp, uint32_t
         PT_CK(hipEventRecord(E[0], stream));
         PT_CK(trace_wide_queued(W, reinterpret_cast<const float *>(st.rays), pool, 0, pp.prim.as<uint32_t>(),
                                 pp.thit.as<float>(), pp.bary.as<float>(), err, separate_rays ? st.rayq[par] : st.live[par],
-                                c + (separate_rays ? kCntRays : kCntLive), stream, counts));
+                                c + (separate_rays ? kCntRays : kCntLive), st.counters + cnt_heads(par, false), stream,
+                                counts));
         PT_CK(hipEventRecord(E[1], stream));
         PT_CK(trace_wide_queued(W, reinterpret_cast<const float *>(st.srays), 2 * pool, 1, pp.sprim.as<uint32_t>(),
-                                nullptr, nullptr, err, st.shadowq[par], c + kCntShadow, stream,
-                                counts ? counts + 3 : nullptr));
+                                nullptr, nullptr, err, st.shadowq[par], c + kCntShadow,
+                                st.counters + cnt_heads(par, true), stream, counts ? counts + 3 : nullptr));
         PT_CK(hipEventRecord(E[2], stream));
         if (gd) shade_grad_kernel<<<grid, kBlock, 0, stream>>>(S, st, P);
         else if (integrator == kIntMegakernelPath) shade_kernel<kIntMegakernelPath><<<grid, kBlock, 0, stream>>>(S, st, P);
@@ -1691,7 +1698,7 @@ hipError_t render(const SceneDev &S, const WideTrace &W0, uint32_t spp, uint32_t
         else shade_kernel<kIntPath><<<grid, kBlock, 0, stream>>>(S, st, P);
         PT_CK(hipGetLastError());
         PT_CK(hipEventRecord(E[3], stream));
-        round_end_kernel<<<1, 64, 0, stream>>>(st.counters, par, hc + kCntWords * par);
+        round_end_kernel<<<1, kBlock, 0, stream>>>(st.counters, par, hc + kCntWords * par);
         PT_CK(hipGetLastError());
         PT_CK(hipEventRecord(E[4], stream));
         return hipSuccess;
@@ -1830,7 +1837,7 @@ hipError_t render_shared(const std::vector<BatchJob> &jobs, uint32_t pool, uint3
             if (*g) hipGraphDestroy(*g);
         }
     } guard{ev, &graph, &exec};
-    init_counters_kernel<<<1, 64, 0, stream>>>(st.counters, pool);
+    init_counters_kernel<<<1, kBlock, 0, stream>>>(st.counters, pool);
     PT_CK(hipEventRecord(ev[0], stream));
     init_pool_multi_kernel<<<grid, kBlock, 0, stream>>>(st, P);
     PT_CK(hipGetLastError());
@@ -1841,14 +1848,16 @@ hipError_t render_shared(const std::vector<BatchJob> &jobs, uint32_t pool, uint3
             uint32_t *c = st.counters + cnt_block(k);
             if ((e2 = trace_wide_multi_queued(W, d_jw, st.job, 0, reinterpret_cast<const float *>(st.rays), pool, 0,
                                               pp.prim.as<uint32_t>(), pp.thit.as<float>(), pp.bary.as<float>(), err,
-                                              st.live[k & 1u], c + kCntLive, stream)) != hipSuccess)
+                                              st.live[k & 1u], c + kCntLive, st.counters + cnt_heads(k, false),
+                                              stream)) != hipSuccess)
                 return e2;
             if ((e2 = trace_wide_multi_queued(W, d_jw, st.job, 1, reinterpret_cast<const float *>(st.srays),
                                               2 * pool, 1, pp.sprim.as<uint32_t>(), nullptr, nullptr, err,
-                                              st.shadowq[k & 1u], c + kCntShadow, stream)) != hipSuccess)
+                                              st.shadowq[k & 1u], c + kCntShadow, st.counters + cnt_heads(k, true),
+                                              stream)) != hipSuccess)
                 return e2;
             shade_multi_kernel<<<grid, kBlock, 0, stream>>>(st, P);
-            round_end_multi_kernel<<<1, 64, 0, stream>>>(st.counters, k);
+            round_end_multi_kernel<<<1, kBlock, 0, stream>>>(st.counters, k);
             if ((e2 = hipGetLastError()) != hipSuccess) return e2;
         }
         return hipSuccess;

@@ -59,27 +59,30 @@ struct WideTrace {
 
 // counts (device, nullable): adds [wide nodes visited, child box tests, triangle tests];
 // a node whose boxes are tested again after a hit in one of its leaves is no new visit.
-// queue (device, n entries) and queue_len (device, the two words [0] and [kQueueHead]
-// zeroed by the caller) hold the compacted active rays: queue_len[0] their number,
-// queue_len[kQueueHead] the traversal's counter of rows handed out.
-constexpr int kQueueHead = 2;
+// queue (device, n entries) and queue_len (device, one word zeroed by the caller) hold the
+// compacted active rays and their number; heads (device, kHeadWords words zeroed by the
+// caller, 64-byte aligned) count the rows handed out.
+constexpr uint32_t kHeads = 32;       // counters of rows, each serving its share of them
+constexpr uint32_t kHeadStride = 16;  // words between two: a cache line of their own
+constexpr uint32_t kHeadWords = kHeads * kHeadStride;
 hipError_t trace_wide(const WideTrace &B, const float *rays, uint32_t n, int any_hit, uint32_t *prim_out,
                       float *t_out, float *bary_out, uint32_t *err, unsigned long long *counts, uint32_t *queue,
-                      uint32_t *queue_len, hipStream_t stream);
+                      uint32_t *queue_len, uint32_t *heads, hipStream_t stream);
 
-// The rays of a queue filled by the caller (queue_len[0] of at most n entries;
-// queue_len[kQueueHead] has to be zero, rows below a head left from another traversal
-// would be skipped). Ray i of several jobs is traced against jobs[ray_job[i >> job_shift]] (nodes, order, tri_leaf,
+// The rays of a queue filled by the caller (*queue_len of at most n entries; heads have to
+// be zero, rows below a head left from another traversal would be skipped). Ray i of
+// several jobs is traced against jobs[ray_job[i >> job_shift]] (nodes, order, tri_leaf,
 // prim_order, num_nodes, num_prims); B supplies the spill area.
 hipError_t trace_wide_multi_queued(const WideTrace &B, const WideTrace *jobs, const uint32_t *ray_job,
                                    uint32_t job_shift, const float *rays, uint32_t n, int any_hit, uint32_t *prim_out,
                                    float *t_out, float *bary_out, uint32_t *err, const uint32_t *queue,
-                                   uint32_t *queue_len, hipStream_t stream);
-// The same for one tree (queue and queue_len as above).
+                                   const uint32_t *queue_len, uint32_t *heads, hipStream_t stream);
+// The same for one tree (queue, queue_len and heads as above).
 // counts (device, nullable): adds [nodes visited, child box tests, primitive tests].
 hipError_t trace_wide_queued(const WideTrace &B, const float *rays, uint32_t n, int any_hit, uint32_t *prim_out,
                              float *t_out, float *bary_out, uint32_t *err, const uint32_t *queue,
-                             uint32_t *queue_len, hipStream_t stream, unsigned long long *counts = nullptr);
+                             const uint32_t *queue_len, uint32_t *heads, hipStream_t stream,
+                             unsigned long long *counts = nullptr);
 
 constexpr uint32_t kLdsStack = 12;
 

@@ -707,19 +707,24 @@ __device__ __forceinline__ void add_counts(unsigned long long *counts, uint32_t 
 }
 
 // Persistent traversal: a grid that fills the GPU once; every wave takes rows of up to
-// kWave queue slots (wide_row), and a lane whose ray has finished takes the row's next slot as soon as
-// kRefill lanes are idle, so that the waves keep most lanes busy instead of waiting
-// for their slowest ray. The first kDealt eighths of the queue are dealt out (wave w
-// takes row w of every `waves` rows); the rest goes row by row to whichever wave asks
-// next (queue_len[kQueueHead]), so that no wave is left with more work than the others. One
-// counter serves the atomics at some 6 ns each, which is why not all rows go that way
-// and none is shorter (1080p camera rays into 10M triangles: all dealt 1294 us, none
-// 1109, 5/8 1032, 5/8 with rows of 32 at the end 1121; 33M paths of a path-traced
-// image: 122.5, 121.7, 118.3 and 124.8 ms). Each ray is traced on its own
-// (wide_ray_start, then wide_node, wide_leaf and wide_advance until one reports the ray
-// finished, wide_ray_finish), so which lane or wave takes it changes nothing. MULTI: every ray selects its own
-// tree, jw[ray_job[i >> job_shift]] (jobs of a batched render); the spill area
-// stays the launch's.
+// kWave queue slots (wide_row), and a lane whose ray has finished takes the row's next slot
+// as soon as kRefill lanes are idle, so that the waves keep most lanes busy instead of
+// waiting for their slowest ray. The first kDealt eighths of the queue are dealt out (wave
+// w takes row w of every `waves` rows); the rest goes row by row to whichever wave asks
+// next, so that no wave is left with more work than the others (1080p camera rays into 10M
+// triangles: all dealt 1294 us, none 1109, 5/8 1032, 5/8 with rows of 32 at the end 1121;
+// 33M paths of a path-traced image: 122.5, 121.7, 118.3 and 124.8 ms). A counter in memory
+// serves an atomic in some 6 ns, and every wave's last one finds nothing left: with one
+// counter for all waves, rays that cost little wait for it. So the rows of the rest go
+// round kHeads counters, each on a line of its own and asked by the workgroups whose index
+// is its own modulo kHeads, and a queue that was dealt out whole is not asked for more.
+// Two million rays past one triangle 332 -> 73 us a call, 360,000 102 -> 42 us (93 and 50
+// with all rows dealt); 33M path-traced paths 104.2 -> 100.7 ms, with 8 counters 101.0 and a
+// gradient of 1M triangles +0.6 %.
+// Each ray is traced on its own (wide_ray_start, then wide_node, wide_leaf and wide_advance
+// until one reports the ray finished, wide_ray_finish), so which lane or wave takes it
+// changes nothing. MULTI: every ray selects its own tree, jw[ray_job[i >> job_shift]] (jobs
+// of a batched render); the spill area stays the launch's.
 constexpr uint32_t kRefill = 16;
 constexpr uint32_t kWideWaves = kWideBlock / kWave;
 // Slots of a row: a queue with less than kWave rays for each of kSpread waves (one per
@@ -749,7 +754,8 @@ constexpr uint32_t kLeafShare = 3;
 template <bool COUNT, bool MULTI, bool SHAPES>
 __device__ __forceinline__ void trace_wide_persistent_body(const WideTrace &B, const float4 *__restrict__ rays,
                                                            const uint32_t *__restrict__ queue,
-                                                           uint32_t *__restrict__ queue_len, int any_hit,
+                                                           const uint32_t *__restrict__ queue_len,
+                                                           uint32_t *__restrict__ heads, int any_hit,
                                                            uint32_t *__restrict__ prim_out,
                                                            float *__restrict__ t_out, float *__restrict__ bary_out,
                                                            uint32_t *__restrict__ err,
@@ -757,7 +763,7 @@ __device__ __forceinline__ void trace_wide_persistent_body(const WideTrace &B, c
                                                            const WideTrace *__restrict__ jw,
                                                            const uint32_t *__restrict__ ray_job, uint32_t job_shift,
                                                            uint2 (*s_stack)[kWideBlock]) {
-    const uint32_t n = queue_len[0];
+    const uint32_t n = *queue_len;
     const uint32_t lane = __lane_id();
     const uint32_t waves = gridDim.x * kWideWaves;
     WideTree T = tree_of(MULTI ? jw : &B);  // MULTI: the tree of the lane's current ray
@@ -775,6 +781,7 @@ __device__ __forceinline__ void trace_wide_persistent_body(const WideTrace &B, c
     const uint64_t row_all = uint64_t(waves) * row;  // slots of one row of every wave
     uint32_t rows = max(1u, uint32_t(n / row_all * kDealt / 8));
     const uint64_t dealt = rows * row_all;
+    const uint32_t groups = min(gridDim.x, kHeads), head = blockIdx.x % groups;
     while (true) {
         const uint64_t idle = __ballot(!live);
         if (more && (idle == ~0ull || uint32_t(__popcll(idle)) >= kRefill)) {
@@ -797,8 +804,8 @@ __device__ __forceinline__ void trace_wide_persistent_body(const WideTrace &B, c
             } else if (left == 0) {  // the next row of the rest
                 rows = 1;
                 uint32_t k = 0;
-                if (lane == 0) k = atomicAdd(&queue_len[kQueueHead], 1u);
-                const uint64_t at = dealt + uint64_t(__builtin_amdgcn_readfirstlane(k)) * row;
+                if (dealt < n && lane == 0) k = atomicAdd(&heads[head * kHeadStride], 1u);
+                const uint64_t at = dealt + (uint64_t(__builtin_amdgcn_readfirstlane(k)) * groups + head) * row;
                 more = at < n;
                 if (more) {
                     next = uint32_t(at);
@@ -842,22 +849,22 @@ __device__ __forceinline__ void trace_wide_persistent_body(const WideTrace &B, c
 template <bool COUNT, bool SHAPES>
 __global__ __launch_bounds__(kWideBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) void trace_wide_kernel(
     WideTrace B, const float4 *__restrict__ rays, const uint32_t *__restrict__ queue,
-    uint32_t *__restrict__ queue_len, int any_hit, uint32_t *__restrict__ prim_out,
+    const uint32_t *__restrict__ queue_len, uint32_t *__restrict__ heads, int any_hit, uint32_t *__restrict__ prim_out,
     float *__restrict__ t_out, float *__restrict__ bary_out, uint32_t *__restrict__ err,
     unsigned long long *__restrict__ counts) {
     __shared__ uint2 s_stack[kLdsStack][kWideBlock];
-    trace_wide_persistent_body<COUNT, false, SHAPES>(B, rays, queue, queue_len, any_hit, prim_out, t_out, bary_out,
+    trace_wide_persistent_body<COUNT, false, SHAPES>(B, rays, queue, queue_len, heads, any_hit, prim_out, t_out, bary_out,
                                                      err, counts, nullptr, nullptr, 0, s_stack);
 }
 
 template <bool SHAPES>
 __global__ __launch_bounds__(kWideBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) void trace_wide_multi_kernel(
     WideTrace B, const float4 *__restrict__ rays, const uint32_t *__restrict__ queue,
-    uint32_t *__restrict__ queue_len, int any_hit, uint32_t *__restrict__ prim_out,
+    const uint32_t *__restrict__ queue_len, uint32_t *__restrict__ heads, int any_hit, uint32_t *__restrict__ prim_out,
     float *__restrict__ t_out, float *__restrict__ bary_out, uint32_t *__restrict__ err,
     const WideTrace *__restrict__ jw, const uint32_t *__restrict__ ray_job, uint32_t job_shift) {
     __shared__ uint2 s_stack[kLdsStack][kWideBlock];
-    trace_wide_persistent_body<false, true, SHAPES>(B, rays, queue, queue_len, any_hit, prim_out, t_out, bary_out,
+    trace_wide_persistent_body<false, true, SHAPES>(B, rays, queue, queue_len, heads, any_hit, prim_out, t_out, bary_out,
                                                     err, nullptr, jw, ray_job, job_shift, s_stack);
 }
 
@@ -968,11 +975,11 @@ static uint32_t persistent_grid(Kernel kernel, uint32_t n, uint32_t quarters) {
 static hipError_t trace_wide_queued_counts(const WideTrace &B, const float4 *r, uint32_t n, int any_hit,
                                            uint32_t *prim_out, float *t_out, float *bary_out, uint32_t *err,
                                            unsigned long long *counts, const uint32_t *queue,
-                                           uint32_t *queue_len, hipStream_t stream) {
+                                           const uint32_t *queue_len, uint32_t *heads, hipStream_t stream) {
     const auto kernel = B.shapes ? (counts ? trace_wide_kernel<true, true> : trace_wide_kernel<false, true>)
                                  : (counts ? trace_wide_kernel<true, false> : trace_wide_kernel<false, false>);
     const uint32_t grid = persistent_grid(kernel, n, B.grid_quarters);
-    kernel<<<grid, kWideBlock, 0, stream>>>(B, r, queue, queue_len, any_hit, prim_out, t_out, bary_out, err, counts);
+    kernel<<<grid, kWideBlock, 0, stream>>>(B, r, queue, queue_len, heads, any_hit, prim_out, t_out, bary_out, err, counts);
     return hipGetLastError();
 }
 
@@ -980,40 +987,41 @@ static hipError_t trace_wide_queued_counts(const WideTrace &B, const float4 *r, 
 static hipError_t launch_multi(const WideTrace &B, const WideTrace *jobs, const uint32_t *ray_job,
                                uint32_t job_shift, const float4 *r, uint32_t n, int any_hit, uint32_t *prim_out,
                                float *t_out, float *bary_out, uint32_t *err, const uint32_t *queue,
-                               uint32_t *queue_len, hipStream_t stream) {
+                               const uint32_t *queue_len, uint32_t *heads, hipStream_t stream) {
     const auto kernel = B.shapes ? trace_wide_multi_kernel<true> : trace_wide_multi_kernel<false>;
     const uint32_t grid = persistent_grid(kernel, n, B.grid_quarters);
-    kernel<<<grid, kWideBlock, 0, stream>>>(B, r, queue, queue_len, any_hit, prim_out, t_out, bary_out, err, jobs,
+    kernel<<<grid, kWideBlock, 0, stream>>>(B, r, queue, queue_len, heads, any_hit, prim_out, t_out, bary_out, err, jobs,
                                             ray_job, job_shift);
     return hipGetLastError();
 }
 
 hipError_t trace_wide(const WideTrace &B, const float *rays, uint32_t n, int any_hit, uint32_t *prim_out,
                       float *t_out, float *bary_out, uint32_t *err, unsigned long long *counts, uint32_t *queue,
-                      uint32_t *queue_len, hipStream_t stream) {
+                      uint32_t *queue_len, uint32_t *heads, hipStream_t stream) {
     if (n == 0) return hipSuccess;
     const uint32_t cgrid = (n + kCompactBlock * kCompactItems - 1) / (kCompactBlock * kCompactItems);
     const float4 *r = reinterpret_cast<const float4 *>(rays);
     compact_rays_kernel<<<cgrid, kCompactBlock, 0, stream>>>(r, n, queue, queue_len, prim_out, t_out, bary_out);
     return trace_wide_queued_counts(B, r, n, any_hit, prim_out, t_out, bary_out, err, counts, queue, queue_len,
-                                    stream);
+                                    heads, stream);
 }
 
 hipError_t trace_wide_multi_queued(const WideTrace &B, const WideTrace *jobs, const uint32_t *ray_job,
                                    uint32_t job_shift, const float *rays, uint32_t n, int any_hit, uint32_t *prim_out,
                                    float *t_out, float *bary_out, uint32_t *err, const uint32_t *queue,
-                                   uint32_t *queue_len, hipStream_t stream) {
+                                   const uint32_t *queue_len, uint32_t *heads, hipStream_t stream) {
     if (n == 0) return hipSuccess;
     return launch_multi(B, jobs, ray_job, job_shift, reinterpret_cast<const float4 *>(rays), n, any_hit, prim_out,
-                        t_out, bary_out, err, queue, queue_len, stream);
+                        t_out, bary_out, err, queue, queue_len, heads, stream);
 }
 
 hipError_t trace_wide_queued(const WideTrace &B, const float *rays, uint32_t n, int any_hit, uint32_t *prim_out,
                              float *t_out, float *bary_out, uint32_t *err, const uint32_t *queue,
-                             uint32_t *queue_len, hipStream_t stream, unsigned long long *counts) {
+                             const uint32_t *queue_len, uint32_t *heads, hipStream_t stream,
+                             unsigned long long *counts) {
     if (n == 0) return hipSuccess;
     return trace_wide_queued_counts(B, reinterpret_cast<const float4 *>(rays), n, any_hit, prim_out, t_out, bary_out,
-                                    err, counts, queue, queue_len, stream);
+                                    err, counts, queue, queue_len, heads, stream);
 }
 
 }  // namespace pbrtm

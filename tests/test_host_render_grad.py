@@ -59,8 +59,8 @@ def columns_stay_missing():
 
 def device_error():
     def launch(kernel, blocks, threads, captured, args):
-        if "trace_wide_kernel" in kernel:  # (tree, rays, queue, length, any_hit, prim, t, bary, err, counts)
-            fake_hip.poke_u32(fake_hip.pointer(args, 8), 8)  # a traversal stack overflow
+        if "trace_wide_kernel" in kernel:  # (tree, rays, queue, length, heads, any_hit, prim, t, bary, err, counts)
+            fake_hip.poke_u32(fake_hip.pointer(args, 9), 8)  # a traversal stack overflow
 
     fake_hip.install(launch)
     import pbrtm
