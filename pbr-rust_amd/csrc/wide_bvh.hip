@@ -716,11 +716,13 @@ __device__ __forceinline__ void add_counts(unsigned long long *counts, uint32_t 
 // 33M paths of a path-traced image: 122.5, 121.7, 118.3 and 124.8 ms). A counter in memory
 // serves an atomic in some 6 ns, and every wave's last one finds nothing left: with one
 // counter for all waves, rays that cost little wait for it. So the rows of the rest go
-// round kHeads counters, each on a line of its own and asked by the workgroups whose index
-// is its own modulo kHeads, and a queue that was dealt out whole is not asked for more.
-// Two million rays past one triangle 332 -> 73 us a call, 360,000 102 -> 42 us (93 and 50
-// with all rows dealt); 33M path-traced paths 104.2 -> 100.7 ms, with 8 counters 101.0 and a
-// gradient of 1M triangles +0.6 %.
+// round kHeads counters, each on a line of its own; a wave asks the one of its workgroup's
+// index modulo kHeads, and when that one's rows are gone up to kAsked - 1 of the next, so
+// that no counter's rows are left to its own waves alone. A queue that was dealt out whole
+// is not asked for more. 1.96 million rays past one triangle 332 -> 83 us a call, 360,000
+// 102 -> 42 us (94 and 52 with all rows dealt); 33M path-traced paths 104.1 -> 100.0 ms.
+// With one counter asked, 73 and 42 us, but 463M paths of 64 mixed jobs 335.8 -> 351.7 ms
+// (337.7 with four, 341 with two), with all of them asked 190 us and 104.9 ms.
 // Each ray is traced on its own (wide_ray_start, then wide_node, wide_leaf and wide_advance
 // until one reports the ray finished, wide_ray_finish), so which lane or wave takes it
 // changes nothing. MULTI: every ray selects its own tree, jw[ray_job[i >> job_shift]] (jobs
@@ -733,7 +735,7 @@ constexpr uint32_t kWideWaves = kWideBlock / kWave;
 // launch lasts as long as its longest ray, step by step (1-2 us each), and lanes of a wave
 // wait for each other's node and leaf steps; with eight times the waves the steps
 // themselves slow down. Calls of 999 camera rays into 100k triangles, 14,400 and 153,600
-// into 1M, with rows of 64: 174, 455 and 540 us; now 141, 386 and 535; spread over 8192
+// into 1M, with rows of 64: 174, 455 and 540 us; so 141, 386 and 535; spread over 8192
 // waves 138, 410 and 706.
 constexpr uint32_t kSpread = 1024;
 __host__ __device__ constexpr uint32_t wide_row(uint32_t n) {
@@ -741,6 +743,7 @@ __host__ __device__ constexpr uint32_t wide_row(uint32_t n) {
     return r < 1u ? 1u : (r > uint32_t(kWave) ? uint32_t(kWave) : r);
 }
 constexpr uint32_t kDealt = 5;
+constexpr uint32_t kAsked = 4;
 // A wave steps either its lanes that wait at a node or those that wait at a leaf's
 // primitive, never both paths for a few lanes each: the leaves go when they are at
 // least a third of the others. Waiting longer fills the leaf steps but idles more
@@ -748,7 +751,7 @@ constexpr uint32_t kDealt = 5;
 // 1/3, 107.1 at 1/6; 1/2 slows short queues (16 mixed jobs +1 %); 1/8, 1/12 and a fixed
 // count of 8 lanes are slower still. Against testing every leaf where a lane met it: 1080p camera rays into 10M
 // triangles 1780 -> 1246 us, shadow rays into 1M 909 -> 701 us, 999 rays 209 -> 178 us
-// (and 96 -> 73 VGPRs, 6 waves per SIMD).
+// (and 96 -> 75 VGPRs, 6 waves per SIMD).
 constexpr uint32_t kLeafShare = 3;
 
 template <bool COUNT, bool MULTI, bool SHAPES>
@@ -781,7 +784,8 @@ __device__ __forceinline__ void trace_wide_persistent_body(const WideTrace &B, c
     const uint64_t row_all = uint64_t(waves) * row;  // slots of one row of every wave
     uint32_t rows = max(1u, uint32_t(n / row_all * kDealt / 8));
     const uint64_t dealt = rows * row_all;
-    const uint32_t groups = min(gridDim.x, kHeads), head = blockIdx.x % groups;
+    const uint32_t groups = min(gridDim.x, kHeads);  // heads in use
+    uint32_t head = blockIdx.x % groups, empty = 0;  // the head asked next, heads found empty
     while (true) {
         const uint64_t idle = __ballot(!live);
         if (more && (idle == ~0ull || uint32_t(__popcll(idle)) >= kRefill)) {
@@ -806,10 +810,12 @@ __device__ __forceinline__ void trace_wide_persistent_body(const WideTrace &B, c
                 uint32_t k = 0;
                 if (dealt < n && lane == 0) k = atomicAdd(&heads[head * kHeadStride], 1u);
                 const uint64_t at = dealt + (uint64_t(__builtin_amdgcn_readfirstlane(k)) * groups + head) * row;
-                more = at < n;
-                if (more) {
+                if (at < n) {
                     next = uint32_t(at);
                     left = min(n - next, row);
+                } else {
+                    head = head + 1u == groups ? 0u : head + 1u;
+                    more = dealt < n && ++empty < min(groups, kAsked);
                 }
             }
             continue;
@@ -838,7 +844,7 @@ __device__ __forceinline__ void trace_wide_persistent_body(const WideTrace &B, c
 }
 
 // The occupancy floor of 5 waves per SIMD keeps the registers of the per-ray-tree and the
-// analytic instances within 96 without spills; the single-tree triangle instance needs 73
+// analytic instances within 96 without spills; the single-tree triangle instance needs 75
 // and runs at the 6 that the LDS stack (24 KiB per block) allows. Held to 6, the
 // per-ray-tree one spills four registers: 16 mixed jobs 5.46 -> 5.62 ms. A refill
 // waits for 16 idle lanes: the rays' start (two loads, reciprocals, shear) costs a step of

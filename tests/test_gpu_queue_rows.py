@@ -68,7 +68,7 @@ def test_film_order(ctx, spp, pool):
 @pytest.mark.parametrize("n", [360_000, 1_210_000])
 def test_cheap_rays_do_not_wait_for_each_other(ctx, n):
     """Rays past a single triangle, a node each: the call is a few launches and the queue's
-    traffic (the binary traversal, without a queue, takes 29 and 39 us, this one 42 and 62; 102
+    traffic (the binary traversal, without a queue, takes 29 and 40 us, this one 42 and 71; 102
     and 260 us when all waves asked one counter for their rows)."""
     import time
 
