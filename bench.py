@@ -54,8 +54,8 @@ FILM_RECORD_BYTES = 16 + 4  # per path: sensor RGB + filter weight, finishing ro
 # with --calibrate-copy), for the default workload. Taken from the profile named
 # beside it, not measured by this run.
 TRAFFIC = {
-    "trace_wide_kernel": (2_275_583_424, "profiles/trace_wide_hlbvh10m_1080p_pmc_traffic.md"),
-    "build": (13_289_255_040, "profiles/trace_wide_hlbvh10m_1080p_pmc_traffic.md"),
+    "trace_wide_kernel": (2_230_260_848, "profiles/trace_wide_hlbvh10m_1080p_pmc_traffic.md"),
+    "build": (13_599_504_720, "profiles/trace_wide_hlbvh10m_1080p_pmc_traffic.md"),
 }
 
 
