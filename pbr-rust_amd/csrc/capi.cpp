@@ -544,6 +544,7 @@ int pbrtm_bvh_intersect(pbrtm_bvh *bvh, const float *rays, uint64_t n, int any_h
             W.num_nodes = bvh->wide.num_nodes;
             W.num_prims = bvh->n;
             W.max_depth = bvh->wide.max_depth;
+            W.box = tree_box(bvh->bounds, W.num_nodes);
             W.spill_per_ray = W.max_depth > kLdsStack ? W.max_depth - kLdsStack + 1 : 0;
             if (W.spill_per_ray) {
                 CK(ctx, ctx->spill.reserve(size_t(n) * W.spill_per_ray * sizeof(uint2)), "alloc stack spill");
@@ -598,6 +599,7 @@ int pbrtm_bvh_intersect_noalloc(pbrtm_bvh *bvh, const float *rays, uint64_t n, i
         W.num_nodes = bvh->wide.num_nodes;
         W.num_prims = bvh->n;
         W.max_depth = bvh->wide.max_depth;
+        W.box = tree_box(bvh->bounds, W.num_nodes);
         W.spill_per_ray = W.max_depth > kLdsStack ? W.max_depth - kLdsStack + 1 : 0;
         if (uint64_t(W.spill_per_ray) * n * sizeof(uint2) > kNoAllocSpillBytes)
             return fail(ctx, PBRTM_ERR_INVALID,
@@ -873,6 +875,7 @@ WideTrace scene_trace(const pbrtm_scene *sc) {
     W.num_nodes = bvh->wide.num_nodes;
     W.num_prims = bvh->n;
     W.max_depth = bvh->wide.max_depth;
+    W.box = tree_box(bvh->bounds, W.num_nodes);
     W.shapes = sc->dev.shapes;
     W.spill_per_ray = W.max_depth > kLdsStack ? W.max_depth - kLdsStack + 1 : 0;
     return W;

@@ -67,7 +67,19 @@ PBRTM_HD int box_quant_hi(float v, float org, float step, float inv_step) {
 // touches o has t = 0 or NaN in the reference), and moves its planes outwards by 2^-30
 // of the size of the tree and the ray's distance from it, whatever their scale.
 // Rays without a direction, with NaNs or far outside any scene (BoxRay::generic) take
-// the reference's own test on the decoded planes.
+// the reference's own test on the decoded planes. So do rays from so far away that err,
+// which grows with |B|, is no longer small against the tree's boxes: it widens them by
+// 2^-20 of the distance, and were the nodes of equal squares on a face of the tree's box
+// their edge would be extent / sqrt(num_nodes). A ray is conservative up to a distance of
+// 3 * 2^16 such edges, where it widens by 3/16 of one. The reference's test makes a visit
+// a fourth dearer. 524,288 closest hits without and with the rule, in ms:
+//   height field of 3.9M triangles, 500 / 1000 extents away: 0.42 / 0.68, with it 0.33 / 0.36
+//   the same with 320,000 triangles, 1000 / 2000: 0.29 / 0.35, with it 0.28 / 0.27
+//   10M random triangles, 500 / 2000 / 30,000: 1.28 / 10.9 / 497, with it 1.46 / 8.3 / 54
+//   20,000 random triangles, 4000 / 30,000: 0.66 / 1.99, with it 0.77 / 1.35
+// Random triangles fill the box, so their nodes are larger than on a face. A line by the
+// cube root of num_nodes saves what they lose at the first distances, and leaves the height
+// fields as they are without the rule.
 constexpr float kBoxErr = 16.0f * 5.9604644775390625e-08f;
 
 // A ray's reciprocal direction for the box tests (clamped; as it is if generic) and its
@@ -76,18 +88,31 @@ struct BoxRay {
     f3 inv, err;
     bool generic;
 };
-// size(): the largest distance along an axis from o to the far side of the tree's box;
-// asked for rays with a clamped axis only.
-template <typename Size>
-PBRTM_HD BoxRay box_ray(f3 o, f3 d, f3 inv, Size size) {
+// What a ray's start needs to know of a tree: the lower corner of its box, the box's largest
+// extent, and the distance from the corner along an axis up to which rays are conservative.
+struct TreeBox {
+    f3 lo;
+    float extent, reach;
+};
+inline TreeBox tree_box(const float bounds[6], uint32_t num_nodes) {
+    float extent = 0.f;
+    for (int a = 0; a < 3; ++a) {
+        const float e = bounds[3 + a] - bounds[a];
+        extent = e > extent || e != e ? e : extent;  // a NaN stays: every ray is generic
+    }
+    return {{bounds[0], bounds[1], bounds[2]}, extent, extent * (0x1.8p17f / sqrtf(float(num_nodes)))};
+}
+PBRTM_HD BoxRay box_ray(f3 o, f3 d, f3 inv, TreeBox tree) {
     const f3 a = abs3(inv);
     const float least = fminf(fminf(a.x, a.y), a.z), cap = least * 0x1p32f;
     BoxRay r{inv, {0.f, 0.f, 0.f}, false};
     const float span = fabsf(o.x) + fabsf(o.y) + fabsf(o.z) + fabsf(d.x) + fabsf(d.y) + fabsf(d.z);
-    if (!(least <= 0x1p20f && span <= 0x1p60f)) {
+    const f3 to = abs3(sub3(tree.lo, o));
+    const float far = fmaxf(fmaxf(to.x, to.y), to.z);
+    if (!(least <= 0x1p20f && span <= 0x1p60f && far <= tree.reach)) {
         r.generic = true;
     } else if (!(fmaxf(fmaxf(a.x, a.y), a.z) <= cap)) {
-        const float err = 4.0f * size() * least;
+        const float err = 4.0f * (far + tree.extent) * least;
         if (!(a.x <= cap)) r.inv.x = copysignf(cap, inv.x), r.err.x = err;
         if (!(a.y <= cap)) r.inv.y = copysignf(cap, inv.y), r.err.y = err;
         if (!(a.z <= cap)) r.inv.z = copysignf(cap, inv.z), r.err.z = err;

@@ -3,6 +3,7 @@
 
 #include "pbrtm_device.h"
 #include "pbrtm_internal.h"
+#include "wide_box.h"
 
 namespace pbrtm {
 
@@ -52,6 +53,7 @@ struct WideTrace {
     const uint32_t *prim_order;
     const pt::DShape *shapes;  // analytic primitives (leaf pad word = index + 1), null for triangle-only trees
     uint32_t num_nodes, num_prims, max_depth;
+    TreeBox box;
     uint2 *spill;           // per-ray stack overflow area (max_depth - kLdsStack entries per ray), may be null
     uint32_t spill_per_ray;
     uint32_t grid_quarters; // persistent traversal grid: this many quarters of the resident maximum (0 = all)
@@ -72,7 +74,7 @@ hipError_t trace_wide(const WideTrace &B, const float *rays, uint32_t n, int any
 // The rays of a queue filled by the caller (*queue_len of at most n entries; heads have to
 // be zero, rows below a head left from another traversal would be skipped). Ray i of
 // several jobs is traced against jobs[ray_job[i >> job_shift]] (nodes, order, tri_leaf,
-// prim_order, num_nodes, num_prims); B supplies the spill area.
+// prim_order, num_nodes, num_prims, box); B supplies the spill area.
 hipError_t trace_wide_multi_queued(const WideTrace &B, const WideTrace *jobs, const uint32_t *ray_job,
                                    uint32_t job_shift, const float *rays, uint32_t n, int any_hit, uint32_t *prim_out,
                                    float *t_out, float *bary_out, uint32_t *err, const uint32_t *queue,

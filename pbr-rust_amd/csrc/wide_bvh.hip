@@ -456,9 +456,9 @@ __device__ __forceinline__ bool leaf_box_hit(const WideTree &T, uint32_t first, 
 // plane to test it with box_hit's operations took about twice the instructions of the
 // conservative test (wide_box.h): 1080p camera rays into 10M triangles 1995 -> 1780 us,
 // their bounce 1490 -> 1327 us, 919,601 shadow rays into 1M triangles 1080 -> 909 us a call.
-// A ray along an axis reads the root's node to know the tree's size; with a constant in its
-// place 524,288 of them take 0.65 ms through a scene of extent 1 (300k triangles) and 1.9
-// seconds through one of extent 2^40 or 2^-30, now 0.64 ms through all of them. With an
+// Its terms know the tree's box (WideTrace::box); with constants in its place 524,288 rays
+// along an axis take 0.65 ms through a scene of extent 1 (300k triangles) and 1.9 seconds
+// through one of extent 2^40 or 2^-30, now 0.64 ms through all of them. With an
 // allowance for rounding planes to FP32, as many random rays through that scene 4,096,
 // 16,384 and 65,536 times its extent from the world's origin took 1.12, 2.36 and 13.9 ms,
 // now 0.85, 0.81 and 0.80.
@@ -477,12 +477,7 @@ __device__ __forceinline__ bool wide_ray_start(WideRay &R, const float4 *__restr
     R.hit = TriHit{0.f, 0.f, 0.f, 0.f};
     const f3 inv = {1.0f / d.x, 1.0f / d.y, 1.0f / d.z};
     R.oct = uint32_t(inv.x < 0.f) | (uint32_t(inv.y < 0.f) << 1) | (uint32_t(inv.z < 0.f) << 2);
-    const BoxRay box = box_ray(R.o, d, inv, [&] {
-        const uint4 hd = *reinterpret_cast<const uint4 *>(T.nodes);  // the root's origin and steps
-        return fmaxf(fmaxf(fabsf(__uint_as_float(hd.x) - R.o.x) + 255.f * pow2f(int(int8_t(hd.w & 0xFFu))),
-                           fabsf(__uint_as_float(hd.y) - R.o.y) + 255.f * pow2f(int(int8_t((hd.w >> 8) & 0xFFu)))),
-                     fabsf(__uint_as_float(hd.z) - R.o.z) + 255.f * pow2f(int(int8_t((hd.w >> 16) & 0xFFu))));
-    });
+    const BoxRay box = box_ray(R.o, d, inv, T.tree->box);
     R.binv = box.inv;
     R.berr = box.err;
     if (box.generic) R.oct |= kRayGeneric;

@@ -1,9 +1,9 @@
 // Host run of the 8-wide tree's box arithmetic (csrc/wide_box.h) against the reference's
 // slab test (box_hit): random and adversarial boxes and rays. Prints per form of rays
-//   <form> rays <n> entered <exact> missed <m> extra <e>
+//   <form> rays <n> entered <exact> missed <m> extra <e> generic <g>
 // where "entered" counts children whose exact box box_hit enters, "missed" those of them
 // that the conservative test rejects, and "extra" the children it enters although box_hit
-// rejects their decoded quantized box. Exits 1 if a quantized box does not contain its box.
+// rejects their decoded quantized box, and "generic" rays that take box_hit itself. Exits 1 if a quantized box does not contain its box.
 #include <cmath>
 using std::isfinite;
 using std::isinf;
@@ -33,11 +33,12 @@ int main(int argc, char **argv) {
     const int n = atoi(argv[2]);
     const double scale = atof(argv[3]), offset = atof(argv[4]);
     g_state = strtoull(argv[5], nullptr, 10);
+    const uint32_t nodes = uint32_t(atoi(argv[6]));  // of the tree
     // "clear-<form>": no planes or distances that coincide on purpose, no t_max
     const bool clear = !strncmp(form, "clear-", 6);
     const char *kind = clear ? form + 6 : form;
     auto is = [&](const char *f) { return !strcmp(kind, f); };
-    uint64_t entered = 0, missed = 0, extra = 0;
+    uint64_t entered = 0, missed = 0, extra = 0, generic = 0;
     for (int it = 0; it < n; ++it) {
         // the tree's box, a node in it and a child of the node, each at times flat or flush
         double rl[3], rh[3], nl[3], nh[3];
@@ -112,13 +113,9 @@ int main(int argc, char **argv) {
             if (tn > 0.f) t_max = tn;
         }
         const bool exact = box_hit(lo, hi, ro, inv, neg, t_max);
-        const BoxRay R = box_ray(ro, rd, inv, [&] {
-            const float ov[3] = {ro.x, ro.y, ro.z};
-            float size = 0.f;
-            for (int a = 0; a < 3; ++a)
-                size = std::fmax(size, fabsf(root_lo[a] - ov[a]) + 255.f * pow2f(box_step_exp(root_hi[a] - root_lo[a])));
-            return size;
-        });
+        const float bounds[6] = {root_lo[0], root_lo[1], root_lo[2], root_hi[0], root_hi[1], root_hi[2]};
+        const BoxRay R = box_ray(ro, rd, inv, tree_box(bounds, nodes));
+        generic += R.generic;
         float dl[3], dh[3];
         uint32_t qn[3], qf[3];
         BoxAxis ax[3];
@@ -138,7 +135,7 @@ int main(int argc, char **argv) {
                    t_max, lo[0], lo[1], lo[2], hi[0], hi[1], hi[2]);
         extra += pass && !decoded;
     }
-    printf("%s rays %d entered %llu missed %llu extra %llu\n", form, n, (unsigned long long)entered,
-           (unsigned long long)missed, (unsigned long long)extra);
+    printf("%s rays %d entered %llu missed %llu extra %llu generic %llu\n", form, n, (unsigned long long)entered,
+           (unsigned long long)missed, (unsigned long long)extra, (unsigned long long)generic);
     return 0;
 }

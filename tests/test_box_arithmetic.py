@@ -23,9 +23,9 @@ def program(tmp_path_factory):
     subprocess.run(["g++", "-std=c++17", "-O2", "-ffp-contract=off", "-I", os.path.join(HERE, "..", "pbr-rust_amd", "csrc"),
                     "-I", ROCM, "-o", str(exe), os.path.join(HERE, "native", "wide_box.cpp")], check=True)
 
-    def run(form, n, place, seed):
-        p = subprocess.run([str(exe), form, str(n), str(place[0]), str(place[1]), str(seed)], capture_output=True,
-                           text=True, timeout=300)
+    def run(form, n, place, seed, nodes=1):
+        p = subprocess.run([str(exe), form, str(n), str(place[0]), str(place[1]), str(seed), str(nodes)],
+                           capture_output=True, text=True, timeout=300)
         assert p.returncode == 0, p.stdout
         words = p.stdout.split()
         at = words.index("entered")
@@ -49,3 +49,13 @@ def test_few_boxes_are_entered_in_vain(program, form, place):
     at most 8 % more than box_hit enters of the decoded boxes."""
     entered, missed, extra, out = program("clear-" + form, 1_000_000, place, 3)
     assert missed == 0 and extra <= 0.08 * entered, out
+
+
+@pytest.mark.parametrize("nodes,low,high", [(1, 0, 0), (1000, 0, 0), (1_000_000, 0.3, 0.5), (10_000_000, 0.5, 0.7)])
+def test_rays_from_far_away_take_the_reference_s_test(program, nodes, low, high):
+    """Origins up to 4 ... 4096 extents away, evenly in the logarithm, within a cube of that size.
+    The conservative test ends at 196608 / sqrt(nodes) extents along an axis: with one node or a
+    thousand nowhere, with a million at 197, with ten million at 62."""
+    entered, missed, extra, out = program("clear-far", 1_000_000, (1, 0), 5, nodes)
+    generic = int(out.split()[-1]) / 1_000_000
+    assert missed == 0 and low <= generic <= high, out

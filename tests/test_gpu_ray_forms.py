@@ -187,3 +187,28 @@ def test_work_does_not_depend_on_the_scene_s_place(ctx, form, scale, offset):
         bvh.free()
     print(f"{form} scale {scale} offset {offset}: visits and tests per ray {counts[0]} -> {counts[1]}", flush=True)
     assert counts[1][0] <= 1.1 * counts[0][0] and counts[1][1] <= 1.3 * counts[0][1]
+
+
+@pytest.mark.parametrize("distance", [20.0, 2000.0, 40000.0])
+def test_work_from_far_away(ctx, distance):
+    """Rays into 200,000 triangles from `distance` extents away find the hits of the reference's
+    order and test about as many triangles. (An allowance that grows with the distance once
+    had them test seven times as many at 30,000 extents.)"""
+    tri = pbrtm.gen_soup(200_000, seed=61, mu=-5.0)
+    lo, hi = tri.min(axis=(0, 1)).astype(np.float64), tri.max(axis=(0, 1)).astype(np.float64)
+    rng = np.random.default_rng(62)
+    eye = (lo + hi) / 2 + distance * (hi - lo).max() * np.array([0.3, 0.5, -0.81])
+    d = rng.uniform(lo, hi, (4000, 3)) - eye
+    rays = np.zeros((4000, 8), np.float32)
+    rays[:, 0:3], rays[:, 3] = eye, np.inf
+    rays[:, 4:7] = d / np.linalg.norm(d, axis=1, keepdims=True)
+    bvh = ctx.build(tri)
+    tests, out = [], []
+    for binary in (True, False):
+        stats = np.zeros(3, np.uint64)
+        out.append(bvh.intersect(rays, stats=stats, binary=binary))
+        tests.append(stats[2] / len(rays))
+    bvh.free()
+    print(f"distance {distance}: tests per ray {tests[0]:.1f} binary, {tests[1]:.1f} wide", flush=True)
+    assert np.array_equal(out[0][0], out[1][0]) and _same(out[0][1], out[1][1]) and _same(out[0][2], out[1][2])
+    assert tests[1] <= 1.5 * tests[0]
